@@ -22,7 +22,7 @@ BIN = os.path.join(HERE, "bin")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-# -packed-fp32-ops: no v_pk_*_f32 (some forms have misbehaved on this pool).
+# -packed-fp32-ops: no v_pk_*_f32 (some forms have given wrong results on gfx950).
 # -ffp-contract=off: residual updates round like the reference (mul, then add).
 HIP_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=" + ARCH,
@@ -32,6 +32,7 @@ HIP_FLAGS = [
 
 HIP_SOURCES = [
     "kernels/ccd_kernels.hip",
+    "kernels/layout_kernels.hip",
     "kernels/tiled_kernels.hip",
     "kernels/batch_kernels.hip",
     "kernels/foldin_kernels.hip",

@@ -19,26 +19,22 @@
 // upload (stable, so ties keep their order).  The highest-degree rows and
 // columns -- the entries gathered most often -- become a contiguous prefix
 // of every factor vector, which the sweeps stage in LDS, and the sweep work
-// units become contiguous row ranges.  When the whole gathered vector of a
-// layout fits the LDS prefix of a plain sweep, the elements of each row are
-// sorted by internal index as well: the fused passes, which split their LDS
-// between two gathered arrays, then find most tiles of the tiled copy
-// gathering only from LDS.  (For a larger gathered vector the sort would
-// pack the gathers beyond the prefix into the row ends, which measured
-// slower, so element order is kept there.)  Sorting reorders the terms of
+// units become contiguous row ranges.  The elements of each row are sorted by
+// internal index, so that a row splits at any bound into the elements
+// gathered from below it and the rest, and a lane's consecutive elements
+// beyond an LDS prefix share cache lines.  Sorting reorders the terms of
 // each per-row sum, which are trees anyway, not the reference's serial
 // order.  W, H, the test set and the residual are mapped at the boundary;
 // callers only ever see their own numbering.
 #include "ccd_ctx.h"
+#include "layout.h"
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <map>
 #include <cstdio>
 #include <cstring>
 #include <string>
-#include <thread>
 #include <vector>
 
 namespace ccdi {
@@ -50,6 +46,16 @@ int set_err(ccd_ctx* c, int code, const std::string& msg) {
 
 void dfree(void* p) {
     if (p) (void)hipFree(p);
+}
+
+int ensure_stage(ccd_ctx* c, size_t count) {
+    if (c->stage && c->stage_cap >= count) return CCD_OK;
+    dfree(c->stage);
+    c->stage = nullptr;
+    c->stage_cap = 0;
+    HIP_TRY(c, dalloc(&c->stage, count));
+    c->stage_cap = count;
+    return CCD_OK;
 }
 
 void free_tiled(TiledLayout& T) {
@@ -82,6 +88,8 @@ void free_layout(DevLayout& L) {
     dfree(L.split_beg);
     dfree(L.partials);
     dfree(L.pair);
+    dfree(L.src);
+    dfree(L.dperm);
     L = DevLayout{};
 }
 
@@ -316,33 +324,78 @@ int do_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* xs, co
 using PassFn = int (*)(ccd_ctx*, DevLayout&, const void*, void*, const void*, const void*, const void*,
                       const void*, bool, bool, bool, bool, float, int);
 
-int upload_layout(ccd_ctx* c, DevLayout& L, int64_t rows, int64_t gdim, uint64_t nnz, const uint32_t* ptr,
-                  const uint32_t* idx, const float* val) {
+// Device memory of one set-up call.
+template <class T>
+struct Scratch {
+    T* p = nullptr;
+    Scratch() = default;
+    Scratch(const Scratch&) = delete;
+    Scratch& operator=(const Scratch&) = delete;
+    ~Scratch() { release(); }
+    hipError_t alloc(size_t count) { return dalloc(&p, count); }
+    void release() {
+        dfree(p);
+        p = nullptr;
+    }
+};
+
+// One compressed copy into internal numbering: its rows in `perm` order (by
+// falling length), indices through ipos (device, caller's index ->
+// internal), the elements of every row sorted by internal index.  didx: the
+// caller's indices on the device, checked.
+int upload_layout(ccd_ctx* c, DevLayout& L, int64_t rows, int64_t gdim, uint64_t nnz, const uint32_t* cptr,
+                  const uint32_t* didx, const float* val, const std::vector<uint32_t>& perm, const uint32_t* ipos) {
     L.rows = rows;
     L.gdim = gdim;
     L.nnz = nnz;
     L.idx16 = gdim <= 65536;
-    L.hptr.assign(ptr, ptr + rows + 1);
     L.split_cap = 0;
+    L.hptr.resize((size_t)rows + 1);
+    L.hptr[0] = 0;
+    ccd::RenumRows cls{0, 0, 0, 0};
+    const uint32_t long_len = ccd::renum_long_len((uint32_t)gdim);
+    for (int64_t i = 0; i < rows; ++i) {
+        const uint32_t len = cptr[perm[i] + 1] - cptr[perm[i]];
+        L.hptr[i + 1] = L.hptr[i] + len;
+        if (len > long_len) {
+            ++cls.nlong;
+            cls.long_elems = L.hptr[i + 1];
+        } else if (len > ccd::RENUM_SHORT) {
+            ++cls.nmid;
+        } else if (len) {
+            ++cls.nshort;
+        }
+    }
+    const uint32_t* ptr = L.hptr.data();
     HIP_TRY(c, dalloc(&L.ptr, rows + 1));
-    HIP_TRY(c, ccd::copy_sync(c->stream, L.ptr, ptr, sizeof(uint32_t) * (rows + 1), hipMemcpyHostToDevice));
-    if (L.idx16) {
-        std::vector<uint16_t> tmp(nnz);
-        for (uint64_t e = 0; e < nnz; ++e) tmp[e] = (uint16_t)idx[e];
-        uint16_t* d = nullptr;
-        HIP_TRY(c, dalloc(&d, nnz));
+    HIP_TRY(c, hipMemcpyAsync(L.ptr, ptr, sizeof(uint32_t) * (rows + 1), hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, dalloc(&L.dperm, rows));
+    HIP_TRY(c, hipMemcpyAsync(L.dperm, perm.data(), sizeof(uint32_t) * rows, hipMemcpyHostToDevice, c->stream));
+    {
+        uint8_t* d = nullptr;
+        HIP_TRY(c, dalloc(&d, (L.idx16 ? 2 : 4) * (size_t)nnz));
         L.idx = d;
-        HIP_TRY(c, ccd::copy_sync(c->stream, d, tmp.data(), sizeof(uint16_t) * nnz, hipMemcpyHostToDevice));
-    } else {
-        uint32_t* d = nullptr;
-        HIP_TRY(c, dalloc(&d, nnz));
-        L.idx = d;
-        HIP_TRY(c, ccd::copy_sync(c->stream, d, idx, sizeof(uint32_t) * nnz, hipMemcpyHostToDevice));
     }
     HIP_TRY(c, dalloc(&L.val, nnz));
     HIP_TRY(c, dalloc(&L.val0, nnz));
-    HIP_TRY(c, ccd::copy_sync(c->stream, L.val0, val, sizeof(float) * nnz, hipMemcpyHostToDevice));
-    HIP_TRY(c, ccd::copy_sync(c->stream, L.val, L.val0, sizeof(float) * nnz, hipMemcpyDeviceToDevice));
+    HIP_TRY(c, dalloc(&L.src, nnz));
+    if (nnz) {
+        // the caller's values pass through L.val
+        Scratch<uint32_t> dptr, dup;
+        HIP_TRY(c, dptr.alloc((size_t)rows + 1));
+        HIP_TRY(c, dup.alloc((size_t)cls.nlong + 1));
+        HIP_TRY(c, hipMemcpyAsync(dptr.p, cptr, sizeof(uint32_t) * (rows + 1), hipMemcpyHostToDevice, c->stream));
+        HIP_TRY(c, hipMemcpyAsync(L.val, val, sizeof(float) * nnz, hipMemcpyHostToDevice, c->stream));
+        const ccd::RenumArgs ra{dptr.p, didx, L.val, L.dperm, ipos, L.ptr, L.idx, L.val0, L.src, (uint32_t)gdim};
+        const hipError_t e1 = ccd::launch_renumber(ra, L.idx16, cls, dup.p, c->stream);
+        const hipError_t e2 = hipMemcpyAsync(L.val, L.val0, sizeof(float) * nnz, hipMemcpyDeviceToDevice, c->stream);
+        const hipError_t e3 = hipStreamSynchronize(c->stream);  // before dptr and dup go
+        HIP_TRY(c, e1);
+        HIP_TRY(c, e2);
+        HIP_TRY(c, e3);
+    } else {
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+    }
 
     HostPlan P = make_plan(ptr, rows, c->plan);
     if (P.split_beg.back() >= (1u << 24) || P.units.size() >= 0xffffffffull)
@@ -482,71 +535,54 @@ int do_tiled_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* 
     return CCD_OK;
 }
 
-// Positions sorted by falling degree (stable).
+// Positions sorted by falling degree (stable): a counting sort, unless one
+// degree far exceeds the row count.
 std::vector<uint32_t> degree_order(const uint32_t* ptr, int64_t rows) {
     std::vector<uint32_t> perm((size_t)rows);
-    for (int64_t r = 0; r < rows; ++r) perm[r] = (uint32_t)r;
-    std::stable_sort(perm.begin(), perm.end(),
-                     [&](uint32_t a, uint32_t b) { return ptr[a + 1] - ptr[a] > ptr[b + 1] - ptr[b]; });
+    uint32_t top = 0;
+    for (int64_t r = 0; r < rows; ++r) top = std::max(top, ptr[r + 1] - ptr[r]);
+    if ((uint64_t)top > 4ull * (uint64_t)rows + (1u << 20)) {
+        for (int64_t r = 0; r < rows; ++r) perm[r] = (uint32_t)r;
+        std::stable_sort(perm.begin(), perm.end(),
+                         [&](uint32_t a, uint32_t b) { return ptr[a + 1] - ptr[a] > ptr[b + 1] - ptr[b]; });
+        return perm;
+    }
+    std::vector<uint32_t> at((size_t)top + 2, 0u);  // at[d]: place of the next row of degree d
+    for (int64_t r = 0; r < rows; ++r) ++at[ptr[r + 1] - ptr[r]];
+    uint32_t place = 0;
+    for (uint32_t d = top + 1; d-- > 0;) {
+        const uint32_t count = at[d];
+        at[d] = place;
+        place += count;
+    }
+    for (int64_t r = 0; r < rows; ++r) perm[at[ptr[r + 1] - ptr[r]]++] = (uint32_t)r;
     return perm;
 }
 
-// Element order inside each row of a renumbered layout: the caller's, or
-// ascending internal index (so that a row splits at any bound into the
-// elements gathered from below it and the rest, and a lane's consecutive
-// elements beyond the LDS prefix share cache lines).
-enum class RowOrder { keep, sort };
-
-// One compressed layout in internal numbering: rows in `perm` order, indices
-// mapped through `ipos` (caller's index -> internal), elements inside each
-// row in `order` (equal sort keys keep their order).  src[o]: the caller's
-// position of internal element o.  Rows are processed in parallel, in
-// chunks taken from a shared counter.
-void renumber(int64_t rows, const uint32_t* ptr, const uint32_t* idx, const float* val,
-              const std::vector<uint32_t>& perm, const std::vector<uint32_t>& ipos, std::vector<uint32_t>& optr,
-              std::vector<uint32_t>& oidx, std::vector<float>& oval, std::vector<uint32_t>& src, RowOrder order) {
-    optr.assign((size_t)rows + 1, 0u);
-    for (int64_t i = 0; i < rows; ++i) optr[i + 1] = optr[i] + (ptr[perm[i] + 1] - ptr[perm[i]]);
-    oidx.resize(optr[rows]);
-    oval.resize(optr[rows]);
-    src.resize(optr[rows]);
-    constexpr int64_t CHUNK = 512;
-    std::atomic<int64_t> next{0};
-    auto work = [&]() {
-        std::vector<uint64_t> key;
-        for (int64_t b; (b = next.fetch_add(CHUNK)) < rows;) {
-            for (int64_t i = b; i < std::min(rows, b + CHUNK); ++i) {
-                const uint32_t r = perm[i], e0 = ptr[r], len = ptr[r + 1] - ptr[r];
-                key.resize(len);
-                for (uint32_t q = 0; q < len; ++q)
-                    key[q] = (uint64_t)(order == RowOrder::sort ? ipos[idx[e0 + q]] : 0u) << 32 | q;
-                if (order != RowOrder::keep) std::sort(key.begin(), key.end());
-                const uint32_t o = optr[i];
-                for (uint32_t q = 0; q < len; ++q) {
-                    const uint32_t e = e0 + (uint32_t)key[q];
-                    oidx[o + q] = ipos[idx[e]];
-                    oval[o + q] = val[e];
-                    src[o + q] = e;
-                }
-            }
-        }
-    };
-    const uint64_t nnz = optr[rows];
-    const unsigned nt = nnz < (1u << 20) ? 1u : std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    std::vector<std::thread> pool;
-    for (unsigned t = 1; t < nt; ++t) pool.emplace_back(work);
-    work();
-    for (auto& th : pool) th.join();
-}
-
-const char* check_compressed(int64_t rows, int64_t dim, uint64_t nnz, const uint32_t* ptr, const uint32_t* idx) {
+const char* check_pointers(int64_t rows, uint64_t nnz, const uint32_t* ptr) {
     if (ptr[0] != 0) return "pointer array must start at 0";
     for (int64_t r = 0; r < rows; ++r)
         if (ptr[r + 1] < ptr[r]) return "pointer array is not monotone";
     if ((uint64_t)ptr[rows] != nnz) return "last pointer differs from nnz";
-    for (uint64_t e = 0; e < nnz; ++e)
-        if ((int64_t)idx[e] >= dim) return "index out of range";
     return nullptr;
+}
+
+// The caller's indices on the device, checked there: *out_of_range set when
+// one is not below dim.
+int upload_indices(ccd_ctx* c, Scratch<uint32_t>& d, const uint32_t* idx, uint64_t nnz, int64_t dim,
+                   bool* out_of_range) {
+    *out_of_range = false;
+    if (nnz == 0) return CCD_OK;
+    Scratch<uint32_t> flag;
+    HIP_TRY(c, d.alloc(nnz));
+    HIP_TRY(c, flag.alloc(1));
+    uint32_t bad = 0;
+    HIP_TRY(c, hipMemcpyAsync(d.p, idx, sizeof(uint32_t) * nnz, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, ccd::launch_fill(reinterpret_cast<float*>(flag.p), 0.0f, 1, c->stream));
+    HIP_TRY(c, ccd::launch_index_check(d.p, nnz, (uint32_t)dim, flag.p, c->stream));
+    HIP_TRY(c, ccd::copy_sync(c->stream, &bad, flag.p, sizeof(bad), hipMemcpyDeviceToHost));
+    *out_of_range = bad != 0;
+    return CCD_OK;
 }
 
 }  // namespace ccdi
@@ -628,6 +664,7 @@ int32_t ccd_destroy(ccd_ctx* c) {
     dfree(c->H16);
     dfree(c->u16);
     dfree(c->v16);
+    dfree(c->stage);
     dfree(c->rmse_bsum);
     dfree(c->rmse_dev);
     dfree(c->obj_dev);
@@ -660,10 +697,18 @@ int32_t ccd_upload(ccd_ctx* c, int64_t m, int64_t n, uint64_t nnz, const uint32_
         return set_err(c, CCD_ERR_INVALID, "shape out of range (m, n < 2^31, nnz < 2^32)");
     if (!row_ptr || !col_ptr || (nnz && (!col_idx || !csr_val || !row_idx || !csc_val)))
         return set_err(c, CCD_ERR_INVALID, "null array");
-    if (const char* why = check_compressed(m, n, nnz, row_ptr, col_idx)) return set_err(c, CCD_ERR_INVALID, std::string("CSR: ") + why);
-    if (const char* why = check_compressed(n, m, nnz, col_ptr, row_idx)) return set_err(c, CCD_ERR_INVALID, std::string("CSC: ") + why);
+    if (const char* why = check_pointers(m, nnz, row_ptr)) return set_err(c, CCD_ERR_INVALID, std::string("CSR: ") + why);
     HIP_TRY(c, hipSetDevice(c->device));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
+    // every check comes before the first change: a refused upload leaves the
+    // context as it was
+    Scratch<uint32_t> ridx, kidx;
+    bool bad = false;
+    if (int rc = upload_indices(c, ridx, col_idx, nnz, n, &bad)) return rc;
+    if (bad) return set_err(c, CCD_ERR_INVALID, "CSR: index out of range");
+    if (const char* why = check_pointers(n, nnz, col_ptr)) return set_err(c, CCD_ERR_INVALID, std::string("CSC: ") + why);
+    if (int rc = upload_indices(c, kidx, row_idx, nnz, m, &bad)) return rc;
+    if (bad) return set_err(c, CCD_ERR_INVALID, "CSC: index out of range");
     drop_graph(c);
     ++c->gen;
     free_layout(c->csr);
@@ -678,19 +723,17 @@ int32_t ccd_upload(ccd_ctx* c, int64_t m, int64_t n, uint64_t nnz, const uint32_
         std::vector<uint32_t> rpos((size_t)m), cpos((size_t)n);
         for (int64_t i = 0; i < m; ++i) rpos[rperm[i]] = (uint32_t)i;
         for (int64_t j = 0; j < n; ++j) cpos[cperm[j]] = (uint32_t)j;
-        std::vector<uint32_t> p2, i2, src;
-        std::vector<float> v2;
         // Rows sorted by gathered index: the tiled sweeps can then split
         // each row at any bound (build_tiled) and keep the elements gathered
         // from beyond an LDS prefix in tiles of their own.
-        renumber(m, row_ptr, col_idx, csr_val, rperm, cpos, p2, i2, v2, src, RowOrder::sort);
-        int rc = upload_layout(c, c->csr, m, n, nnz, p2.data(), i2.data(), v2.data());
-        if (rc) return rc;
-        c->csr.src = std::move(src);
-        renumber(n, col_ptr, row_idx, csc_val, cperm, rpos, p2, i2, v2, src, RowOrder::sort);
-        rc = upload_layout(c, c->csc, n, m, nnz, p2.data(), i2.data(), v2.data());
-        if (rc) return rc;
-        c->csc.src = std::move(src);
+        Scratch<uint32_t> drpos, dcpos;
+        HIP_TRY(c, drpos.alloc((size_t)m));
+        HIP_TRY(c, dcpos.alloc((size_t)n));
+        HIP_TRY(c, ccd::copy_sync(c->stream, drpos.p, rpos.data(), sizeof(uint32_t) * (size_t)m, hipMemcpyHostToDevice));
+        HIP_TRY(c, ccd::copy_sync(c->stream, dcpos.p, cpos.data(), sizeof(uint32_t) * (size_t)n, hipMemcpyHostToDevice));
+        if (int rc = upload_layout(c, c->csr, m, n, nnz, row_ptr, ridx.p, csr_val, rperm, dcpos.p)) return rc;
+        ridx.release();
+        if (int rc = upload_layout(c, c->csc, n, m, nnz, col_ptr, kidx.p, csc_val, cperm, drpos.p)) return rc;
         c->csr.perm = std::move(rperm);
         c->csc.perm = std::move(cperm);
     }
@@ -767,17 +810,17 @@ int32_t ccd_set_factors(ccd_ctx* c, uint32_t k, const float* W, const float* H) 
         HIP_TRY(c, dalloc(&c->H, (size_t)k * c->n));
         c->k = k;
     }
-    {
-        std::vector<float> t2((size_t)k * std::max(c->m, c->n));
-        for (uint32_t t = 0; t < k; ++t)
-            for (int64_t i = 0; i < c->m; ++i) t2[(size_t)t * c->m + i] = W[(size_t)t * c->m + c->csr.perm[i]];
-        HIP_TRY(c, ccd::copy_sync(c->stream, c->W, t2.data(), sizeof(float) * (size_t)k * c->m, hipMemcpyHostToDevice));
-        for (uint32_t t = 0; t < k; ++t)
-            for (int64_t j = 0; j < c->n; ++j) t2[(size_t)t * c->n + j] = H[(size_t)t * c->n + c->csc.perm[j]];
-        HIP_TRY(c, ccd::copy_sync(c->stream, c->H, t2.data(), sizeof(float) * (size_t)k * c->n, hipMemcpyHostToDevice));
+    const size_t nW = (size_t)k * c->m, nH = (size_t)k * c->n;
+    if (int rc = ensure_stage(c, std::max(nW, nH))) return rc;
+    HIP_TRY(c, hipMemcpyAsync(c->stage, W, sizeof(float) * nW, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, ccd::launch_permute_ranks(c->stage, c->W, c->csr.dperm, k, c->m, true, c->stream));
+    HIP_TRY(c, hipMemcpyAsync(c->stage, H, sizeof(float) * nH, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, ccd::launch_permute_ranks(c->stage, c->H, c->csc.dperm, k, c->n, true, c->stream));
+    if (c->nnz) {
+        HIP_TRY(c, hipMemcpyAsync(c->csr.val, c->csr.val0, 4 * c->nnz, hipMemcpyDeviceToDevice, c->stream));
+        HIP_TRY(c, hipMemcpyAsync(c->csc.val, c->csc.val0, 4 * c->nnz, hipMemcpyDeviceToDevice, c->stream));
     }
-    HIP_TRY(c, ccd::copy_sync(c->stream, c->csr.val, c->csr.val0, 4 * c->nnz, hipMemcpyDeviceToDevice));
-    HIP_TRY(c, ccd::copy_sync(c->stream, c->csc.val, c->csc.val0, 4 * c->nnz, hipMemcpyDeviceToDevice));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
     c->factors = true;
     c->continued = false;
     return CCD_OK;
@@ -1073,16 +1116,14 @@ int32_t ccd_get_factors(ccd_ctx* c, float* W, float* H) {
     HIP_TRY(c, hipSetDevice(c->device));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     const uint32_t k = c->k;
-    std::vector<float> t2((size_t)k * std::max(c->m, c->n));
-    if (W) {
-        HIP_TRY(c, hipMemcpy(t2.data(), c->W, sizeof(float) * (size_t)k * c->m, hipMemcpyDeviceToHost));
-        for (uint32_t t = 0; t < k; ++t)
-            for (int64_t i = 0; i < c->m; ++i) W[(size_t)t * c->m + c->csr.perm[i]] = t2[(size_t)t * c->m + i];
-    }
-    if (H) {
-        HIP_TRY(c, hipMemcpy(t2.data(), c->H, sizeof(float) * (size_t)k * c->n, hipMemcpyDeviceToHost));
-        for (uint32_t t = 0; t < k; ++t)
-            for (int64_t j = 0; j < c->n; ++j) H[(size_t)t * c->n + c->csc.perm[j]] = t2[(size_t)t * c->n + j];
+    const size_t nW = (size_t)k * c->m, nH = (size_t)k * c->n;
+    if (int rc = ensure_stage(c, std::max(nW, nH))) return rc;
+    for (int q = 0; q < 2; ++q) {
+        float* out = q == 0 ? W : H;
+        if (!out) continue;
+        HIP_TRY(c, ccd::launch_permute_ranks(q == 0 ? c->W : c->H, c->stage, q == 0 ? c->csr.dperm : c->csc.dperm, k,
+                                             q == 0 ? c->m : c->n, false, c->stream));
+        HIP_TRY(c, ccd::copy_sync(c->stream, out, c->stage, sizeof(float) * (q == 0 ? nW : nH), hipMemcpyDeviceToHost));
     }
     return CCD_OK;
 }
@@ -1092,13 +1133,14 @@ int32_t ccd_get_residual(ccd_ctx* c, float* csr_val, float* csc_val) {
     if (!c->uploaded) return set_err(c, CCD_ERR_STATE, "nothing uploaded");
     HIP_TRY(c, hipSetDevice(c->device));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    std::vector<float> tmp(c->nnz);
+    if (c->nnz == 0) return CCD_OK;
+    if (int rc = ensure_stage(c, c->nnz)) return rc;
     for (int q = 0; q < 2; ++q) {
         float* out = q == 0 ? csr_val : csc_val;
         const DevLayout& L = q == 0 ? c->csr : c->csc;
         if (!out) continue;
-        HIP_TRY(c, hipMemcpy(tmp.data(), L.val, 4 * c->nnz, hipMemcpyDeviceToHost));
-        for (uint64_t e = 0; e < c->nnz; ++e) out[L.src[e]] = tmp[e];
+        HIP_TRY(c, ccd::launch_scatter(L.val, L.src, c->stage, c->nnz, c->stream));
+        HIP_TRY(c, ccd::copy_sync(c->stream, out, c->stage, 4 * c->nnz, hipMemcpyDeviceToHost));
     }
     return CCD_OK;
 }

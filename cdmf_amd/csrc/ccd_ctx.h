@@ -73,13 +73,14 @@ struct DevLayout {
     uint64_t split_cap = 0;
     uint32_t split_x = 0, split_p = 0;
     std::vector<uint32_t> hptr;      // host copy of the internal ptr (planning)
-    std::vector<uint32_t> src;       // caller's position of each internal element (residual download)
+    uint32_t* src = nullptr;         // caller's position of each internal element (residual download)
     // Split of the current tiled layout (build_tiled): rows, whose elements
     // ascend by internal index, split at split_at (0: not split); below[i]
     // leading elements of row i are gathered from below it.
     uint32_t split_at = 0;
     std::vector<uint32_t> below;
     std::vector<uint32_t> perm;      // internal row -> caller's row
+    uint32_t* dperm = nullptr;       // the same on the device
     TiledLayout tl;
 };
 
@@ -121,6 +122,10 @@ struct ccd_ctx {
     int lds_block = 0;         // LDS bytes a block may use
     int lds_cu = 0;            // LDS bytes of a CU
     std::map<uint32_t, int> occupancy;  // persistent kernel -> blocks per CU by register use
+    // grow-only staging of the caller's arrays on the device (factors and
+    // residual on their way between the two numberings)
+    float* stage = nullptr;
+    size_t stage_cap = 0;
     double* rmse_bsum = nullptr;
     double* rmse_dev = nullptr;  // one slot per outer iteration
     double* obj_dev = nullptr;   // objective, loss, regulariser
@@ -162,6 +167,8 @@ hipError_t dalloc(T** p, size_t count) {
 }
 
 void dfree(void* p);
+// Context staging of at least `count` floats (ccd_ctx::stage).
+int ensure_stage(ccd_ctx* c, size_t count);
 void drop_graph(ccd_ctx* c);
 // Bytes per index of the tiled copy of L: 2 up to 2^16 gathered entries, 3
 // up to 2^24, else 4.

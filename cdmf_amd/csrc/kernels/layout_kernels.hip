@@ -1,0 +1,281 @@
+// Set-up kernels of a solver context: the caller's numbering to the internal
+// one and back.  Factors, residual and index arrays cross the ABI in the
+// caller's order; the permutations, the renumbering of both compressed
+// copies and the sort inside each row run here, so that a set-up call costs
+// its copies over PCIe and little else.
+#include "layout.h"
+
+#include "ccd_kernels.h"
+
+#include <algorithm>
+
+namespace ccd {
+namespace {
+
+constexpr int WAVE = 64;
+constexpr int BLOCK = 256;
+constexpr uint32_t RANKS_PER_BLOCK = 8;  // ranks a block of permute_ranks_kernel walks
+
+// Rank-major [k][rows] factors between the caller's numbering and the
+// internal one (perm: internal -> caller's).  Bound by the random side, 4 B
+// an entry out of one rank's row (at most a few MB, so L2 serves it); the
+// other side and perm are coalesced, and perm is read once for
+// RANKS_PER_BLOCK ranks.
+template <bool TO_INTERNAL>
+__global__ __launch_bounds__(BLOCK) void permute_ranks_kernel(const float* __restrict__ src, float* __restrict__ dst,
+                                                              const uint32_t* __restrict__ perm, uint32_t k,
+                                                              uint64_t rows) {
+    const uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= rows) return;
+    const uint64_t r = perm[i];
+    for (uint32_t t0 = blockIdx.y * RANKS_PER_BLOCK; t0 < k; t0 += gridDim.y * RANKS_PER_BLOCK) {
+        const uint32_t t1 = min(k, t0 + RANKS_PER_BLOCK);
+#pragma unroll 8
+        for (uint32_t t = t0; t < t1; ++t) {
+            if (TO_INTERNAL) dst[t * rows + i] = src[t * rows + r];
+            else dst[t * rows + r] = src[t * rows + i];
+        }
+    }
+}
+
+// dst[map[e]] = src[e]
+__global__ __launch_bounds__(BLOCK) void scatter_kernel(const float* __restrict__ src,
+                                                        const uint32_t* __restrict__ map, float* __restrict__ dst,
+                                                        uint64_t count) {
+    const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
+    for (uint64_t e = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; e < count; e += stride) dst[map[e]] = src[e];
+}
+
+__global__ __launch_bounds__(BLOCK) void index_check_kernel(const uint32_t* __restrict__ idx, uint64_t count,
+                                                            uint32_t dim, uint32_t* __restrict__ bad) {
+    const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
+    bool b = false;
+    for (uint64_t e = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; e < count; e += stride) b |= idx[e] >= dim;
+    if (b) atomicOr(bad, 1u);
+}
+
+template <typename IdxT>
+__device__ __forceinline__ void put(const RenumArgs& a, uint32_t o, uint32_t key, uint32_t e) {
+    static_cast<IdxT*>(a.oidx)[o] = (IdxT)key;
+    a.oval[o] = a.val[e];
+    a.osrc[o] = e;
+}
+
+// Rows of at most RENUM_SHORT elements, one wave each: an element's place is
+// the number of elements before it in (index, caller's position) order,
+// counted against every lane's key in turn.
+template <typename IdxT>
+__global__ __launch_bounds__(BLOCK) void renum_short_kernel(RenumArgs a, uint32_t row0, uint32_t rows) {
+    const uint32_t w = blockIdx.x * (BLOCK / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (w >= rows) return;
+    const uint32_t row = row0 + w, lane = threadIdx.x & (WAVE - 1);
+    const uint32_t o = a.optr[row], len = a.optr[row + 1] - o, e = a.ptr[a.perm[row]] + lane;
+    const bool ok = lane < len;
+    const uint32_t key = ok ? a.ipos[a.idx[e]] : 0xffffffffu;
+    uint32_t rank = 0;
+    for (uint32_t j = 0; j < len; ++j) {
+        const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)key, (int)j);
+        rank += kj < key + (j < lane ? 1u : 0u) ? 1u : 0u;
+    }
+    if (ok) put<IdxT>(a, o + rank, key, e);
+}
+
+// Rows of RENUM_SHORT + 1 .. MID_MAX elements, one block each, the same
+// count against the row's keys in LDS (four a read, the same four for every
+// lane).  len^2 / 64 compares a wave: past the bound of renum_long_len the
+// bitmap below is cheaper.
+constexpr uint32_t MID_MAX = 1024;
+template <typename IdxT, int NQ>
+__device__ __forceinline__ void renum_mid_row(const RenumArgs& a, uint32_t* keys, uint32_t o, uint32_t len,
+                                              uint32_t e0) {
+    uint32_t key[NQ], rank[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const uint32_t p = threadIdx.x + BLOCK * q;
+        key[q] = p < len ? a.ipos[a.idx[e0 + p]] : 0xffffffffu;
+        rank[q] = 0;
+        keys[p] = key[q];  // past the row: larger than any key
+    }
+    __syncthreads();
+    for (uint32_t j = 0; j < len; j += 4) {
+        const uint4 k4 = *reinterpret_cast<const uint4*>(keys + j);
+        const uint32_t kj[4] = {k4.x, k4.y, k4.z, k4.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+                rank[q] += kj[u] < key[q] + (j + u < threadIdx.x + BLOCK * q ? 1u : 0u) ? 1u : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const uint32_t p = threadIdx.x + BLOCK * q;
+        if (p < len) put<IdxT>(a, o + rank[q], key[q], e0 + p);
+    }
+}
+
+template <typename IdxT>
+__global__ __launch_bounds__(BLOCK) void renum_mid_kernel(RenumArgs a, uint32_t row0) {
+    __shared__ __align__(16) uint32_t keys[MID_MAX];
+    const uint32_t row = row0 + blockIdx.x;
+    const uint32_t o = a.optr[row], len = a.optr[row + 1] - o, e0 = a.ptr[a.perm[row]];
+    if (len <= BLOCK) renum_mid_row<IdxT, 1>(a, keys, o, len, e0);
+    else if (len <= 2 * BLOCK) renum_mid_row<IdxT, 2>(a, keys, o, len, e0);
+    else renum_mid_row<IdxT, 4>(a, keys, o, len, e0);
+}
+
+// Longer rows, one block each: the row's indices are set in a bitmap of the
+// gathered dimension in LDS (in windows of WIN_WORDS words), and an
+// element's place is the number of bits set before its own (a prefix sum
+// per group of 8 words, then popcounts).  Linear in the row's length plus
+// gdim / 32.  An index that occurs twice in a row sets dup[row] and
+// dup[nlong]; renum_dup_kernel then places that row's elements by counting.
+constexpr uint32_t WIN_WORDS = 32768;  // 2^20 indices, 144 KB with the prefix sums
+constexpr uint32_t GROUP = 8;
+template <typename IdxT, int BS>
+__global__ __launch_bounds__(BS) void renum_long_kernel(RenumArgs a, uint32_t* __restrict__ dup, uint32_t words) {
+    extern __shared__ __align__(16) uint32_t bits[];  // words, then words / GROUP prefix sums
+    __shared__ uint32_t wsum[BS / WAVE];
+    uint32_t* pre = bits + words;
+    const uint32_t row = blockIdx.x, lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x >> 6;
+    const uint32_t o = a.optr[row], len = a.optr[row + 1] - o, e0 = a.ptr[a.perm[row]];
+    const uint32_t ng = words / GROUP, per = (ng + BS - 1) / BS;
+    uint32_t below = 0;
+    int twice = 0;
+    for (uint64_t w0 = 0; w0 < a.gdim; w0 += (uint64_t)words * 32) {
+        const uint32_t lo = (uint32_t)w0;
+        for (uint32_t q = threadIdx.x; q < words; q += BS) bits[q] = 0u;
+        __syncthreads();
+        for (uint32_t p = threadIdx.x; p < len; p += BS) {
+            const uint32_t k = a.ipos[a.idx[e0 + p]] - lo;  // wraps past the window for smaller indices
+            if (k < words * 32) {
+                const uint32_t bit = 1u << (k & 31u);
+                if (atomicOr(&bits[k >> 5], bit) & bit) twice = 1;
+            }
+        }
+        __syncthreads();
+        // exclusive prefix sums of the groups' bit counts
+        uint32_t mine = 0;
+        for (uint32_t g = threadIdx.x * per; g < min(ng, (threadIdx.x + 1) * per); ++g) {
+            pre[g] = mine;
+#pragma unroll
+            for (uint32_t u = 0; u < GROUP; ++u) mine += (uint32_t)__popc(bits[g * GROUP + u]);
+        }
+        uint32_t incl = mine;
+#pragma unroll
+        for (int d = 1; d < WAVE; d <<= 1) {
+            const uint32_t t = __shfl_up(incl, d);
+            if (lane >= (uint32_t)d) incl += t;
+        }
+        if (lane == WAVE - 1) wsum[wv] = incl;
+        __syncthreads();
+        uint32_t off = incl - mine, total = 0;
+        for (uint32_t q = 0; q < BS / WAVE; ++q) {
+            if (q < wv) off += wsum[q];
+            total += wsum[q];
+        }
+        for (uint32_t g = threadIdx.x * per; g < min(ng, (threadIdx.x + 1) * per); ++g) pre[g] += off;
+        __syncthreads();
+        for (uint32_t p = threadIdx.x; p < len; p += BS) {
+            const uint32_t key = a.ipos[a.idx[e0 + p]], k = key - lo;
+            if (k >= words * 32) continue;
+            const uint32_t w = k >> 5;
+            uint32_t rank = below + pre[w / GROUP] + (uint32_t)__popc(bits[w] & ((1u << (k & 31u)) - 1u));
+            for (uint32_t u = w / GROUP * GROUP; u < w; ++u) rank += (uint32_t)__popc(bits[u]);
+            put<IdxT>(a, o + rank, key, e0 + p);
+        }
+        below += total;
+        __syncthreads();
+    }
+    if (twice) {
+        dup[row] = 1u;
+        dup[gridDim.x] = 1u;
+    }
+}
+
+// Long rows that hold an index twice: every element counted against the
+// whole row.  Rare, so nothing is staged; without such a row the blocks
+// leave at once.
+template <typename IdxT>
+__global__ __launch_bounds__(BLOCK) void renum_dup_kernel(RenumArgs a, const uint32_t* __restrict__ dup,
+                                                          uint32_t nlong, uint32_t elems) {
+    if (!dup[nlong]) return;
+    for (uint64_t x = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; x < elems; x += (uint64_t)gridDim.x * BLOCK) {
+        uint32_t r0 = 0, r1 = nlong;  // row of layout position x
+        while (r1 - r0 > 1) {
+            const uint32_t mid = r0 + (r1 - r0) / 2;
+            if (a.optr[mid] <= x) r0 = mid;
+            else r1 = mid;
+        }
+        if (!dup[r0]) continue;
+        const uint32_t o = a.optr[r0], len = a.optr[r0 + 1] - o, e0 = a.ptr[a.perm[r0]];
+        const uint32_t p = (uint32_t)x - o, key = a.ipos[a.idx[e0 + p]];
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < len; ++j) rank += a.ipos[a.idx[e0 + j]] < key + (j < p ? 1u : 0u) ? 1u : 0u;
+        put<IdxT>(a, o + rank, key, e0 + p);
+    }
+}
+
+uint32_t grid_for(uint64_t count) {
+    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((count + BLOCK - 1) / BLOCK, 1), 16384);
+}
+
+}  // namespace
+
+hipError_t launch_permute_ranks(const float* src, float* dst, const uint32_t* perm, uint32_t k, uint64_t rows,
+                                bool to_internal, hipStream_t s) {
+    if (k == 0 || rows == 0) return hipSuccess;
+    const uint32_t y = std::min<uint32_t>((k + RANKS_PER_BLOCK - 1) / RANKS_PER_BLOCK, 65535u);
+    const dim3 grid((uint32_t)((rows + BLOCK - 1) / BLOCK), y);
+    if (to_internal)
+        hipLaunchKernelGGL(permute_ranks_kernel<true>, grid, dim3(BLOCK), 0, s, src, dst, perm, k, rows);
+    else
+        hipLaunchKernelGGL(permute_ranks_kernel<false>, grid, dim3(BLOCK), 0, s, src, dst, perm, k, rows);
+    return hipGetLastError();
+}
+
+hipError_t launch_scatter(const float* src, const uint32_t* map, float* dst, uint64_t count, hipStream_t s) {
+    if (count == 0) return hipSuccess;
+    hipLaunchKernelGGL(scatter_kernel, dim3(grid_for(count)), dim3(BLOCK), 0, s, src, map, dst, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_index_check(const uint32_t* idx, uint64_t count, uint32_t dim, uint32_t* bad, hipStream_t s) {
+    if (count == 0) return hipSuccess;
+    hipLaunchKernelGGL(index_check_kernel, dim3(grid_for(count)), dim3(BLOCK), 0, s, idx, count, dim, bad);
+    return hipGetLastError();
+}
+
+// Where a block's count over 256 keys and the bitmap of a small gathered
+// dimension cost about the same; a bitmap past 8 KB takes longer to clear
+// and sum than to count four times as many keys.
+uint32_t renum_long_len(uint32_t gdim) { return gdim <= 65536u ? 256u : MID_MAX; }
+
+template <typename IdxT>
+static hipError_t renumber(const RenumArgs& a, const RenumRows& n, uint32_t* dup, hipStream_t s) {
+    if (n.nlong) {
+        hipError_t e = launch_fill(reinterpret_cast<float*>(dup), 0.0f, (uint64_t)n.nlong + 1, s);
+        if (e != hipSuccess) return e;
+        const uint32_t words = std::min<uint32_t>((uint32_t)((((uint64_t)a.gdim + 31) / 32 + GROUP - 1) / GROUP * GROUP),
+                                                  WIN_WORDS);
+        const size_t lds = sizeof(uint32_t) * (words + words / GROUP);
+        if (words <= 2048)
+            hipLaunchKernelGGL((renum_long_kernel<IdxT, 256>), dim3(n.nlong), dim3(256), lds, s, a, dup, words);
+        else
+            hipLaunchKernelGGL((renum_long_kernel<IdxT, 1024>), dim3(n.nlong), dim3(1024), lds, s, a, dup, words);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL(renum_dup_kernel<IdxT>, dim3(grid_for(n.long_elems)), dim3(BLOCK), 0, s, a, dup, n.nlong,
+                           n.long_elems);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    if (n.nmid) hipLaunchKernelGGL(renum_mid_kernel<IdxT>, dim3(n.nmid), dim3(BLOCK), 0, s, a, n.nlong);
+    if (n.nshort)
+        hipLaunchKernelGGL(renum_short_kernel<IdxT>, dim3((n.nshort + BLOCK / WAVE - 1) / (BLOCK / WAVE)), dim3(BLOCK),
+                           0, s, a, n.nlong + n.nmid, n.nshort);
+    return hipGetLastError();
+}
+
+hipError_t launch_renumber(const RenumArgs& a, bool idx16, const RenumRows& n, uint32_t* dup, hipStream_t s) {
+    return idx16 ? renumber<uint16_t>(a, n, dup, s) : renumber<uint32_t>(a, n, dup, s);
+}
+
+}  // namespace ccd
