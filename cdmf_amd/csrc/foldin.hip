@@ -3,6 +3,7 @@
 // the fold-in of new rows (kernels/foldin_kernels.hip).
 #include "cdmf_foldin.h"
 #include "ccd_kernels.h"
+#include "layout.h"
 
 #include <algorithm>
 #include <cmath>
@@ -453,12 +454,10 @@ int32_t ccd_mlp_train(ccd_mlp* m, uint64_t rows, const float* X, const float* T,
 
 // ------------------------------------------------- allocation-free path ---
 // Scratch of ccd_fold_rows_noalloc: one call's staged batch -- row pointer,
-// long-row list, indices, values, the per-rating residual buffer of the long
-// rows, start factors and result factors -- carved from one file-scope
-// device array.  Every GPU the library runs on holds its own copy (about
-// 28 MB) until the process ends.  Calls on one GPU share it: calls that
-// overlap on one GPU race.  Nothing in it needs to start at zero (the sweep
-// kernel seeds the residual buffer from the values, and W from W0 or 0).
+// long-row list, indices, values, start factors and result factors -- carved
+// from one file-scope device array.  Every GPU the library runs on holds its
+// own copy (about 20 MB) until the process ends.  Calls on one GPU share it:
+// calls that overlap on one GPU race.  Nothing in it needs to start at zero.
 namespace {
 constexpr uint64_t NA_MAX_ROWS = 4096;
 constexpr uint64_t NA_MAX_NNZ = 1ull << 21;
@@ -467,8 +466,7 @@ constexpr size_t NA_OFF_PTR = 0;
 constexpr size_t NA_OFF_LONG = NA_OFF_PTR + na_round(4 * (NA_MAX_ROWS + 1));
 constexpr size_t NA_OFF_IDX = NA_OFF_LONG + na_round(4 * NA_MAX_ROWS);
 constexpr size_t NA_OFF_VAL = NA_OFF_IDX + na_round(4 * NA_MAX_NNZ);
-constexpr size_t NA_OFF_RBUF = NA_OFF_VAL + na_round(4 * NA_MAX_NNZ);
-constexpr size_t NA_OFF_W0 = NA_OFF_RBUF + na_round(4 * NA_MAX_NNZ);
+constexpr size_t NA_OFF_W0 = NA_OFF_VAL + na_round(4 * NA_MAX_NNZ);
 constexpr size_t NA_OFF_W = NA_OFF_W0 + na_round(4 * NA_MAX_ROWS * ccd::FOLD_KMAX);
 constexpr size_t NA_BYTES = NA_OFF_W + na_round(4 * NA_MAX_ROWS * ccd::FOLD_KMAX);
 }  // namespace
@@ -504,16 +502,24 @@ struct ccd_fold {
     uint32_t k = 0;
     int64_t n = 0;
     float lambda = 0.0f;
-    float *H = nullptr, *HT = nullptr;
+    float* HT = nullptr;  // [n + 1][fold_ld(k)], ccd::FoldArgs
     uint32_t *ptr = nullptr, *idx = nullptr, *long_rows = nullptr;
-    uint32_t nlong = 0;
-    float *val = nullptr, *rbuf = nullptr, *W0 = nullptr, *W = nullptr, *F = nullptr;
-    size_t cap_ptr = 0, cap_idx = 0, cap_val = 0, cap_rbuf = 0, cap_w0 = 0, cap_w = 0, cap_f = 0, cap_long = 0;
+    uint32_t* bad = nullptr;  // fold_check_device
+    uint32_t nlong = 0, nfeat = 0;  // rows longer than FOLD_WAVE, and than FOLD_SHORT
+    float *val = nullptr, *W0 = nullptr, *W = nullptr, *F = nullptr;
+    size_t cap_ptr = 0, cap_idx = 0, cap_val = 0, cap_w0 = 0, cap_w = 0, cap_f = 0, cap_long = 0;
     hipEvent_t ea = nullptr, eb = nullptr;
     unsigned char* scratch = nullptr;  // this device's scratch (ccd_fold_rows_noalloc)
 };
 
 namespace {
+
+// Ratings from which the index check runs on the device: the host's loop takes
+// about 0.5 ns a rating (5 ms of a 9.9M-rating batch), the device's about 25 us
+// with its wait.
+constexpr uint64_t DEVICE_CHECK = 65536;
+
+uint32_t fold_ld(uint32_t k) { return (k + 15) & ~15u; }  // row length of HT
 
 int fold_check(ccd_fold* f, int64_t rows, const uint32_t* ptr, const uint32_t* idx, const float* val) {
     if (rows < 0 || rows > 0x7fffffff || !ptr || (rows && !idx && ptr[rows] > 0) || (rows && !val && ptr[rows] > 0))
@@ -522,32 +528,66 @@ int fold_check(ccd_fold* f, int64_t rows, const uint32_t* ptr, const uint32_t* i
     for (int64_t i = 0; i < rows; ++i)
         if (ptr[i + 1] < ptr[i]) return obj_err(f->err, CCD_ERR_INVALID, "ptr not monotone");
     const uint64_t nnz = ptr[rows];
+    if (nnz >= DEVICE_CHECK) return CCD_OK;  // indices: fold_check_device
     for (uint64_t e = 0; e < nnz; ++e)
         if ((int64_t)idx[e] >= f->n) return obj_err(f->err, CCD_ERR_INVALID, "column index out of range");
     return CCD_OK;
+}
+
+// The index check of a large batch on the device, before anything reads
+// through the indices.  didx: the batch's indices, their copy in the stream.
+int fold_check_device(ccd_fold* f, const uint32_t* didx, uint64_t nnz) {
+    if (nnz < DEVICE_CHECK) return CCD_OK;
+    uint32_t bad = 0;
+    OBJ_TRY(f, ccd::launch_fill(reinterpret_cast<float*>(f->bad), 0.0f, 1, f->stream));
+    OBJ_TRY(f, ccd::launch_index_check(didx, nnz, (uint32_t)f->n, f->bad, f->stream));
+    OBJ_TRY(f, ccd::copy_sync(f->stream, &bad, f->bad, sizeof(bad), hipMemcpyDeviceToHost));
+    return bad ? obj_err(f->err, CCD_ERR_INVALID, "column index out of range") : CCD_OK;
+}
+
+uint32_t count_long(int64_t rows, const uint32_t* ptr, uint32_t len) {
+    uint32_t c = 0;
+    for (int64_t i = 0; i < rows; ++i) c += ptr[i + 1] - ptr[i] > len ? 1u : 0u;
+    return c;
+}
+
+// Rows of more than FOLD_WAVE ratings by falling length class (the binary
+// exponent of length - 1; FOLD_WAVE and FOLD_SHORT are class bounds), in row
+// order inside a class: the costliest blocks of a launch start first.
+void list_long(int64_t rows, const uint32_t* ptr, uint32_t* out) {
+    static_assert((ccd::FOLD_WAVE & (ccd::FOLD_WAVE - 1)) == 0 && (ccd::FOLD_SHORT & (ccd::FOLD_SHORT - 1)) == 0,
+                  "length classes end at powers of two");
+    uint32_t at[33] = {};
+    auto cls = [&](int64_t i) { return __builtin_clz(ptr[i + 1] - ptr[i] - 1); };  // longer: smaller
+    for (int64_t i = 0; i < rows; ++i)
+        if (ptr[i + 1] - ptr[i] > ccd::FOLD_WAVE) ++at[cls(i) + 1];
+    for (int q = 1; q < 33; ++q) at[q] += at[q - 1];
+    for (int64_t i = 0; i < rows; ++i)
+        if (ptr[i + 1] - ptr[i] > ccd::FOLD_WAVE) out[at[cls(i)]++] = (uint32_t)i;
 }
 
 int fold_upload(ccd_fold* f, int64_t rows, const uint32_t* ptr, const uint32_t* idx, const float* val,
                 ccd::FoldArgs* a) {
     if (int rc = fold_check(f, rows, ptr, idx, val)) return rc;
     const uint64_t nnz = ptr[rows];
-    std::vector<uint32_t> lr;  // rows handled by a block each
-    for (int64_t i = 0; i < rows; ++i)
-        if (ptr[i + 1] - ptr[i] > ccd::FOLD_SHORT) lr.push_back((uint32_t)i);
+    std::vector<uint32_t> lr((size_t)count_long(rows, ptr, ccd::FOLD_WAVE));
+    list_long(rows, ptr, lr.data());
     OBJ_TRY(f, hipSetDevice(f->device));
     OBJ_TRY(f, ensure(&f->ptr, &f->cap_ptr, (size_t)rows + 1));
     OBJ_TRY(f, ensure(&f->idx, &f->cap_idx, nnz));
     OBJ_TRY(f, ensure(&f->val, &f->cap_val, nnz));
-    OBJ_TRY(f, ensure(&f->rbuf, &f->cap_rbuf, nnz));
     OBJ_TRY(f, ensure(&f->long_rows, &f->cap_long, lr.size()));
-    OBJ_TRY(f, ccd::copy_sync(f->stream, f->ptr, ptr, 4 * ((size_t)rows + 1), hipMemcpyHostToDevice));
+    OBJ_TRY(f, hipMemcpyAsync(f->ptr, ptr, 4 * ((size_t)rows + 1), hipMemcpyHostToDevice, f->stream));
+    // lr goes out of scope here, so its copy is complete on return
     if (!lr.empty()) OBJ_TRY(f, ccd::copy_sync(f->stream, f->long_rows, lr.data(), 4 * lr.size(), hipMemcpyHostToDevice));
     f->nlong = (uint32_t)lr.size();
+    f->nfeat = count_long(rows, ptr, ccd::FOLD_SHORT);
     if (nnz) {
-        OBJ_TRY(f, ccd::copy_sync(f->stream, f->idx, idx, 4 * nnz, hipMemcpyHostToDevice));
-        OBJ_TRY(f, ccd::copy_sync(f->stream, f->val, val, 4 * nnz, hipMemcpyHostToDevice));
+        OBJ_TRY(f, hipMemcpyAsync(f->idx, idx, 4 * nnz, hipMemcpyHostToDevice, f->stream));
+        OBJ_TRY(f, hipMemcpyAsync(f->val, val, 4 * nnz, hipMemcpyHostToDevice, f->stream));
+        if (int rc = fold_check_device(f, f->idx, nnz)) return rc;
     }
-    *a = ccd::FoldArgs{f->ptr, f->idx, f->val, f->H, f->HT, (uint32_t)rows, f->k, (uint32_t)f->n, 0, f->lambda};
+    *a = ccd::FoldArgs{f->ptr, f->idx, f->val, f->HT, (uint32_t)rows, f->k, fold_ld(f->k), (uint32_t)f->n, 0, f->lambda};
     return CCD_OK;
 }
 
@@ -567,13 +607,16 @@ int32_t ccd_fold_create(int32_t device, uint32_t k, int64_t n, const float* H, f
     ccd_fold* f = new (std::nothrow) ccd_fold();
     if (!f) return CCD_ERR_ALLOC;
     f->device = device, f->k = k, f->n = n, f->lambda = lambda;
-    const size_t kn = (size_t)k * n;
+    const size_t kn = (size_t)k * n, nht = ((size_t)n + 1) * fold_ld(k);
+    float* dH = nullptr;  // the caller's [k][n], until it is transposed
     bool ok = hipSetDevice(device) == hipSuccess && hipStreamCreateWithFlags(&f->stream, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreate(&f->ea) == hipSuccess && hipEventCreate(&f->eb) == hipSuccess &&
-              dalloc(&f->H, kn) == hipSuccess && dalloc(&f->HT, kn) == hipSuccess &&
-              ccd::copy_sync(f->stream, f->H, H, 4 * kn, hipMemcpyHostToDevice) == hipSuccess &&
-              ccd::launch_transpose(f->H, f->HT, k, (uint32_t)n, f->stream) == hipSuccess &&
+              dalloc(&dH, kn) == hipSuccess && dalloc(&f->HT, nht) == hipSuccess && dalloc(&f->bad, 1) == hipSuccess &&
+              ccd::launch_fill(f->HT, 0.0f, nht, f->stream) == hipSuccess &&
+              ccd::copy_sync(f->stream, dH, H, 4 * kn, hipMemcpyHostToDevice) == hipSuccess &&
+              ccd::launch_transpose(dH, f->HT, k, (uint32_t)n, fold_ld(k), f->stream) == hipSuccess &&
               hipStreamSynchronize(f->stream) == hipSuccess && scratch_on(device, &f->scratch) == hipSuccess;
+    dfree(dH);
     if (!ok) {
         ccd_fold_destroy(f);
         return CCD_ERR_HIP;
@@ -586,7 +629,7 @@ int32_t ccd_fold_destroy(ccd_fold* f) {
     if (!f) return CCD_OK;
     (void)hipSetDevice(f->device);
     if (f->stream) (void)hipStreamSynchronize(f->stream);
-    void* bufs[] = {f->H, f->HT, f->ptr, f->idx, f->val, f->rbuf, f->W0, f->W, f->F, f->long_rows};
+    void* bufs[] = {f->HT, f->bad, f->ptr, f->idx, f->val, f->W0, f->W, f->F, f->long_rows};
     for (void* b : bufs) dfree(b);
     if (f->ea) (void)hipEventDestroy(f->ea);
     if (f->eb) (void)hipEventDestroy(f->eb);
@@ -604,7 +647,7 @@ int32_t ccd_fold_features(ccd_fold* f, int64_t rows, const uint32_t* ptr, const 
     if (int rc = fold_upload(f, rows, ptr, idx, val, &a)) return rc;
     const size_t nf = (size_t)rows * (2 * f->k + 2);
     OBJ_TRY(f, ensure(&f->F, &f->cap_f, nf));
-    OBJ_TRY(f, ccd::launch_fold_features(a, f->long_rows, f->nlong, f->F, f->stream));
+    OBJ_TRY(f, ccd::launch_fold_features(a, f->long_rows, f->nfeat, f->F, f->stream));
     OBJ_TRY(f, hipStreamSynchronize(f->stream));
     if (nf) OBJ_TRY(f, hipMemcpy(F, f->F, 4 * nf, hipMemcpyDeviceToHost));
     return CCD_OK;
@@ -623,7 +666,7 @@ int32_t ccd_fold_rows(ccd_fold* f, int64_t rows, const uint32_t* ptr, const uint
         if (nw) OBJ_TRY(f, ccd::copy_sync(f->stream, f->W0, W0, 4 * nw, hipMemcpyHostToDevice));
     }
     OBJ_TRY(f, hipEventRecord(f->ea, f->stream));
-    OBJ_TRY(f, ccd::launch_fold_sweeps(a, f->long_rows, f->nlong, W0 ? f->W0 : nullptr, f->W, f->rbuf, f->stream));
+    OBJ_TRY(f, ccd::launch_fold_sweeps(a, f->long_rows, f->nlong, W0 ? f->W0 : nullptr, f->W, f->stream));
     OBJ_TRY(f, hipEventRecord(f->eb, f->stream));
     OBJ_TRY(f, hipEventSynchronize(f->eb));
     float ms = 0.0f;
@@ -645,29 +688,29 @@ int32_t ccd_fold_rows_noalloc(ccd_fold* f, int64_t rows, const uint32_t* ptr, co
                            std::to_string(rows) + " rows, " + std::to_string(nnz) + " ratings)");
     // long rows (one block each), listed in a fixed-size host array
     uint32_t lr[NA_MAX_ROWS];
-    uint32_t nlong = 0;
-    for (int64_t i = 0; i < rows; ++i)
-        if (ptr[i + 1] - ptr[i] > ccd::FOLD_SHORT) lr[nlong++] = (uint32_t)i;
+    const uint32_t nlong = count_long(rows, ptr, ccd::FOLD_WAVE);
+    list_long(rows, ptr, lr);
     unsigned char* S = f->scratch;
     uint32_t* dptr = reinterpret_cast<uint32_t*>(S + NA_OFF_PTR);
     uint32_t* dlong = reinterpret_cast<uint32_t*>(S + NA_OFF_LONG);
     uint32_t* didx = reinterpret_cast<uint32_t*>(S + NA_OFF_IDX);
     float* dval = reinterpret_cast<float*>(S + NA_OFF_VAL);
-    float* drbuf = reinterpret_cast<float*>(S + NA_OFF_RBUF);
     float* dW0 = reinterpret_cast<float*>(S + NA_OFF_W0);
     float* dW = reinterpret_cast<float*>(S + NA_OFF_W);
     const size_t nw = (size_t)rows * f->k;
     OBJ_TRY(f, hipSetDevice(f->device));
-    OBJ_TRY(f, ccd::copy_sync(f->stream, dptr, ptr, 4 * ((size_t)rows + 1), hipMemcpyHostToDevice));
+    OBJ_TRY(f, hipMemcpyAsync(dptr, ptr, 4 * ((size_t)rows + 1), hipMemcpyHostToDevice, f->stream));
     if (nlong) OBJ_TRY(f, ccd::copy_sync(f->stream, dlong, lr, 4 * (size_t)nlong, hipMemcpyHostToDevice));
     if (nnz) {
-        OBJ_TRY(f, ccd::copy_sync(f->stream, didx, idx, 4 * nnz, hipMemcpyHostToDevice));
-        OBJ_TRY(f, ccd::copy_sync(f->stream, dval, val, 4 * nnz, hipMemcpyHostToDevice));
+        OBJ_TRY(f, hipMemcpyAsync(didx, idx, 4 * nnz, hipMemcpyHostToDevice, f->stream));
+        OBJ_TRY(f, hipMemcpyAsync(dval, val, 4 * nnz, hipMemcpyHostToDevice, f->stream));
+        if (int rc = fold_check_device(f, didx, nnz)) return rc;
     }
     if (W0 && nw) OBJ_TRY(f, ccd::copy_sync(f->stream, dW0, W0, 4 * nw, hipMemcpyHostToDevice));
-    const ccd::FoldArgs a{dptr, didx, dval, f->H, f->HT, (uint32_t)rows, f->k, (uint32_t)f->n, sweeps, f->lambda};
+    const ccd::FoldArgs a{dptr, didx, dval, f->HT, (uint32_t)rows, f->k, fold_ld(f->k), (uint32_t)f->n, sweeps,
+                          f->lambda};
     OBJ_TRY(f, hipEventRecord(f->ea, f->stream));
-    OBJ_TRY(f, ccd::launch_fold_sweeps(a, dlong, nlong, W0 ? dW0 : nullptr, dW, drbuf, f->stream));
+    OBJ_TRY(f, ccd::launch_fold_sweeps(a, dlong, nlong, W0 ? dW0 : nullptr, dW, f->stream));
     OBJ_TRY(f, hipEventRecord(f->eb, f->stream));
     OBJ_TRY(f, hipEventSynchronize(f->eb));
     float ms = 0.0f;
@@ -692,11 +735,11 @@ int32_t ccd_fold_warm(ccd_fold* f, ccd_mlp* m, int64_t rows, const uint32_t* ptr
     OBJ_TRY(f, ensure(&f->F, &f->cap_f, nf));
     OBJ_TRY(f, hipStreamSynchronize(m->stream));
     OBJ_TRY(f, hipEventRecord(f->ea, f->stream));
-    OBJ_TRY(f, ccd::launch_fold_features(a, f->long_rows, f->nlong, f->F, f->stream));
+    OBJ_TRY(f, ccd::launch_fold_features(a, f->long_rows, f->nfeat, f->F, f->stream));
     if (bf16_weights < 0 || bf16_weights > 2) return obj_err(f->err, CCD_ERR_INVALID, "bf16_weights must be 0, 1 or 2");
     if (int rc = mlp_forward_dev(m, (uint64_t)rows, f->F, f->W0, bf16_weights, f->stream))
         return obj_err(f->err, rc, "MLP: " + m->err);
-    OBJ_TRY(f, ccd::launch_fold_sweeps(a, f->long_rows, f->nlong, f->W0, f->W, f->rbuf, f->stream));
+    OBJ_TRY(f, ccd::launch_fold_sweeps(a, f->long_rows, f->nlong, f->W0, f->W, f->stream));
     OBJ_TRY(f, hipEventRecord(f->eb, f->stream));
     OBJ_TRY(f, hipEventSynchronize(f->eb));
     float ms = 0.0f;

@@ -472,32 +472,36 @@ int batch_blocks_per_cu(int sigma, size_t lds_bytes);
 
 // ---------------------------------------------------------------- fold-in ---
 // Rows (CSR, the new users' ratings) folded in against fixed item factors:
-// H [k][n] rank-major for the sweeps, HT [n][k] for the features.
+// HT [n + 1][ld], one row per item, zero past rank k and in row n.
 constexpr int FOLD_KMAX = 128;
 struct FoldArgs {
     const uint32_t* ptr;  // rows + 1
     const uint32_t* idx;
     const float* val;
-    const float* H;
     const float* HT;
     uint32_t rows;
     uint32_t k;
+    uint32_t ld;  // k rounded up to 16
     uint32_t n;
     int sweeps;
     float lambda;
 };
-// Rows longer than FOLD_SHORT ratings are listed in long_rows[0 .. nlong)
-// and get a block each.
+// Rows longer than FOLD_WAVE ratings get a block each in the sweeps, rows
+// longer than FOLD_SHORT in the features; the others a wave.  long_rows
+// lists the former by falling length class, so that the latter lead it.
+constexpr uint32_t FOLD_WAVE = 128;
 constexpr uint32_t FOLD_SHORT = 1024;
 // F [rows][2k + 2]: rating-weighted mean and variance of the rated items' H
-// columns, log(1 + degree), mean rating (FP64 sums)
+// columns, log(1 + degree), mean rating (FP64 sums); nlong rows of
+// long_rows exceed FOLD_SHORT
 hipError_t launch_fold_features(const FoldArgs& a, const uint32_t* long_rows, uint32_t nlong, float* F,
                                 hipStream_t s);
-// W [rows][k] after a.sweeps sweeps from W0 ([rows][k], null = zeros); rbuf:
-// nnz floats of scratch (used by rows above 16384 ratings)
+// W [rows][k] after a.sweeps sweeps from W0 ([rows][k], null = zeros); nlong
+// rows of long_rows exceed FOLD_WAVE
 hipError_t launch_fold_sweeps(const FoldArgs& a, const uint32_t* long_rows, uint32_t nlong, const float* W0, float* W,
-                              float* rbuf, hipStream_t s);
-hipError_t launch_transpose(const float* src, float* dst, uint32_t rows, uint32_t cols, hipStream_t s);
+                              hipStream_t s);
+// dst[c * ld + r] = src[r * cols + c]
+hipError_t launch_transpose(const float* src, float* dst, uint32_t rows, uint32_t cols, uint32_t ld, hipStream_t s);
 
 // -------------------------------------------------------------------- MLP ---
 // C(i, j) = sum_p A(i, p) B(p, j) for i < M, j < N, p < K with

@@ -4,12 +4,9 @@
 //   a = r^ + w_t h_t,  w_t = sum a h_t / (lambda |row| + sum h_t^2),  r^ = a - w_t h_t
 // (the u-side update of src/cdmf_ref.cpp:7-17 on one row).
 //
-// The sweeps take one launch of 1024-thread blocks for both row classes:
-// blocks below nlong take one long row each (more than FOLD_SHORT ratings,
-// listed by the host) with all 16 waves; the other blocks take 16 short
-// rows, one per wave.  The features take a launch per class.  Residual, indices and gathered h values stay in registers for the
-// whole solve (rows above 16384 ratings keep the rest in a global buffer).
-// Per-row sums are reduced in a fixed order: deterministic.
+// computed on the row's normal equations (below).  The features and the
+// sweeps take a launch for the long rows, listed by the host, and one for
+// the others.  Per-row sums are reduced in a fixed order: deterministic.
 #include "ccd_kernels.h"
 
 namespace ccd {
@@ -19,17 +16,7 @@ constexpr int WAVE = 64;
 constexpr int BLOCK = 256;
 constexpr int LBLOCK = 1024;
 constexpr int LWAVES = LBLOCK / WAVE;
-constexpr int FOLD_E = 16;   // elements per lane of a short row (1024 per row)
-constexpr int LONG_E = 16;   // elements per thread of a long row (16384 per row)
 constexpr int FEAT_U = 32;   // H-row loads in flight per feature step
-static_assert(WAVE * FOLD_E == (int)FOLD_SHORT, "short-row bound of the host's long-row list");
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
 // Feature sums of a row's elements s .. e - 1 for rank t, over the chunks
 // of 64 elements c0, c0 + cstep, ...: S = sum r, m = sum r h, v = sum r h^2
 // (FP64, in element order within each chunk, chunks in order).  A chunk's
@@ -41,7 +28,6 @@ __device__ __forceinline__ float wave_sum(float v) {
 // branch around the loads.
 __device__ __forceinline__ void feature_sums(const FoldArgs& a, uint32_t s, uint32_t e, uint32_t c0, uint32_t cstep,
                                              uint32_t t, bool tok, double& S, double& m, double& v) {
-    const uint32_t k = a.k;
     const uint32_t tt = tok ? t : 0u;
     const int lane = threadIdx.x & (WAVE - 1);
     for (uint32_t base = s + c0 * WAVE; base < e; base += cstep * WAVE) {
@@ -57,7 +43,7 @@ __device__ __forceinline__ void feature_sums(const FoldArgs& a, uint32_t s, uint
 #pragma unroll
             for (int u = 0; u < FEAT_U; ++u) {
                 const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cv, FEAT_U * half + u);
-                h[u] = a.HT[(size_t)c * k + tt];
+                h[u] = a.HT[(size_t)c * a.ld + tt];
             }
 #pragma unroll
             for (int u = 0; u < FEAT_U; ++u) {
@@ -153,180 +139,319 @@ __global__ __launch_bounds__(WAVE) void fold_features_short_kernel(FoldArgs a, f
     }
 }
 
-// One short row on one wave.  w_t lives in lane t % 64, slot t / 64, and is
-// broadcast with a shuffle (t uniform, whole wave active).
-__device__ __forceinline__ void sweep_short_row(const FoldArgs& a, uint32_t row, int lane, const float* __restrict__ W0,
-                                                float* __restrict__ W) {
-    constexpr int NS = FOLD_KMAX / WAVE;
-    const uint32_t s = a.ptr[row], e = a.ptr[row + 1], d = e - s;
-    const uint32_t k = a.k;
-    const float* __restrict__ H = a.H;
-    float wr[NS];
+// ------------------------------------------------------------ sweeps ---
+// The sweeps work on a row's normal equations G = H_O^T H_O (k x k) and
+// b = H_O^T r: in exact arithmetic the update of rank t,
+//   w_t = (b_t - sum_{s != t} G_ts w_s) / (lambda |O| + G_tt),
+// is the one over the row's residual, but a sweep costs k^2 operations on
+// one wave instead of |O| k gathers.  Everything is FP64 from the products
+// on, so the result is closer to the exact sweeps than an FP32 residual
+// carried through them (2.5e-8, the final
+// rounding, against 6e-7 relative on the shapes below).
+//
+// G comes from the FP64 matrix cores, v_mfma_f64_16x16x4_f64: four ratings a
+// step, NT = ceil(k / 16) loads of 16 consecutive entries of an item's HT
+// row per rating, each of them both operands of its tile pairs (upper
+// triangle only).  Operand layout: lane l supplies A[l % 16][l / 16] and
+// B[l / 16][l % 16] and receives D[4 q + l / 16][l % 16], q = 0..3.
+// NT (NT + 1) / 2 pairs of 64 cycles per four ratings bound this part.
+//
+// The sweep keeps e_s = (numerator_s) / (denominator_s) - w_s on lane s: rank
+// t's change D is e_t, and e_s -= (G_st / denominator_s) D for every s.  One
+// step is one cross-lane read of e_t and one FMA (the scaled matrix comes
+// from LDS, a column per lane, ahead of time), and the k steps of a sweep
+// are a serial chain: its latency (about 60 cycles a step) bounds one row,
+// its issue slots (about 27) a batch of short ones.
+//
+// One row of 206 ratings, k = 40, 20 sweeps: 679 -> 29 us; 48,019 rows with
+// 9.9M ratings: 23.6 -> 1.4 ms (7 sweeps 9.1 -> 1.1 ms), against the same
+// sweeps over the FP32 residual in registers.
+using f64x4 = __attribute__((__vector_size__(4 * sizeof(double)))) double;
+constexpr int GSTEP = 4;          // steps of four ratings whose loads are in flight together
+constexpr int GRAM_PAIRS = 12;    // tile pairs a wave accumulates at once (96 registers)
+
+constexpr int pair_count(int nt) { return nt * (nt + 1) / 2; }
+// tile pair p of the upper triangle, row by row
+constexpr int pair_row(int nt, int p) {
+    int r = 0;
+    while (p >= nt - r) p -= nt - r++;
+    return r;
+}
+constexpr int pair_col(int nt, int p) {
+    int r = 0;
+    while (p >= nt - r) p -= nt - r++;
+    return r + p;
+}
+
+// entries of G in LDS: rows of 16 NT, whole groups of the chain
+constexpr int CHAIN = 8;
+__host__ __device__ constexpr uint32_t fold_matrix(int nt, uint32_t k) { return 16u * nt * ((k + CHAIN - 1) / CHAIN * CHAIN); }
+
+template <int NT, int P0, int P, int I = 0>
+__device__ __forceinline__ void gram_mfma(const double (&h)[NT], f64x4 (&acc)[P]) {
+    if constexpr (I < P) {
+        constexpr int ti = pair_row(NT, P0 + I), tj = pair_col(NT, P0 + I);
+        acc[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(h[ti], h[tj], acc[I], 0, 0, 0);
+        gram_mfma<NT, P0, P, I + 1>(h, acc);
+    }
+}
+
+template <int NT, int P0, int P, int I = 0>
+__device__ __forceinline__ void gram_store(const f64x4 (&acc)[P], double* G, uint32_t k, int lane, bool first) {
+    if constexpr (I < P) {
+        constexpr int LD = 16 * NT;
+        constexpr int ti = pair_row(NT, P0 + I), tj = pair_col(NT, P0 + I);
+        const uint32_t c = 16 * tj + lane % 16;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t r = 16 * ti + 4 * q + lane / 16;
+            if (r < k && c < k) {
+                const double v = first ? acc[I][q] : G[r * LD + c] + acc[I][q];
+                G[r * LD + c] = v;
+                if (ti != tj) G[c * LD + r] = v;
+            }
+        }
+        gram_store<NT, P0, P, I + 1>(acc, G, k, lane, first);
+    }
+}
+
+// G (k x k, rows of 16 NT) and b (k) in LDS of the ratings s .. s + d - 1, by the NW waves of
+// the block: wave wv takes chunks wv, wv + NW, ... of 64 ratings, and the
+// waves' sums are added in wave order.  Ends with every wave's part stored
+// (the caller synchronises).
+template <int NT, int NW, int P0 = 0>
+__device__ __forceinline__ void gram(const FoldArgs& a, uint32_t s, uint32_t d, double* G, double* b) {
+    constexpr int PALL = pair_count(NT), P = PALL - P0 < GRAM_PAIRS ? PALL - P0 : GRAM_PAIRS;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const uint32_t wv = NW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t k = a.k, sub = lane / 16, col = lane % 16;
+    f64x4 acc[P];
+    double bacc[NT];
+#pragma unroll
+    for (int i = 0; i < P; ++i) acc[i] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < NT; ++t) bacc[t] = 0.0;
+    for (uint32_t c0 = wv * WAVE; c0 < d; c0 += NW * WAVE) {
+        const uint32_t p = c0 + lane;
+        const uint32_t cv = p < d ? __builtin_nontemporal_load(a.idx + s + p) : a.n;  // row n of HT is zero
+        const float rv = p < d ? __builtin_nontemporal_load(a.val + s + p) : 0.0f;
+        const uint32_t n = d - c0 < (uint32_t)WAVE ? d - c0 : (uint32_t)WAVE;
+        for (uint32_t j = 0; 4 * j < n; j += GSTEP) {
+            float h[GSTEP][NT];
+#pragma unroll
+            for (int u = 0; u < GSTEP; ++u) {
+                const uint32_t c = (uint32_t)__shfl((int)cv, (int)(4 * (j + u) + sub));
+                const float* hr = a.HT + (size_t)c * a.ld + col;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) h[u][t] = hr[16 * t];
+            }
+#pragma unroll
+            for (int u = 0; u < GSTEP; ++u) {
+                double hd[NT];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) hd[t] = (double)h[u][t];
+                if constexpr (P0 == 0) {
+                    const double r = (double)__shfl(rv, (int)(4 * (j + u) + sub));
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) bacc[t] = __builtin_fma(r, hd[t], bacc[t]);
+                }
+                gram_mfma<NT, P0, P>(hd, acc);
+            }
+        }
+    }
+    const uint32_t parts = NW == 1 ? 1u : min((uint32_t)NW, (d + WAVE - 1) / WAVE);
+    if constexpr (P0 == 0) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            bacc[t] += __shfl_xor(bacc[t], 16);
+            bacc[t] += __shfl_xor(bacc[t], 32);
+        }
+    }
+    for (uint32_t w = 0; w < parts; ++w) {
+        if (w == wv) {
+            gram_store<NT, P0, P>(acc, G, k, lane, w == 0);
+            if constexpr (P0 == 0) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const uint32_t i = 16 * t + col;
+                    if (sub == 0 && i < k) b[i] = w == 0 ? bacc[t] : b[i] + bacc[t];
+                }
+            }
+        }
+        if (NW > 1) __syncthreads();
+    }
+    if constexpr (P0 + P < PALL) gram<NT, NW, P0 + P>(a, s, d, G, b);
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const long long x = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((unsigned long long)x >> 32), lane);
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// v with lane LANE replaced by the uniform x
+template <int LANE>
+__device__ __forceinline__ double with_lane(double v, double x) {
+    unsigned long long a = (unsigned long long)__double_as_longlong(v), b = (unsigned long long)__double_as_longlong(x);
+    uint32_t lo = (uint32_t)a, hi = (uint32_t)(a >> 32);
+    asm("v_writelane_b32 %0, %1, %2" : "+v"(lo) : "s"((uint32_t)b), "n"(LANE));
+    asm("v_writelane_b32 %0, %1, %2" : "+v"(hi) : "s"((uint32_t)(b >> 32)), "n"(LANE));
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+template <int NS, int J, int L0, int U = 0>
+__device__ __forceinline__ void fold_steps(const double (&g)[NS][CHAIN], double (&e)[NS], double& cap) {
+    if constexpr (U < CHAIN) {
+        const double D = lane_value(e[J], L0 + U);
+        cap = with_lane<L0 + U>(cap, D);
+#pragma unroll
+        for (int j = 0; j < NS; ++j) e[j] = __builtin_fma(-g[j][U], D, e[j]);
+        fold_steps<NS, J, L0, U + 1>(g, e, cap);
+    }
+}
+
+// The chain over ranks 64 J + 8 Q .. of the matrix at m (row 64 J, this
+// lane's column of slot 0), group by group; LD: row length in LDS.  Lane and
+// row offsets are constants, so a step is two reads and two writes of a lane
+// and one FMA per slot.
+template <int NS, int J, int LD, int Q = 0>
+__device__ __forceinline__ void fold_chain(const double* m, uint32_t groups, const double (&g)[NS][CHAIN],
+                                           double (&e)[NS], double& cap) {
+    if ((uint32_t)Q >= groups) return;
+    // the next group's entries, read ahead of this group's chain
+    double gn[NS][CHAIN];
+    constexpr int QN = Q + 1 < WAVE / CHAIN ? Q + 1 : 0;
+    const double* mn = m + ((uint32_t)QN < groups ? QN * CHAIN * LD : 0);
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+#pragma unroll
+        for (int u = 0; u < CHAIN; ++u) gn[j][u] = mn[u * LD + WAVE * j];
+    fold_steps<NS, J, Q * CHAIN>(g, e, cap);
+    if constexpr (Q + 1 < WAVE / CHAIN) fold_chain<NS, J, LD, Q + 1>(m, groups, gn, e, cap);
+}
+
+// The sweeps of one row from its G and b in LDS, by one wave: lane l holds
+// ranks l and, for k > 64 (NS = 2), l + 64.  Column s of G is only touched by
+// rank s's lane, which scales it in place.  Rows k .. of G up to a multiple
+// of CHAIN are cleared, so the chain runs in whole groups.
+template <int NS, int LD>
+__device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint32_t d, double* G, const double* b,
+                                           const float* __restrict__ W0, float* __restrict__ W) {
+    const uint32_t lane = threadIdx.x & (WAVE - 1), k = a.k;
+    const double lamd = (double)(a.lambda * (float)d);
+    double e[NS], w[NS];
+    const double* base = G + (lane < (uint32_t)LD ? lane : 0u);  // lanes past the matrix read column 0, times 0
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        const uint32_t t = lane + WAVE * j;
-        wr[j] = (W0 && t < k) ? W0[(size_t)row * k + t] : 0.0f;
-    }
-    auto wget = [&](uint32_t t) -> float {
-        float v = 0.0f;
-#pragma unroll
-        for (int j = 0; j < NS; ++j)
-            if (t / WAVE == (uint32_t)j) v = __shfl(wr[j], (int)(t % WAVE));
-        return v;
-    };
-    const float lamd = a.lambda * (float)d;
-    uint32_t c[FOLD_E];
-    float r[FOLD_E], hv[FOLD_E];
-#pragma unroll
-    for (int q = 0; q < FOLD_E; ++q) {
-        const uint32_t p = lane + WAVE * q;
-        const bool ok = p < d;
-        c[q] = ok ? a.idx[s + p] : 0u;
-        r[q] = ok ? a.val[s + p] : 0.0f;
-    }
-    // residual of the starting factors, ranks in ascending order
-    for (uint32_t t = 0; t < k; ++t) {
-        const float wt = wget(t);
-        const float* ht = H + (size_t)t * a.n;
-#pragma unroll
-        for (int q = 0; q < FOLD_E; ++q)
-            if (lane + WAVE * q < d) r[q] = r[q] - wt * ht[c[q]];
-    }
-    for (int sw = 0; sw < a.sweeps; ++sw) {
-        for (uint32_t t = 0; t < k; ++t) {
-            const float wo = wget(t);
-            const float* ht = H + (size_t)t * a.n;
-            float g = 0.0f, hh = 0.0f;
-#pragma unroll
-            for (int q = 0; q < FOLD_E; ++q) {
-                const bool ok = lane + WAVE * q < d;
-                const float h = ok ? ht[c[q]] : 0.0f;
-                hv[q] = h;
-                const float av = r[q] + wo * h;
-                r[q] = av;
-                g += av * h;
-                hh += h * h;
+        const uint32_t s = lane + WAVE * j;
+        e[j] = 0.0;
+        w[j] = 0.0;
+        if (s < k) {
+            double* col = G + s;
+            w[j] = W0 ? (double)W0[(size_t)row * k + s] : 0.0;
+            const double inv = 1.0 / (lamd + col[s * LD]);
+            double p = b[s];
+            if (W0) {  // the numerator leaves the rank's own term out
+                for (uint32_t u = 0; u < k; ++u) {
+                    const double wu = (double)W0[(size_t)row * k + u];
+                    if (u != s) p = __builtin_fma(-col[u * LD], wu, p);
+                }
             }
-            g = wave_sum(g);
-            hh = wave_sum(hh);
-            const float wn = d ? g / (lamd + hh) : 0.0f;
-#pragma unroll
-            for (int q = 0; q < FOLD_E; ++q) r[q] = r[q] - wn * hv[q];
+            e[j] = __builtin_fma(p, inv, -w[j]);
+#pragma unroll 4
+            for (uint32_t u = 0; u < k; ++u) col[u * LD] = u == s ? 1.0 : col[u * LD] * inv;
+        }
+        if (s < (uint32_t)LD)
+            for (uint32_t u = k; u % CHAIN; ++u) G[u * LD + s] = 0.0;
+    }
+    // one wave: its LDS writes above come before its reads below
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int sw = 0; sw < a.sweeps; ++sw) {
+        double g[NS][CHAIN], cap = 0.0;
+        auto first = [&](const double* m) {
 #pragma unroll
             for (int j = 0; j < NS; ++j)
-                if (t / WAVE == (uint32_t)j && (uint32_t)lane == t % WAVE) wr[j] = wn;
+#pragma unroll
+                for (int u = 0; u < CHAIN; ++u) g[j][u] = m[u * LD + WAVE * j];
+        };
+        first(base);
+        fold_chain<NS, 0, LD>(base, (min(k, (uint32_t)WAVE) + CHAIN - 1) / CHAIN, g, e, cap);
+        w[0] += cap;
+        if constexpr (NS == 2) {
+            const double* m = base + WAVE * LD;
+            cap = 0.0;
+            first(m);
+            fold_chain<NS, 1, LD>(m, (k - WAVE + CHAIN - 1) / CHAIN, g, e, cap);
+            w[1] += cap;
         }
     }
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        const uint32_t t = lane + WAVE * j;
-        if (t < k) W[(size_t)row * k + t] = wr[j];
+        const uint32_t s = lane + WAVE * j;
+        if (s < k) W[(size_t)row * k + s] = (float)w[j];
     }
 }
 
-// One long row on the whole block: thread i holds elements i + 1024 q,
-// q < LONG_E; elements beyond 16384 keep their residual in rbuf.  w in LDS;
-// per rank one block reduction of (g, h): wave sums, then the 16 wave
-// partials in wave order.
-__device__ __forceinline__ void sweep_long_row(const FoldArgs& a, uint32_t row, const float* __restrict__ W0,
-                                               float* __restrict__ W, float* __restrict__ rbuf, float* wsh,
-                                               float (*red)[LWAVES]) {
-    const uint32_t s = a.ptr[row], e = a.ptr[row + 1], d = e - s;
-    const uint32_t k = a.k;
-    const float* __restrict__ H = a.H;
-    const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
-    for (uint32_t t = threadIdx.x; t < k; t += LBLOCK) wsh[t] = W0 ? W0[(size_t)row * k + t] : 0.0f;
-    __syncthreads();
-    const float lamd = a.lambda * (float)d;
-    constexpr uint32_t CAP = LBLOCK * LONG_E;
-    uint32_t c[LONG_E];
-    float r[LONG_E], hv[LONG_E];
-#pragma unroll
-    for (int q = 0; q < LONG_E; ++q) {
-        const uint32_t p = threadIdx.x + LBLOCK * q;
-        const bool ok = p < d;
-        c[q] = ok ? a.idx[s + p] : 0u;
-        r[q] = ok ? a.val[s + p] : 0.0f;
-    }
-    for (uint32_t t = 0; t < k; ++t) {
-        const float wt = wsh[t];
-        const float* ht = H + (size_t)t * a.n;
-#pragma unroll
-        for (int q = 0; q < LONG_E; ++q)
-            if (threadIdx.x + LBLOCK * q < d) r[q] = r[q] - wt * ht[c[q]];
-        for (uint32_t p = CAP + threadIdx.x; p < d; p += LBLOCK)
-            rbuf[s + p] = (t == 0 ? a.val[s + p] : rbuf[s + p]) - wt * ht[a.idx[s + p]];
-    }
-    for (int sw = 0; sw < a.sweeps; ++sw) {
-        for (uint32_t t = 0; t < k; ++t) {
-            const float wo = wsh[t];
-            const float* ht = H + (size_t)t * a.n;
-            float g = 0.0f, hh = 0.0f;
-#pragma unroll
-            for (int q = 0; q < LONG_E; ++q) {
-                const bool ok = threadIdx.x + LBLOCK * q < d;
-                const float h = ok ? ht[c[q]] : 0.0f;
-                hv[q] = h;
-                const float av = r[q] + wo * h;
-                r[q] = av;
-                g += av * h;
-                hh += h * h;
-            }
-            for (uint32_t p = CAP + threadIdx.x; p < d; p += LBLOCK) {
-                const float h = ht[a.idx[s + p]];
-                const float av = rbuf[s + p] + wo * h;
-                rbuf[s + p] = av;
-                g += av * h;
-                hh += h * h;
-            }
-            g = wave_sum(g);
-            hh = wave_sum(hh);
-            if (lane == 0) {
-                red[0][wv] = g;
-                red[1][wv] = hh;
-            }
-            __syncthreads();
-            float gt = 0.0f, ht2 = 0.0f;
-            for (int w = 0; w < LWAVES; ++w) {
-                gt += red[0][w];
-                ht2 += red[1][w];
-            }
-            const float wn = gt / (lamd + ht2);
-#pragma unroll
-            for (int q = 0; q < LONG_E; ++q) r[q] = r[q] - wn * hv[q];
-            for (uint32_t p = CAP + threadIdx.x; p < d; p += LBLOCK) rbuf[s + p] = rbuf[s + p] - wn * ht[a.idx[s + p]];
-            if (threadIdx.x == 0) wsh[t] = wn;
-            __syncthreads();  // red is reused by the next rank
-        }
-    }
-    for (uint32_t t = threadIdx.x; t < k; t += LBLOCK) W[(size_t)row * k + t] = wsh[t];
+// Rows of more than FOLD_WAVE ratings: one block each, in the order of the
+// host's list (longest first, so the last blocks to run are short).  The
+// waves share the products; the first one then runs the sweeps while the
+// others' slots go to the next block.
+constexpr int FOLD_LWAVES = 8;
+template <int NT>
+__global__ __launch_bounds__(FOLD_LWAVES* WAVE) void fold_sweep_long_kernel(FoldArgs a,
+                                                                           const uint32_t* __restrict__ long_rows,
+                                                                           const float* __restrict__ W0,
+                                                                           float* __restrict__ W) {
+    extern __shared__ __align__(16) double fold_lds[];  // G, then b
+    double* b = fold_lds + fold_matrix(NT, a.k);
+    const uint32_t row = long_rows[blockIdx.x];
+    const uint32_t s = a.ptr[row], d = a.ptr[row + 1] - s;
+    gram<NT, FOLD_LWAVES>(a, s, d, fold_lds, b);
+    if (threadIdx.x >= WAVE) return;
+    fold_solve<(NT > 4 ? 2 : 1), 16 * NT>(a, row, d, fold_lds, b, W0, W);
 }
 
-__global__ __launch_bounds__(LBLOCK) void fold_sweep_kernel(FoldArgs a, const uint32_t* __restrict__ long_rows,
-                                                            uint32_t nlong, const float* __restrict__ W0,
-                                                            float* __restrict__ W, float* __restrict__ rbuf) {
-    __shared__ float wsh[FOLD_KMAX];
-    __shared__ float red[2][LWAVES];
-    if (blockIdx.x < nlong) {
-        sweep_long_row(a, long_rows[blockIdx.x], W0, W, rbuf, wsh, red);
+// The other rows, one single-wave block each.
+template <int NT>
+__global__ __launch_bounds__(WAVE) void fold_sweep_short_kernel(FoldArgs a, const float* __restrict__ W0,
+                                                                float* __restrict__ W) {
+    extern __shared__ __align__(16) double fold_lds[];
+    double* b = fold_lds + fold_matrix(NT, a.k);
+    const uint32_t row = blockIdx.x;
+    const uint32_t s = a.ptr[row], d = a.ptr[row + 1] - s;
+    if (d > FOLD_WAVE) return;
+    if (d == 0 || a.sweeps == 0) {  // nothing to solve: 0 after a sweep, the start before one
+        for (uint32_t t = threadIdx.x; t < a.k; t += WAVE)
+            W[(size_t)row * a.k + t] = a.sweeps == 0 && W0 ? W0[(size_t)row * a.k + t] : 0.0f;
         return;
     }
-    const uint32_t row = (blockIdx.x - nlong) * LWAVES + threadIdx.x / WAVE;
-    if (row >= a.rows) return;
-    if (a.ptr[row + 1] - a.ptr[row] > FOLD_SHORT) return;
-    sweep_short_row(a, row, threadIdx.x & (WAVE - 1), W0, W);
+    gram<NT, 1>(a, s, d, fold_lds, b);
+    __syncthreads();  // one wave: orders its LDS writes and reads
+    fold_solve<(NT > 4 ? 2 : 1), 16 * NT>(a, row, d, fold_lds, b, W0, W);
+}
+
+template <int NT>
+hipError_t launch_sweeps_nt(const FoldArgs& a, const uint32_t* long_rows, uint32_t nlong, const float* W0, float* W,
+                            hipStream_t s) {
+    const size_t lds = sizeof(double) * (fold_matrix(NT, a.k) + a.k);
+    if (nlong)
+        hipLaunchKernelGGL(fold_sweep_long_kernel<NT>, dim3(nlong), dim3(FOLD_LWAVES * WAVE), lds, s, a, long_rows, W0,
+                           W);
+    if (nlong < a.rows)
+        hipLaunchKernelGGL(fold_sweep_short_kernel<NT>, dim3(a.rows), dim3(WAVE), lds, s, a, W0, W);
+    return hipGetLastError();
 }
 
 __global__ __launch_bounds__(BLOCK) void transpose_kernel(const float* __restrict__ src, float* __restrict__ dst,
-                                                          uint32_t rows, uint32_t cols) {
+                                                          uint32_t rows, uint32_t cols, uint32_t ld) {
     const uint64_t total = (uint64_t)rows * cols;
     for (uint64_t q = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; q < total; q += (uint64_t)gridDim.x * BLOCK) {
         const uint64_t r = q / cols, c = q % cols;
-        dst[c * rows + r] = src[q];
+        dst[c * ld + r] = src[q];
     }
 }
-
-uint32_t grid_rows(uint64_t rows, uint32_t nlong) { return nlong + (uint32_t)((rows + LWAVES - 1) / LWAVES); }
 
 }  // namespace
 
@@ -340,20 +465,27 @@ hipError_t launch_fold_features(const FoldArgs& a, const uint32_t* long_rows, ui
 }
 
 hipError_t launch_fold_sweeps(const FoldArgs& a, const uint32_t* long_rows, uint32_t nlong, const float* W0, float* W,
-                              float* rbuf, hipStream_t s) {
+                              hipStream_t s) {
     if (a.rows == 0) return hipSuccess;
-    if (a.k > (uint32_t)FOLD_KMAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(fold_sweep_kernel, dim3(grid_rows(a.rows, nlong)), dim3(LBLOCK), 0, s, a, long_rows, nlong, W0,
-                       W, rbuf);
-    return hipGetLastError();
+    switch ((a.k + 15) / 16) {
+        case 1: return launch_sweeps_nt<1>(a, long_rows, nlong, W0, W, s);
+        case 2: return launch_sweeps_nt<2>(a, long_rows, nlong, W0, W, s);
+        case 3: return launch_sweeps_nt<3>(a, long_rows, nlong, W0, W, s);
+        case 4: return launch_sweeps_nt<4>(a, long_rows, nlong, W0, W, s);
+        case 5: return launch_sweeps_nt<5>(a, long_rows, nlong, W0, W, s);
+        case 6: return launch_sweeps_nt<6>(a, long_rows, nlong, W0, W, s);
+        case 7: return launch_sweeps_nt<7>(a, long_rows, nlong, W0, W, s);
+        case 8: return launch_sweeps_nt<8>(a, long_rows, nlong, W0, W, s);
+        default: return hipErrorInvalidValue;
+    }
 }
 
-hipError_t launch_transpose(const float* src, float* dst, uint32_t rows, uint32_t cols, hipStream_t s) {
+hipError_t launch_transpose(const float* src, float* dst, uint32_t rows, uint32_t cols, uint32_t ld, hipStream_t s) {
     const uint64_t total = (uint64_t)rows * cols;
     if (total == 0) return hipSuccess;
     uint64_t g = (total + BLOCK - 1) / BLOCK;
     if (g > 8192) g = 8192;
-    hipLaunchKernelGGL(transpose_kernel, dim3((uint32_t)g), dim3(BLOCK), 0, s, src, dst, rows, cols);
+    hipLaunchKernelGGL(transpose_kernel, dim3((uint32_t)g), dim3(BLOCK), 0, s, src, dst, rows, cols, ld);
     return hipGetLastError();
 }
 

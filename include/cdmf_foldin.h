@@ -74,7 +74,7 @@ int32_t ccd_fold_rows(ccd_fold* f, int64_t rows, const uint32_t* ptr, const uint
  * reference; for callers that cannot allocate (serving loops folding in
  * batches of new users, code that must not call hipMalloc).  Same kernels
  * and result as ccd_fold_rows (bit for bit); the batch is staged in a
- * library-owned static device scratch of about 28 MB per GPU, held until
+ * library-owned static device scratch of about 20 MB per GPU, held until
  * the process ends, so one call takes at most 4096 rows and 2,097,152
  * ratings (larger batches fail with CCD_ERR_INVALID and a message).  Every
  * call on one GPU shares that GPU's scratch: calls that overlap on one GPU

@@ -101,6 +101,72 @@ def test_fold_rows_very_long_row(oracle_lib):
     fold.close()
 
 
+def _fold_f64(ptr, idx, val, H, lam, sweeps, W0):
+    """The sweeps of plain fold-in in FP64, row by row."""
+    k = H.shape[0]
+    W = np.zeros((ptr.size - 1, k)) if W0 is None else W0.astype(np.float64)
+    for i in range(ptr.size - 1):
+        s, e = int(ptr[i]), int(ptr[i + 1])
+        Ho = H[:, idx[s:e]].astype(np.float64)
+        lamd = float(np.float32(lam) * np.float32(e - s))
+        r = val[s:e] - W[i] @ Ho
+        for _ in range(sweeps):
+            for t in range(k):
+                a = r + W[i, t] * Ho[t]
+                W[i, t] = a @ Ho[t] / (lamd + Ho[t] @ Ho[t]) if e > s else 0.0
+                r = a - W[i, t] * Ho[t]
+    return W
+
+
+@pytest.mark.parametrize("k", [1, 7, 8, 16, 17, 40, 63, 64, 65, 80, 81, 100, 127, 128])
+def test_fold_rows_normal_equations(k):
+    """Row lengths at the edges of a chunk of 64 ratings, of the one-wave
+    rows (128) and of the long rows' eight chunks; ranks at the edges of the
+    16-wide tiles, of the groups of tile pairs and of the two slots a lane
+    holds; from zero and from a start, no sweep, one and three.  The sums
+    and sweeps are FP64, so the result is the FP64 one but for its rounding
+    to FP32 (6e-8) and, next to zero, 1e-9 of its size."""
+    F = _gpu()
+    deg = [0, 1, 2, 3, 4, 5, 15, 17, 63, 64, 65, 127, 128, 129, 191, 512, 513, 1025]
+    rng = np.random.default_rng(k)
+    n = 1200
+    ptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+    idx = np.concatenate([rng.choice(n, size=d, replace=False) for d in deg]).astype(np.uint32)
+    val = rng.integers(1, 6, size=idx.size).astype(np.float32)
+    H = rng.normal(0.1, 0.4, (k, n)).astype(np.float32)
+    W0 = rng.normal(0, 0.3, (len(deg), k)).astype(np.float32)
+    fold = F.FoldIn(H, 0.05)
+    for sweeps in (0, 1, 3):
+        for start in (None, W0):
+            W, _ = fold.rows(ptr, idx, val, sweeps, W0=start)
+            ref = _fold_f64(ptr, idx, val, H, 0.05, sweeps, start)
+            size = max(float(np.abs(ref).max()), 1e-30)
+            np.testing.assert_allclose(W, ref, rtol=6.1e-8, atol=1e-9 * size, err_msg="k=%d sweeps=%d" % (k, sweeps))
+    fold.close()
+
+
+@pytest.mark.parametrize("nnz", [300, 65536, 70000])  # the index check on the host, and on the device
+def test_fold_refuses_indices_out_of_range(nnz):
+    from cdmf_amd.solver import CCDError
+    F = _gpu()
+    n = 500
+    fold = F.FoldIn(np.ones((4, n), np.float32), 0.05)
+    ptr = np.concatenate([np.arange(0, nnz, 250), [nnz]]).astype(np.uint32)
+    idx = (np.arange(nnz) % n).astype(np.uint32)
+    val = np.ones(nnz, np.float32)
+    ok, _ = fold.rows(ptr, idx, val, 1)
+    bad = idx.copy()
+    bad[nnz // 2] = n
+    for call in (fold.rows, fold.rows_noalloc):
+        with pytest.raises(CCDError, match="out of range"):
+            call(ptr, bad, val, 1)
+    with pytest.raises(CCDError, match="out of range"):
+        fold.features(ptr, bad, val)
+    again, _ = fold.rows_noalloc(ptr, idx, val, 1)
+    assert np.array_equal(ok, again)
+    fold.close()
+
+
 def test_fold_rows_reach_ridge_solution():
     F = _gpu()
     ptr, idx, val, H = _rows(3, 60, 500, 8)
