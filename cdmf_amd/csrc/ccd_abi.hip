@@ -106,7 +106,19 @@ inline int group_log2(uint32_t d, uint32_t epl) {
     return lg;
 }
 
-HostPlan make_plan(const uint32_t* ptr, int64_t rows, const ccd_plan_params& pp) {
+// Cost of one pass of a group unit in steps of up to eight elements per lane
+// in flight, for rows of d elements.
+inline uint64_t pass_cost(uint32_t d) { return 1 + d / (8 * 64); }
+
+// waves: those resident in one sweep launch.  A group unit ends at
+// pp.unit_elems elements or 4,096 rows, or earlier, where units of that size
+// would leave waves without one: a pass over 64 / G rows is a chain of
+// dependent loads (about 3 us), so a matrix of few ratings wants its passes
+// spread over all waves rather than queued in a few (41,871 x 16,195 with
+// 1.5M ratings: 366 units, 78 us a sweep; spread out, 14 us).  Two units a
+// wave leave room for their unequal cost.  Where a unit ends changes no
+// result.
+HostPlan make_plan(const uint32_t* ptr, int64_t rows, const ccd_plan_params& pp, uint32_t waves) {
     // rows arrive sorted by falling degree: split rows first, then groups of
     // equal width as contiguous ranges
     HostPlan P;
@@ -124,15 +136,24 @@ HostPlan make_plan(const uint32_t* ptr, int64_t rows, const ccd_plan_params& pp)
     }
     P.split_beg.push_back(slot);
     const uint32_t max_rows = 4096;
+    uint64_t total = 0;
+    for (int64_t i = r; i < rows;) {  // first rows of the passes, as cut below
+        total += pass_cost(deg(i));
+        i += 64u >> group_log2(deg(i), pp.elems_per_lane);
+    }
+    const uint64_t max_cost = std::max<uint64_t>(total / (2ull * std::max(waves, 1u)), 1);
     int64_t i = r;
     while (i < rows) {
         const int lg = group_log2(deg(i), pp.elems_per_lane);
         const uint32_t rpp = 64u >> lg;
         int64_t j = i;
-        uint64_t elems = 0;
+        uint64_t elems = 0, cost = 0;
         while (j < rows && group_log2(deg(j), pp.elems_per_lane) == lg) {
             const uint64_t cnt = (uint64_t)(j - i);
-            if (cnt % rpp == 0 && (elems >= pp.unit_elems || cnt >= max_rows)) break;
+            if (cnt % rpp == 0) {
+                if (elems >= pp.unit_elems || cnt >= max_rows || cost >= max_cost) break;
+                cost += pass_cost(deg(j));
+            }
             elems += deg(j);
             ++j;
         }
@@ -397,7 +418,7 @@ int upload_layout(ccd_ctx* c, DevLayout& L, int64_t rows, int64_t gdim, uint64_t
         HIP_TRY(c, hipStreamSynchronize(c->stream));
     }
 
-    HostPlan P = make_plan(ptr, rows, c->plan);
+    HostPlan P = make_plan(ptr, rows, c->plan, (uint32_t)c->ncu * (ccd::SWEEP_BLOCK / 64));
     if (P.split_beg.back() >= (1u << 24) || P.units.size() >= 0xffffffffull)
         return set_err(c, CCD_ERR_INVALID, "work plan too large: raise ccd_plan_params.piece");
     L.nunits = (uint32_t)P.units.size();

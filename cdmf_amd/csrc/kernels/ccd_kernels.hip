@@ -52,87 +52,119 @@ struct Ctx {
     const FPair<TF>* ldsp;
 };
 
-// One element: residual update (fused passes take both factor values from
-// one pair gather), then the sweep's contribution.
-template <typename TF, typename TA, bool SUB, bool ADD, bool SWEEP>
-__device__ __forceinline__ void one_elem(const Ctx<TF>& k, uint32_t c, float& r, float ysr, float yar, TA& g,
-                                         TA& h) {
+// What one element gathers: the previous and current rank's factor (fused
+// passes take both from one pair) and the sweep's x.
+struct Gathered {
+    float xs, xa, xv;
+};
+
+template <typename TF, bool SUB, bool ADD, bool SWEEP>
+__device__ __forceinline__ Gathered gather_elem(const Ctx<TF>& k, uint32_t c) {
     constexpr bool PAIR = SWEEP && (SUB || ADD);
-    float xv = 0.0f;
+    Gathered o{0.0f, 0.0f, 0.0f};
     if constexpr (PAIR) {
         const FPair<TF> p = gather_pair<TF>(k.ldsp, k.a.hot_p, k.a.xp, c);
-        if (SUB) r = r - tof<TF>(p.prev) * ysr;
-        if (ADD) r = r + tof<TF>(p.cur) * yar;
-        xv = k.a.x_is_cur ? tof<TF>(p.cur) : gather<TF>(k.lds, k.a.hot_x, k.a.x, c);
+        o.xs = tof<TF>(p.prev);
+        o.xa = tof<TF>(p.cur);
+        o.xv = k.a.x_is_cur ? o.xa : gather<TF>(k.lds, k.a.hot_x, k.a.x, c);
     } else {
-        if (SUB) r = r - ldf<TF>(k.a.xs, c) * ysr;
-        if (ADD) r = r + ldf<TF>(k.a.xa, c) * yar;
-        if (SWEEP) xv = gather<TF>(k.lds, k.a.hot_x, k.a.x, c);
+        if (SUB) o.xs = ldf<TF>(k.a.xs, c);
+        if (ADD) o.xa = ldf<TF>(k.a.xa, c);
+        if (SWEEP) o.xv = gather<TF>(k.lds, k.a.hot_x, k.a.x, c);
     }
+    return o;
+}
+
+// One element: residual update, then the sweep's contribution.
+template <typename TA, bool SUB, bool ADD, bool SWEEP>
+__device__ __forceinline__ void one_elem(const Gathered& o, float& r, float ysr, float yar, TA& g, TA& h) {
+    if (SUB) r = r - o.xs * ysr;
+    if (ADD) r = r + o.xa * yar;
     if (SWEEP) {
-        g += (TA)xv * (TA)r;
-        h += (TA)xv * (TA)xv;
+        g += (TA)o.xv * (TA)r;
+        h += (TA)o.xv * (TA)o.xv;
     }
 }
 
+// Elements p, p + step, ... below end by one lane, four at a time: the loads
+// of all four, then their gathers, then the updates in order.  A group's
+// elements past the end load its first one again and are dropped (a group's
+// last one to three elements, one by one, would each wait for their own
+// loads; rows of 64 or fewer lanes hold at most one group a lane).
 template <typename IdxT, typename TF, typename TA, bool SUB, bool ADD, bool SWEEP>
 __device__ __forceinline__ void strided_range(const Ctx<TF>& k, const IdxT* __restrict__ idx, uint32_t p,
                                               const uint32_t end, const uint32_t step, const float ysr,
                                               const float yar, TA& g, TA& h) {
     float* __restrict__ val = k.a.val;
-    // four independent elements per lane in flight
-    for (; p + 3 * step < end; p += 4 * step) {
+    for (; p < end; p += 4 * step) {
         uint32_t c[4];
         float r[4];
+        Gathered o[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) c[q] = __builtin_nontemporal_load(idx + p + q * step);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) r[q] = __builtin_nontemporal_load(val + p + q * step);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) one_elem<TF, TA, SUB, ADD, SWEEP>(k, c[q], r[q], ysr, yar, g, h);
-        if (SUB || ADD) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) __builtin_nontemporal_store(r[q], val + p + q * step);
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t e = p + q * step < end ? p + q * step : p;
+            c[q] = __builtin_nontemporal_load(idx + e);
+            r[q] = __builtin_nontemporal_load(val + e);
         }
-    }
-    for (; p < end; p += step) {
-        const uint32_t c = __builtin_nontemporal_load(idx + p);
-        float r = __builtin_nontemporal_load(val + p);
-        one_elem<TF, TA, SUB, ADD, SWEEP>(k, c, r, ysr, yar, g, h);
-        if (SUB || ADD) __builtin_nontemporal_store(r, val + p);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[q] = gather_elem<TF, SUB, ADD, SWEEP>(k, c[q]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (q > 0 && p + q * step >= end) continue;
+            one_elem<TA, SUB, ADD, SWEEP>(o[q], r[q], ysr, yar, g, h);
+            if (SUB || ADD) __builtin_nontemporal_store(r[q], val + p + q * step);
+        }
     }
 }
 
-// Four consecutive elements starting at 4*q (16-byte aligned): one 16-byte
-// value load, one 16-byte (or 8-byte for 16-bit) index load.
-template <typename IdxT, typename TF, typename TA, bool SUB, bool ADD, bool SWEEP>
-__device__ __forceinline__ void group4(const Ctx<TF>& k, const IdxT* __restrict__ idx, uint32_t q, float ysr,
-                                       float yar, TA& g, TA& h) {
+// N groups of four consecutive elements, group j starting at 4 * (q + 64 j)
+// (16-byte aligned): one 16-byte value load and one 16-byte (or 8-byte for
+// 16-bit) index load each.  All streams are issued before the first gather
+// and all gathers before the first store (the compiler keeps a load behind
+// an earlier store, so each group would wait for its own gathers).
+template <typename IdxT, typename TF, typename TA, bool SUB, bool ADD, bool SWEEP, int N>
+__device__ __forceinline__ void groups4(const Ctx<TF>& k, const IdxT* __restrict__ idx, uint32_t q, float ysr,
+                                        float yar, TA& g, TA& h) {
     vf4* __restrict__ v4 = reinterpret_cast<vf4*>(k.a.val) + q;
-    const vf4 rv = __builtin_nontemporal_load(v4);
-    uint32_t c[4];
-    if constexpr (sizeof(IdxT) == 2) {
-        const vu2 cv = __builtin_nontemporal_load(reinterpret_cast<const vu2*>(idx) + q);
-        c[0] = cv.x & 0xffffu;
-        c[1] = cv.x >> 16;
-        c[2] = cv.y & 0xffffu;
-        c[3] = cv.y >> 16;
-    } else {
-        const vu4 cv = __builtin_nontemporal_load(reinterpret_cast<const vu4*>(idx) + q);
-        c[0] = cv.x;
-        c[1] = cv.y;
-        c[2] = cv.z;
-        c[3] = cv.w;
-    }
-    float r[4] = {rv.x, rv.y, rv.z, rv.w};
+    using IV = typename std::conditional<sizeof(IdxT) == 2, vu2, vu4>::type;
+    const IV* __restrict__ i4 = reinterpret_cast<const IV*>(idx) + q;
+    vf4 rv[N];
+    IV cv[N];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) one_elem<TF, TA, SUB, ADD, SWEEP>(k, c[j], r[j], ysr, yar, g, h);
-    if (SUB || ADD) __builtin_nontemporal_store(vf4{r[0], r[1], r[2], r[3]}, v4);
+    for (int j = 0; j < N; ++j) {
+        cv[j] = __builtin_nontemporal_load(i4 + WAVE * j);
+        rv[j] = __builtin_nontemporal_load(v4 + WAVE * j);
+    }
+    Gathered o[N][4];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        uint32_t c[4];
+        if constexpr (sizeof(IdxT) == 2) {
+            c[0] = cv[j].x & 0xffffu;
+            c[1] = cv[j].x >> 16;
+            c[2] = cv[j].y & 0xffffu;
+            c[3] = cv[j].y >> 16;
+        } else {
+            c[0] = cv[j].x;
+            c[1] = cv[j].y;
+            c[2] = cv[j].z;
+            c[3] = cv[j].w;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) o[j][u] = gather_elem<TF, SUB, ADD, SWEEP>(k, c[u]);
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        float r[4] = {rv[j].x, rv[j].y, rv[j].z, rv[j].w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) one_elem<TA, SUB, ADD, SWEEP>(o[j][u], r[u], ysr, yar, g, h);
+        if (SUB || ADD) __builtin_nontemporal_store(vf4{r[0], r[1], r[2], r[3]}, v4 + WAVE * j);
+    }
 }
 
 // Elements [s, e) by a whole wave: an unaligned head and tail of at most
-// three elements each, then the aligned body as 16-byte groups, two groups
-// (eight elements) per lane in flight.
+// three elements each, then the aligned body as 16-byte groups, four of them
+// (16 elements) per lane in flight.
 template <typename IdxT, typename TF, typename TA, bool SUB, bool ADD, bool SWEEP>
 __device__ __forceinline__ void wave_range(const Ctx<TF>& k, const IdxT* __restrict__ idx, uint32_t s, uint32_t e,
                                            uint32_t lane, float ysr, float yar, TA& g, TA& h) {
@@ -140,17 +172,26 @@ __device__ __forceinline__ void wave_range(const Ctx<TF>& k, const IdxT* __restr
     if (b0 > e) b0 = e;
     uint32_t b1 = e & ~3u;
     if (b1 < b0) b1 = b0;
-    if (lane < b0 - s)
-        strided_range<IdxT, TF, TA, SUB, ADD, SWEEP>(k, idx, s + lane, s + lane + 1, 1, ysr, yar, g, h);
-    if (lane < e - b1)
-        strided_range<IdxT, TF, TA, SUB, ADD, SWEEP>(k, idx, b1 + lane, b1 + lane + 1, 1, ysr, yar, g, h);
+    if (s >= e) return;
+    // head and tail: one element a lane each (other lanes load the first one
+    // again and drop it), so that their latencies overlap
+    const bool head = lane < b0 - s, tail = lane < e - b1;
+    const uint32_t ph = s + (head ? lane : 0u), pt = tail ? b1 + lane : s;
+    const uint32_t ch = __builtin_nontemporal_load(idx + ph), ct = __builtin_nontemporal_load(idx + pt);
+    float rh = __builtin_nontemporal_load(k.a.val + ph), rt = __builtin_nontemporal_load(k.a.val + pt);
+    const Gathered oh = gather_elem<TF, SUB, ADD, SWEEP>(k, ch), ot = gather_elem<TF, SUB, ADD, SWEEP>(k, ct);
+    if (head) one_elem<TA, SUB, ADD, SWEEP>(oh, rh, ysr, yar, g, h);
+    if (tail) one_elem<TA, SUB, ADD, SWEEP>(ot, rt, ysr, yar, g, h);
     const uint32_t q1 = b1 >> 2;
     uint32_t q = (b0 >> 2) + lane;
-    for (; q + WAVE < q1; q += 2 * WAVE) {
-        group4<IdxT, TF, TA, SUB, ADD, SWEEP>(k, idx, q, ysr, yar, g, h);
-        group4<IdxT, TF, TA, SUB, ADD, SWEEP>(k, idx, q + WAVE, ysr, yar, g, h);
+    constexpr uint32_t N = 4;
+    for (; q + (N - 1) * WAVE < q1; q += N * WAVE)
+        groups4<IdxT, TF, TA, SUB, ADD, SWEEP, (int)N>(k, idx, q, ysr, yar, g, h);
+    for (; q < q1; q += WAVE) groups4<IdxT, TF, TA, SUB, ADD, SWEEP, 1>(k, idx, q, ysr, yar, g, h);
+    if (SUB || ADD) {
+        if (head) __builtin_nontemporal_store(rh, k.a.val + ph);
+        if (tail) __builtin_nontemporal_store(rt, k.a.val + pt);
     }
-    if (q < q1) group4<IdxT, TF, TA, SUB, ADD, SWEEP>(k, idx, q, ysr, yar, g, h);
 }
 
 template <typename IdxT, typename TF, typename TA, bool SUB, bool ADD, bool SWEEP>
@@ -210,8 +251,13 @@ __global__ __launch_bounds__(SWEEP_BLOCK) void sweep_kernel(SweepArgs a) {
     const Ctx<TF> k{a, lds, ldsp};
     const int lane = threadIdx.x & (WAVE - 1);
     constexpr uint32_t NW = SWEEP_BLOCK / WAVE;
+    // Consecutive units go to different blocks: units come by falling row
+    // length, and the 16 longest rows in one block would put 20 times the
+    // mean number of gathers on its CU (99.1M ratings, one outer iteration of
+    // 40 ranks: 86 against 76 ms; 1.5M ratings: 18 against 14 us a
+    // sweep).
     const uint32_t stride = gridDim.x * NW;
-    for (uint32_t u = blockIdx.x * NW + (threadIdx.x >> 6); u < a.nunits; u += stride)
+    for (uint32_t u = (threadIdx.x >> 6) * gridDim.x + blockIdx.x; u < a.nunits; u += stride)
         sweep_unit<IdxT, TF, TA, SUB, ADD, SWEEP>(k, a.units[u], lane);
 }
 
@@ -222,7 +268,19 @@ __global__ __launch_bounds__(BLOCK) void finalize_kernel(FinalizeArgs a) {
     const uint32_t row = a.split_rows[i];
     const Pair<TA>* __restrict__ part = static_cast<const Pair<TA>*>(a.partials);
     TA g = 0, h = 0;
-    for (uint32_t q = a.split_beg[i]; q < a.split_beg[i + 1]; ++q) {
+    const uint32_t q1 = a.split_beg[i + 1];
+    uint32_t q = a.split_beg[i];
+    for (; q + 7 < q1; q += 8) {  // eight loads in flight, added in piece order
+        Pair<TA> p[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = part[q + j];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            g += p[j].g;
+            h += p[j].h;
+        }
+    }
+    for (; q < q1; ++q) {
         g += part[q].g;
         h += part[q].h;
     }
