@@ -89,6 +89,8 @@ struct ccd_mlp {
     size_t cap = 0;
     float *Xn = nullptr, *Z1 = nullptr, *A1 = nullptr, *Z2 = nullptr, *A2 = nullptr, *Yn = nullptr, *Tn = nullptr,
           *dY = nullptr, *dZ2 = nullptr, *dZ1 = nullptr;
+    float *I1 = nullptr, *I2 = nullptr;  // hidden activations of inference
+    size_t cap_i1 = 0, cap_i2 = 0;
     double *part = nullptr, *loss = nullptr;
     size_t cap_loss = 0;
     float* gpart = nullptr;  // split-K partials of the weight-gradient products
@@ -123,36 +125,42 @@ const void* wptr(const ccd_mlp* m, bool b16, size_t off) {
     return b16 ? static_cast<const void*>(m->P16 + off) : static_cast<const void*>(m->P + off);
 }
 
-// Yn = MLP(Xn) for n <= cap rows on stream s (workspace Z1..A2 filled).
-int mlp_forward_ws(ccd_mlp* m, uint32_t n, bool b16, hipStream_t s) {
+// Y = MLP(X) for n rows on stream s, hidden activations to A1 and A2.  infer: X and Y
+// raw (the norms are applied on the way in and out); otherwise both
+// standardised, and Z1, Z2 are kept for the gradients (n <= cap).
+int mlp_layers(ccd_mlp* m, uint32_t n, const float* X, float* A1, float* A2, bool infer, bool b16, float* Y,
+               hipStream_t s) {
+    const bool norm = infer && m->has_norm;
     ccd::GemmArgs g{};
-    g.A = m->Xn;
+    g.A = X;
     g.sai = m->in, g.sap = 1, g.sbp = 1, g.sbj = m->in;
     g.M = n, g.N = m->hid, g.K = m->in, g.ldc = m->hid;
-    g.bias = wptr(m, b16, m->ob1), g.C = m->Z1, g.C2 = m->A1;
+    if (norm) g.asub = m->in_sub, g.amul = m->in_mul;
+    g.bias = wptr(m, b16, m->ob1), g.C = infer ? nullptr : m->Z1, g.C2 = A1;
     OBJ_TRY(m, ccd::launch_gemm(g, wptr(m, b16, m->oW1), b16, ccd::GEMM_BIAS_GELU, s));
-    g.A = m->A1;
+    g.asub = g.amul = nullptr;
+    g.A = A1;
     g.sai = m->hid, g.sbj = m->hid, g.K = m->hid;
-    g.bias = wptr(m, b16, m->ob2), g.C = m->Z2, g.C2 = m->A2;
+    g.bias = wptr(m, b16, m->ob2), g.C = infer ? nullptr : m->Z2, g.C2 = A2;
     OBJ_TRY(m, ccd::launch_gemm(g, wptr(m, b16, m->oW2), b16, ccd::GEMM_BIAS_GELU, s));
-    g.A = m->A2;
+    g.A = A2;
     g.N = m->out, g.ldc = m->out;
-    g.bias = wptr(m, b16, m->ob3), g.C = m->Yn, g.C2 = nullptr;
+    if (norm) g.csub = m->out_sub, g.cmul = m->out_mul;
+    g.bias = wptr(m, b16, m->ob3), g.C = Y, g.C2 = nullptr;
     OBJ_TRY(m, ccd::launch_gemm(g, wptr(m, b16, m->oW3), b16, ccd::GEMM_STORE, s));
     return CCD_OK;
 }
 
-// Gradient of mean((Yn - Tn)^2) into G, loss into *loss_dev (after mlp_forward_ws, FP32).
+// Gradient of mean((Yn - Tn)^2) into G, loss into *loss_dev (after mlp_layers, FP32).
 int mlp_backward_ws(ccd_mlp* m, uint32_t n, double* loss_dev, hipStream_t s) {
     OBJ_TRY(m, ccd::launch_mse(m->Yn, m->Tn, (uint64_t)n * m->out, m->dY, m->part, loss_dev, s));
     ccd::GemmArgs g{};
-    // gW3 [out][hid] = dY^T A2
+    // gW3 [out][hid] = dY^T A2; the bias gradients are the row sums of the left operands
     g.A = m->dY, g.sai = 1, g.sap = m->out;
     g.sbp = m->hid, g.sbj = 1;
     g.M = m->out, g.N = m->hid, g.K = n, g.ldc = m->hid, g.C = m->G + m->oW3;
-    g.part = m->gpart, g.part_cap = m->gpart_cap;
+    g.part = m->gpart, g.part_cap = m->gpart_cap, g.rowsum = m->G + m->ob3;
     OBJ_TRY(m, ccd::launch_gemm(g, m->A2, false, ccd::GEMM_STORE, s));
-    OBJ_TRY(m, ccd::launch_colsum(m->dY, n, m->out, m->G + m->ob3, s));
     // dZ2 = (dY W3) * gelu'(Z2)
     g = ccd::GemmArgs{};
     g.A = m->dY, g.sai = m->out, g.sap = 1, g.sbp = m->hid, g.sbj = 1;
@@ -162,9 +170,8 @@ int mlp_backward_ws(ccd_mlp* m, uint32_t n, double* loss_dev, hipStream_t s) {
     g = ccd::GemmArgs{};
     g.A = m->dZ2, g.sai = 1, g.sap = m->hid, g.sbp = m->hid, g.sbj = 1;
     g.M = m->hid, g.N = m->hid, g.K = n, g.ldc = m->hid, g.C = m->G + m->oW2;
-    g.part = m->gpart, g.part_cap = m->gpart_cap;
+    g.part = m->gpart, g.part_cap = m->gpart_cap, g.rowsum = m->G + m->ob2;
     OBJ_TRY(m, ccd::launch_gemm(g, m->A1, false, ccd::GEMM_STORE, s));
-    OBJ_TRY(m, ccd::launch_colsum(m->dZ2, n, m->hid, m->G + m->ob2, s));
     // dZ1 = (dZ2 W2) * gelu'(Z1)
     g = ccd::GemmArgs{};
     g.A = m->dZ2, g.sai = m->hid, g.sap = 1, g.sbp = m->hid, g.sbj = 1;
@@ -174,9 +181,8 @@ int mlp_backward_ws(ccd_mlp* m, uint32_t n, double* loss_dev, hipStream_t s) {
     g = ccd::GemmArgs{};
     g.A = m->dZ1, g.sai = 1, g.sap = m->hid, g.sbp = m->in, g.sbj = 1;
     g.M = m->hid, g.N = m->in, g.K = n, g.ldc = m->in, g.C = m->G + m->oW1;
-    g.part = m->gpart, g.part_cap = m->gpart_cap;
+    g.part = m->gpart, g.part_cap = m->gpart_cap, g.rowsum = m->G + m->ob1;
     OBJ_TRY(m, ccd::launch_gemm(g, m->Xn, false, ccd::GEMM_STORE, s));
-    OBJ_TRY(m, ccd::launch_colsum(m->dZ1, n, m->hid, m->G + m->ob1, s));
     return CCD_OK;
 }
 
@@ -228,17 +234,17 @@ int mlp_forward_dev(ccd_mlp* m, uint64_t rows, const float* X, float* Y, int mod
         return CCD_OK;
     }
     const bool b16 = mode == 1;
-    const uint32_t chunk = 16384;
-    if (int rc = mlp_workspace(m, chunk)) return rc;
+    // rows at a time: three waves of 64 x 64 outputs for every SIMD at 256
+    // hidden units, at most 2 x 64 MB of activations
+    const uint32_t chunk = std::max<uint32_t>(std::min<uint32_t>(65536u, (1u << 24) / m->hid), 4096u);
+    const size_t most = (size_t)std::min<uint64_t>(chunk, rows) * m->hid;
+    OBJ_TRY(m, ensure(&m->I1, &m->cap_i1, most));
+    OBJ_TRY(m, ensure(&m->I2, &m->cap_i2, most));
     if (b16)
         if (int rc = mlp_sync_bf16(m, s)) return rc;
     for (uint64_t r0 = 0; r0 < rows; r0 += chunk) {
         const uint32_t n = (uint32_t)std::min<uint64_t>(chunk, rows - r0);
-        OBJ_TRY(m, ccd::launch_affine_rows(X + r0 * m->in, nullptr, n, m->in, m->has_norm ? m->in_sub : nullptr,
-                                           m->in_mul, m->Xn, s));
-        if (int rc = mlp_forward_ws(m, n, b16, s)) return rc;
-        OBJ_TRY(m, ccd::launch_affine_rows(m->Yn, nullptr, n, m->out, m->has_norm ? m->out_sub : nullptr, m->out_mul,
-                                           Y + r0 * m->out, s));
+        if (int rc = mlp_layers(m, n, X + r0 * m->in, m->I1, m->I2, true, b16, Y + r0 * m->out, s)) return rc;
     }
     return CCD_OK;
 }
@@ -265,8 +271,8 @@ int32_t ccd_mlp_create(int32_t device, uint32_t in, uint32_t hidden, uint32_t ou
     m->oW3 = m->ob2 + hidden;
     m->ob3 = m->oW3 + (size_t)out * hidden;
     m->np = m->ob3 + out;
-    m->gpart_cap = 16ull * std::max<uint64_t>({(uint64_t)hidden * hidden, (uint64_t)hidden * in,
-                                                (uint64_t)out * hidden});
+    m->gpart_cap = 16ull * std::max<uint64_t>({(uint64_t)hidden * (hidden + 1), (uint64_t)hidden * (in + 1),
+                                                (uint64_t)out * (hidden + 1)});
     // Glorot-uniform weights, zero biases, seeded
     std::vector<float> P(m->np, 0.0f);
     uint64_t st = seed ^ 0x6d6c7021ull;
@@ -303,7 +309,7 @@ int32_t ccd_mlp_destroy(ccd_mlp* m) {
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     void* bufs[] = {m->P, m->P16, m->G, m->mom, m->vel, m->in_sub, m->in_mul, m->out_sub, m->out_mul, m->tgt_sub,
                     m->tgt_mul, m->gpart, m->Xn, m->Z1,
-                    m->A1, m->Z2, m->A2, m->Yn, m->Tn, m->dY, m->dZ2, m->dZ1, m->part, m->loss, m->X, m->T, m->perm,
+                    m->A1, m->Z2, m->A2, m->Yn, m->Tn, m->dY, m->dZ2, m->dZ1, m->I1, m->I2, m->part, m->loss, m->X, m->T, m->perm,
                     m->pk, m->pkb};
     for (void* b : bufs) dfree(b);
     if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -368,22 +374,14 @@ int32_t ccd_mlp_forward(ccd_mlp* m, uint64_t rows, const float* X, float* Y, int
     if (!m || (rows && (!X || !Y))) return CCD_ERR_INVALID;
     if (rows == 0) return CCD_OK;
     OBJ_TRY(m, hipSetDevice(m->device));
-    float *dX = nullptr, *dYo = nullptr;
-    OBJ_TRY(m, dalloc(&dX, rows * m->in));
-    if (dalloc(&dYo, rows * m->out) != hipSuccess) {
-        dfree(dX);
-        return obj_err(m->err, CCD_ERR_ALLOC, "output buffer");
-    }
-    int rc = CCD_OK;
-    if (ccd::copy_sync(m->stream, dX, X, 4 * rows * m->in, hipMemcpyHostToDevice) != hipSuccess) rc = CCD_ERR_HIP;
-    if (bf16_weights < 0 || bf16_weights > 2) rc = obj_err(m->err, CCD_ERR_INVALID, "bf16_weights must be 0, 1 or 2");
-    if (!rc) rc = mlp_forward_dev(m, rows, dX, dYo, bf16_weights, m->stream);
-    if (!rc && hipStreamSynchronize(m->stream) != hipSuccess) rc = CCD_ERR_HIP;
-    if (!rc && hipMemcpy(Y, dYo, 4 * rows * m->out, hipMemcpyDeviceToHost) != hipSuccess) rc = CCD_ERR_HIP;
-    dfree(dX);
-    dfree(dYo);
-    if (rc == CCD_ERR_HIP && m->err.empty()) m->err = "copy or launch failed";
-    return rc;
+    if (bf16_weights < 0 || bf16_weights > 2) return obj_err(m->err, CCD_ERR_INVALID, "bf16_weights must be 0, 1 or 2");
+    // the rows pass through the training set's buffers
+    OBJ_TRY(m, ensure(&m->X, &m->cap_x, rows * m->in));
+    OBJ_TRY(m, ensure(&m->T, &m->cap_t, rows * m->out));
+    OBJ_TRY(m, hipMemcpyAsync(m->X, X, 4 * rows * m->in, hipMemcpyHostToDevice, m->stream));
+    if (int rc = mlp_forward_dev(m, rows, m->X, m->T, bf16_weights, m->stream)) return rc;
+    OBJ_TRY(m, ccd::copy_sync(m->stream, Y, m->T, 4 * rows * m->out, hipMemcpyDeviceToHost));
+    return CCD_OK;
 }
 
 int32_t ccd_mlp_loss_grad(ccd_mlp* m, uint64_t rows, const float* Xn, const float* Tn, double* loss, float* grad) {
@@ -391,13 +389,12 @@ int32_t ccd_mlp_loss_grad(ccd_mlp* m, uint64_t rows, const float* Xn, const floa
     OBJ_TRY(m, hipSetDevice(m->device));
     if (int rc = mlp_workspace(m, rows)) return rc;
     if (!m->loss) OBJ_TRY(m, dalloc(&m->loss, 1));
-    OBJ_TRY(m, ccd::copy_sync(m->stream, m->Xn, Xn, 4 * rows * m->in, hipMemcpyHostToDevice));
-    OBJ_TRY(m, ccd::copy_sync(m->stream, m->Tn, Tn, 4 * rows * m->out, hipMemcpyHostToDevice));
-    if (int rc = mlp_forward_ws(m, (uint32_t)rows, false, m->stream)) return rc;
+    OBJ_TRY(m, hipMemcpyAsync(m->Xn, Xn, 4 * rows * m->in, hipMemcpyHostToDevice, m->stream));
+    OBJ_TRY(m, hipMemcpyAsync(m->Tn, Tn, 4 * rows * m->out, hipMemcpyHostToDevice, m->stream));
+    if (int rc = mlp_layers(m, (uint32_t)rows, m->Xn, m->A1, m->A2, false, false, m->Yn, m->stream)) return rc;
     if (int rc = mlp_backward_ws(m, (uint32_t)rows, m->loss, m->stream)) return rc;
-    OBJ_TRY(m, hipStreamSynchronize(m->stream));
-    OBJ_TRY(m, hipMemcpy(loss, m->loss, sizeof(double), hipMemcpyDeviceToHost));
-    OBJ_TRY(m, hipMemcpy(grad, m->G, 4 * m->np, hipMemcpyDeviceToHost));
+    OBJ_TRY(m, hipMemcpyAsync(loss, m->loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
+    OBJ_TRY(m, ccd::copy_sync(m->stream, grad, m->G, 4 * m->np, hipMemcpyDeviceToHost));
     return CCD_OK;
 }
 
@@ -431,7 +428,7 @@ int32_t ccd_mlp_train(ccd_mlp* m, uint64_t rows, const float* X, const float* T,
             OBJ_TRY(m, ccd::launch_affine_rows(m->X, pr, n, m->in, m->has_norm ? m->in_sub : nullptr, m->in_mul, m->Xn, s));
             OBJ_TRY(m, ccd::launch_affine_rows(m->T, pr, n, m->out, m->has_norm ? m->tgt_sub : nullptr, m->tgt_mul,
                                                m->Tn, s));
-            if (int rc = mlp_forward_ws(m, n, false, s)) return rc;
+            if (int rc = mlp_layers(m, n, m->Xn, m->A1, m->A2, false, false, m->Yn, s)) return rc;
             if (int rc = mlp_backward_ws(m, n, m->loss + q, s)) return rc;
             ++m->step;
             ccd::AdamArgs ad{m->P, m->G, m->mom, m->vel, m->np, lr, b1, b2, 1e-8f,
@@ -503,6 +500,7 @@ struct ccd_fold {
     int64_t n = 0;
     float lambda = 0.0f;
     float* HT = nullptr;  // [n + 1][fold_ld(k)], ccd::FoldArgs
+    float* H = nullptr;   // the caller's [k][n], transposed into HT (kept: freeing it would wait for the device)
     uint32_t *ptr = nullptr, *idx = nullptr, *long_rows = nullptr;
     uint32_t* bad = nullptr;  // fold_check_device
     uint32_t nlong = 0, nfeat = 0;  // rows longer than FOLD_WAVE, and than FOLD_SHORT
@@ -608,15 +606,13 @@ int32_t ccd_fold_create(int32_t device, uint32_t k, int64_t n, const float* H, f
     if (!f) return CCD_ERR_ALLOC;
     f->device = device, f->k = k, f->n = n, f->lambda = lambda;
     const size_t kn = (size_t)k * n, nht = ((size_t)n + 1) * fold_ld(k);
-    float* dH = nullptr;  // the caller's [k][n], until it is transposed
     bool ok = hipSetDevice(device) == hipSuccess && hipStreamCreateWithFlags(&f->stream, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreate(&f->ea) == hipSuccess && hipEventCreate(&f->eb) == hipSuccess &&
-              dalloc(&dH, kn) == hipSuccess && dalloc(&f->HT, nht) == hipSuccess && dalloc(&f->bad, 1) == hipSuccess &&
+              dalloc(&f->H, kn) == hipSuccess && dalloc(&f->HT, nht) == hipSuccess && dalloc(&f->bad, 1) == hipSuccess &&
               ccd::launch_fill(f->HT, 0.0f, nht, f->stream) == hipSuccess &&
-              ccd::copy_sync(f->stream, dH, H, 4 * kn, hipMemcpyHostToDevice) == hipSuccess &&
-              ccd::launch_transpose(dH, f->HT, k, (uint32_t)n, fold_ld(k), f->stream) == hipSuccess &&
+              ccd::copy_sync(f->stream, f->H, H, 4 * kn, hipMemcpyHostToDevice) == hipSuccess &&
+              ccd::launch_transpose(f->H, f->HT, k, (uint32_t)n, fold_ld(k), f->stream) == hipSuccess &&
               hipStreamSynchronize(f->stream) == hipSuccess && scratch_on(device, &f->scratch) == hipSuccess;
-    dfree(dH);
     if (!ok) {
         ccd_fold_destroy(f);
         return CCD_ERR_HIP;
@@ -629,7 +625,7 @@ int32_t ccd_fold_destroy(ccd_fold* f) {
     if (!f) return CCD_OK;
     (void)hipSetDevice(f->device);
     if (f->stream) (void)hipStreamSynchronize(f->stream);
-    void* bufs[] = {f->HT, f->bad, f->ptr, f->idx, f->val, f->W0, f->W, f->F, f->long_rows};
+    void* bufs[] = {f->H, f->HT, f->bad, f->ptr, f->idx, f->val, f->W0, f->W, f->F, f->long_rows};
     for (void* b : bufs) dfree(b);
     if (f->ea) (void)hipEventDestroy(f->ea);
     if (f->eb) (void)hipEventDestroy(f->eb);

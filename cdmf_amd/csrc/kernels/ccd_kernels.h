@@ -507,8 +507,9 @@ hipError_t launch_transpose(const float* src, float* dst, uint32_t rows, uint32_
 // C(i, j) = sum_p A(i, p) B(p, j) for i < M, j < N, p < K with
 // A(i, p) = A[i sai + p sap] (FP32), B(p, j) = B[p sbp + j sbj] (FP32 or
 // bfloat16); epilogues: GEMM_STORE C = acc (+ bias[j]); GEMM_BIAS_GELU
-// C = acc + bias[j], C2 = GELU(C); GEMM_GELU_GRAD C = acc * GELU'(aux)
-// (aux, C, C2 row-major with leading dimension ldc).
+// C = acc + bias[j] (C may be null), C2 = GELU(that); GEMM_GELU_GRAD C = acc *
+// GELU'(aux) (aux, C, C2 row-major with leading dimension ldc).  Supported:
+// sap = sbp = 1, GEMM_GELU_GRAD with sap = 1, and, with rowsum, any strides.
 constexpr int GEMM_STORE = 0, GEMM_BIAS_GELU = 1, GEMM_GELU_GRAD = 2;
 struct GemmArgs {
     const float* A;
@@ -518,8 +519,11 @@ struct GemmArgs {
     float* C;
     float* C2;
     const float* aux;
-    float* part;       // optional workspace of part_cap floats: a plain product (GEMM_STORE, no
-    uint64_t part_cap; // bias) with few output tiles splits K over slices, summed in slice order
+    float* part;       // optional workspace of part_cap floats: a weight gradient (GEMM_STORE, no
+    uint64_t part_cap; // bias) over a long K splits it over slices, summed in slice order
+    const float *asub, *amul;  // optional map of A's columns on the way in: (a - asub[p]) amul[p]
+    const float *csub, *cmul;  // optional map of the output (GEMM_STORE): (c - csub[j]) cmul[j]
+    float* rowsum;             // optional (weight gradients): rowsum[i] = sum_p A(i, p)
 };
 hipError_t launch_gemm(const GemmArgs& g, const void* B, bool bf16_b, int epi, hipStream_t s);
 
@@ -544,7 +548,6 @@ struct MlpInferArgs {
 hipError_t launch_mlp_infer(const MlpInferArgs& g, hipStream_t s);
 hipError_t launch_mlp_pack(const float* P, uint32_t in, uint32_t out, uint32_t kin, uint32_t nout, uint16_t* W1,
                            uint16_t* W2, uint16_t* W3, float* b1, float* b2, float* b3, hipStream_t s);
-hipError_t launch_colsum(const float* dZ, uint32_t M, uint32_t N, float* out, hipStream_t s);
 // dY = 2 (Y - T) / count; *out = mean (Y - T)^2 (FP64, fixed order); part: MSE_PARTS doubles
 constexpr uint32_t MSE_PARTS = 1024;
 hipError_t launch_mse(const float* Y, const float* T, uint64_t count, float* dY, double* part, double* out,
