@@ -113,12 +113,6 @@ int prepare(ccd_batch* b, int sigma) {
         c->prec = CCD_PREC_FP32;
         for (ccdi::DevLayout* L : {&c->csr, &c->csc}) {
             if (int rc = ccdi::build_tiled(c, *L, sigma, 0u)) return ctx_err(b, i, rc);
-            if (!L->pair) {
-                double2* d = nullptr;
-                if (ccdi::dalloc(&d, ((size_t)L->gdim + 1) / 2) != hipSuccess)
-                    return berr(b, CCD_ERR_ALLOC, "problem " + std::to_string(i) + ": pair buffer");
-                L->pair = d;
-            }
         }
     }
     return CCD_OK;

@@ -59,37 +59,13 @@ int ensure_stage(ccd_ctx* c, size_t count) {
 }
 
 void free_tiled(TiledLayout& T) {
-    dfree(T.tidx);
-    dfree(T.tval);
-    dfree(T.flags);
-    dfree(T.row0);
-    dfree(T.segoff);
-    dfree(T.segrows);
-    dfree(T.open);
-    dfree(T.gmax);
-    dfree(T.head);
-    dfree(T.tail);
-    dfree(T.spans);
-    dfree(T.vpos);
-    dfree(T.cold_row);
-    dfree(T.srows);
-    dfree(T.part);
+    dfree(T.mem);
     T = TiledLayout{};
 }
 
 void free_layout(DevLayout& L) {
     free_tiled(L.tl);
-    dfree(L.ptr);
-    dfree(L.idx);
-    dfree(L.val);
-    dfree(L.val0);
-    dfree(L.units);
-    dfree(L.split_rows);
-    dfree(L.split_beg);
-    dfree(L.partials);
-    dfree(L.pair);
-    dfree(L.src);
-    dfree(L.dperm);
+    dfree(L.mem);
     L = DevLayout{};
 }
 
@@ -192,7 +168,7 @@ struct Timed {
     bool bound;
     hipEvent_t a = nullptr, b = nullptr;
     Timed(ccd_ctx* ctx, int k, bool bind = false) : c(ctx), kind(k), bound(bind) {
-        if (!c->prof || (k >= 0 && c->prof_kinds && !((c->prof_kinds >> k) & 1u))) return;
+        if (!c->prof || c->prof_iter || (k >= 0 && c->prof_kinds && !((c->prof_kinds >> k) & 1u))) return;
         if (bound && k >= 0 && c->prof_kinds && c->kind_seen[k]++ % PROF_SAMPLE != 0) return;
         a = take_event(c);
         b = take_event(c);
@@ -237,6 +213,29 @@ double layout_bytes(const DevLayout& L, bool tiled, bool split, bool residual_wr
     if (writes_y) b += 4.0 * (double)L.rows;
     return b;
 }
+
+// CCD_PROFILE_ITER: event records at the bounds of the groups of launches
+// that the iteration callback reports, each group ending where the next one
+// begins.
+struct GroupTimer {
+    ccd_ctx* c;
+    hipEvent_t last = nullptr;
+    bool on() const { return c->prof && c->prof_iter; }
+    void begin() {  // the next group starts here
+        if (!on()) return;
+        last = take_event(c);
+        if (last) (void)hipEventRecord(last, c->stream);
+    }
+    void end(int kind) {  // a group of this kind ends here
+        if (!on() || !last) return;
+        hipEvent_t e = take_event(c);
+        if (e) {
+            (void)hipEventRecord(e, c->stream);
+            c->recs.push_back({kind, last, e});
+        }
+        last = e;
+    }
+};
 
 struct RunState {
     ccd_ctx* c;
@@ -345,19 +344,17 @@ int do_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* xs, co
 using PassFn = int (*)(ccd_ctx*, DevLayout&, const void*, void*, const void*, const void*, const void*,
                       const void*, bool, bool, bool, bool, float, int);
 
-// Device memory of one set-up call.
-template <class T>
-struct Scratch {
-    T* p = nullptr;
-    Scratch() = default;
-    Scratch(const Scratch&) = delete;
-    Scratch& operator=(const Scratch&) = delete;
-    ~Scratch() { release(); }
-    hipError_t alloc(size_t count) { return dalloc(&p, count); }
-    void release() {
-        dfree(p);
-        p = nullptr;
-    }
+// Device memory of one upload.
+struct UploadScratch {
+    void* mem = nullptr;
+    uint32_t *ridx = nullptr, *kidx = nullptr;  // the caller's indices
+    uint32_t *rpos = nullptr, *cpos = nullptr;  // caller's row / column -> internal
+    uint32_t *ptr = nullptr, *dup = nullptr;    // of the copy being renumbered
+    uint32_t* bad = nullptr;
+    UploadScratch() = default;
+    UploadScratch(const UploadScratch&) = delete;
+    UploadScratch& operator=(const UploadScratch&) = delete;
+    ~UploadScratch() { dfree(mem); }
 };
 
 // One compressed copy into internal numbering: its rows in `perm` order (by
@@ -365,7 +362,8 @@ struct Scratch {
 // internal), the elements of every row sorted by internal index.  didx: the
 // caller's indices on the device, checked.
 int upload_layout(ccd_ctx* c, DevLayout& L, int64_t rows, int64_t gdim, uint64_t nnz, const uint32_t* cptr,
-                  const uint32_t* didx, const float* val, const std::vector<uint32_t>& perm, const uint32_t* ipos) {
+                  const uint32_t* didx, const float* val, const std::vector<uint32_t>& perm, const uint32_t* ipos,
+                  const UploadScratch& tmp) {
     L.rows = rows;
     L.gdim = gdim;
     L.nnz = nnz;
@@ -388,59 +386,47 @@ int upload_layout(ccd_ctx* c, DevLayout& L, int64_t rows, int64_t gdim, uint64_t
         }
     }
     const uint32_t* ptr = L.hptr.data();
-    HIP_TRY(c, dalloc(&L.ptr, rows + 1));
-    HIP_TRY(c, hipMemcpyAsync(L.ptr, ptr, sizeof(uint32_t) * (rows + 1), hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, dalloc(&L.dperm, rows));
-    HIP_TRY(c, hipMemcpyAsync(L.dperm, perm.data(), sizeof(uint32_t) * rows, hipMemcpyHostToDevice, c->stream));
-    {
-        uint8_t* d = nullptr;
-        HIP_TRY(c, dalloc(&d, (L.idx16 ? 2 : 4) * (size_t)nnz));
-        L.idx = d;
-    }
-    HIP_TRY(c, dalloc(&L.val, nnz));
-    HIP_TRY(c, dalloc(&L.val0, nnz));
-    HIP_TRY(c, dalloc(&L.src, nnz));
-    if (nnz) {
-        // the caller's values pass through L.val
-        Scratch<uint32_t> dptr, dup;
-        HIP_TRY(c, dptr.alloc((size_t)rows + 1));
-        HIP_TRY(c, dup.alloc((size_t)cls.nlong + 1));
-        HIP_TRY(c, hipMemcpyAsync(dptr.p, cptr, sizeof(uint32_t) * (rows + 1), hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(c, hipMemcpyAsync(L.val, val, sizeof(float) * nnz, hipMemcpyHostToDevice, c->stream));
-        const ccd::RenumArgs ra{dptr.p, didx, L.val, L.dperm, ipos, L.ptr, L.idx, L.val0, L.src, (uint32_t)gdim};
-        const hipError_t e1 = ccd::launch_renumber(ra, L.idx16, cls, dup.p, c->stream);
-        const hipError_t e2 = hipMemcpyAsync(L.val, L.val0, sizeof(float) * nnz, hipMemcpyDeviceToDevice, c->stream);
-        const hipError_t e3 = hipStreamSynchronize(c->stream);  // before dptr and dup go
-        HIP_TRY(c, e1);
-        HIP_TRY(c, e2);
-        HIP_TRY(c, e3);
-    } else {
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-    }
-
     HostPlan P = make_plan(ptr, rows, c->plan, (uint32_t)c->ncu * (ccd::SWEEP_BLOCK / 64));
     if (P.split_beg.back() >= (1u << 24) || P.units.size() >= 0xffffffffull)
         return set_err(c, CCD_ERR_INVALID, "work plan too large: raise ccd_plan_params.piece");
     L.nunits = (uint32_t)P.units.size();
     L.nsplit = (uint32_t)P.split_rows.size();
     L.npieces = P.split_beg.back();
-    HIP_TRY(c, dalloc(&L.units, P.units.size()));
-    if (!P.units.empty())
-        HIP_TRY(c, ccd::copy_sync(c->stream, L.units, P.units.data(), sizeof(uint4) * P.units.size(), hipMemcpyHostToDevice));
-    HIP_TRY(c, dalloc(&L.split_rows, P.split_rows.size()));
-    if (!P.split_rows.empty())
-        HIP_TRY(c, ccd::copy_sync(c->stream, L.split_rows, P.split_rows.data(), sizeof(uint32_t) * P.split_rows.size(),
-                                  hipMemcpyHostToDevice));
-    HIP_TRY(c, dalloc(&L.split_beg, P.split_beg.size()));
-    HIP_TRY(c, ccd::copy_sync(c->stream, L.split_beg, P.split_beg.data(), sizeof(uint32_t) * P.split_beg.size(), hipMemcpyHostToDevice));
-    HIP_TRY(c, dalloc(&L.partials, L.npieces));
-    return CCD_OK;
-}
-
-template <class T>
-int upload_vec(ccd_ctx* c, T** dst, const std::vector<T>& v) {
-    HIP_TRY(c, dalloc(dst, v.size()));
-    if (!v.empty()) HIP_TRY(c, ccd::copy_sync(c->stream, *dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+    uint8_t* idx8 = nullptr;
+    double2* pair = nullptr;
+    Carver mem;
+    mem.add(&L.ptr, (size_t)rows + 1);
+    mem.add(&L.dperm, (size_t)rows);
+    mem.add(&L.dbelow, (size_t)rows);
+    mem.add(&idx8, (L.idx16 ? 2 : 4) * (size_t)nnz);
+    mem.add(&L.val, nnz);
+    mem.add(&L.val0, nnz);
+    mem.add(&L.src, nnz);
+    mem.add(&L.units, P.units.size());
+    mem.add(&L.split_rows, P.split_rows.size());
+    mem.add(&L.split_beg, P.split_beg.size());
+    mem.add(&L.partials, L.npieces);
+    mem.add(&pair, ((size_t)gdim + 1) / 2);  // FP32 pairs, so every precision fits
+    HIP_TRY(c, mem.alloc(&L.mem));
+    L.idx = idx8;
+    L.pair = pair;
+    auto to_device = [&](void* dst, const void* src, size_t bytes) {
+        return bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream) : hipSuccess;
+    };
+    HIP_TRY(c, to_device(L.ptr, ptr, sizeof(uint32_t) * (rows + 1)));
+    HIP_TRY(c, to_device(L.dperm, perm.data(), sizeof(uint32_t) * rows));
+    HIP_TRY(c, to_device(L.units, P.units.data(), sizeof(uint4) * P.units.size()));
+    HIP_TRY(c, to_device(L.split_rows, P.split_rows.data(), sizeof(uint32_t) * P.split_rows.size()));
+    HIP_TRY(c, to_device(L.split_beg, P.split_beg.data(), sizeof(uint32_t) * P.split_beg.size()));
+    if (nnz) {
+        // the caller's values pass through L.val
+        HIP_TRY(c, to_device(tmp.ptr, cptr, sizeof(uint32_t) * (rows + 1)));
+        HIP_TRY(c, to_device(L.val, val, sizeof(float) * nnz));
+        const ccd::RenumArgs ra{tmp.ptr, didx, L.val, L.dperm, ipos, L.ptr, L.idx, L.val0, L.src, (uint32_t)gdim};
+        HIP_TRY(c, ccd::launch_renumber(ra, L.idx16, cls, tmp.dup, c->stream));
+        HIP_TRY(c, hipMemcpyAsync(L.val, L.val0, sizeof(float) * nnz, hipMemcpyDeviceToDevice, c->stream));
+    }
+    HIP_TRY(c, hipStreamSynchronize(c->stream));  // the plan's vectors end here
     return CCD_OK;
 }
 
@@ -463,63 +449,69 @@ int build_tiled(ccd_ctx* c, DevLayout& L, int sigma, uint32_t split_at) {
     L.below.clear();
     TiledLayout& T = L.tl;
     if (split) {
-        uint32_t* d = nullptr;
-        HIP_TRY(c, dalloc(&d, (size_t)std::max<int64_t>(L.rows, 1)));
         L.below.resize((size_t)L.rows);
-        hipError_t e = ccd::launch_count_below(L.ptr, L.idx, L.idx16, (uint64_t)L.rows, split_at, d, c->stream);
-        if (e == hipSuccess && L.rows)
-            e = ccd::copy_sync(c->stream, L.below.data(), d, sizeof(uint32_t) * (size_t)L.rows, hipMemcpyDeviceToHost);
-        dfree(d);
-        HIP_TRY(c, e);
+        HIP_TRY(c, ccd::launch_count_below(L.ptr, L.idx, L.idx16, (uint64_t)L.rows, split_at, L.dbelow, c->stream));
+        HIP_TRY(c, ccd::copy_sync(c->stream, L.below.data(), L.dbelow, sizeof(uint32_t) * (size_t)L.rows,
+                                  hipMemcpyDeviceToHost));
     }
     ccd::TileTables H;
-    const std::string why =
-        ccd::build_tile_tables(L.hptr.data(), L.rows, L.nnz, split ? L.below.data() : nullptr, sigma, split, H);
+    const std::string why = ccd::build_tile_tables(L.hptr.data(), L.rows, L.nnz, split ? L.below.data() : nullptr, sigma,
+                                                   split, H, false);
     if (!why.empty()) return set_err(c, CCD_ERR_INVALID, "tile layout: " + why);
-    const uint64_t TS = 64ull * (uint64_t)sigma, nnz = L.nnz, ntiles = H.ntiles;
+    const uint64_t TS = 64ull * (uint64_t)sigma, nnz = L.nnz, ntiles = H.ntiles, padded = ntiles * TS;
     T.ntiles = (uint32_t)ntiles;
     T.nspan = (uint32_t)H.spans.size();
     T.nshort = H.nshort;
-    int rc;
-    if (sigma <= 16) {  // the row-start bits of a lane fit 16 bits: half the stream
-        std::vector<uint16_t> f16(H.flags.begin(), H.flags.end());
-        uint16_t* d = nullptr;
-        rc = upload_vec(c, &d, f16);
-        T.flags = d;
-    } else {
-        uint32_t* d = nullptr;
-        rc = upload_vec(c, &d, H.flags);
-        T.flags = d;
-    }
-    if (rc) return rc;
-    if ((rc = upload_vec(c, &T.row0, H.row0)) ||
-        (rc = upload_vec(c, &T.segoff, H.segoff)) || (rc = upload_vec(c, &T.segrows, H.segrows)) ||
-        (rc = upload_vec(c, &T.open, H.open)) || (rc = upload_vec(c, &T.spans, H.spans)))
-        return rc;
     T.cold_tile0 = H.cold_tile0;
+    T.ib = tiled_index_bytes(L);
+    uint8_t* tidx = nullptr;  // the 3-byte format: u16 plane, then u8 plane
+    uint32_t* flags = nullptr;  // the row-start bits of a lane: 16 bits up to sigma 16, else 32
+    Carver mem;
+    mem.add(&flags, ntiles * (sigma <= 16 ? 32 : 64));
+    mem.add(&T.row0, H.row0.size());
+    mem.add(&T.segoff, H.segoff.size());
+    mem.add(&T.segrows, H.segrows.size());
+    mem.add(&T.open, H.open.size());
+    mem.add(&T.spans, H.spans.size());
+    if (split) {
+        mem.add(&T.vptr, H.vptr.size());
+        mem.add(&T.vpos, nnz);
+        mem.add(&T.cold_row, H.cold_row.size());
+        mem.add(&T.srows, H.srows.size());
+        mem.add(&T.part, H.vptr.size() - 1);
+    }
+    mem.add(&T.tval, padded);
+    mem.add(&T.gmax, ntiles);
+    mem.add(&T.head, ntiles);
+    mem.add(&T.tail, ntiles);
+    mem.add(&tidx, padded * (size_t)T.ib);
+    HIP_TRY(c, mem.alloc(&T.mem));
+    T.flags = flags;
+    T.tidx = tidx;
+    auto to_device = [&](auto* dst, const auto& v) {
+        return v.empty() ? hipSuccess
+                         : hipMemcpyAsync(dst, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice, c->stream);
+    };
+    HIP_TRY(c, to_device(T.row0, H.row0));
+    HIP_TRY(c, to_device(T.segoff, H.segoff));
+    HIP_TRY(c, to_device(T.segrows, H.segrows));
+    HIP_TRY(c, to_device(T.open, H.open));
+    HIP_TRY(c, to_device(T.spans, H.spans));
     if (split) {
         T.nreal = H.nreal;
-        if ((rc = upload_vec(c, &T.vpos, H.vpos)) || (rc = upload_vec(c, &T.cold_row, H.cold_row)) ||
-            (rc = upload_vec(c, &T.srows, H.srows)))
-            return rc;
-        HIP_TRY(c, dalloc(&T.part, H.vptr.size() - 1));
+        HIP_TRY(c, to_device(T.vptr, H.vptr));
+        HIP_TRY(c, to_device(T.cold_row, H.cold_row));
+        HIP_TRY(c, to_device(T.srows, H.srows));
+        HIP_TRY(c, ccd::launch_split_positions(T.vptr, H.vptr.size() - 1, L.ptr, L.dbelow, T.cold_row, T.nreal, T.vpos,
+                                               c->stream));
     }
-    const uint64_t padded = ntiles * TS;
-    HIP_TRY(c, dalloc(&T.tval, padded));
-    HIP_TRY(c, dalloc(&T.gmax, ntiles));
-    HIP_TRY(c, dalloc(&T.head, ntiles));
-    HIP_TRY(c, dalloc(&T.tail, ntiles));
-    T.ib = tiled_index_bytes(L);
-    {
-        uint8_t* d = nullptr;  // the 3-byte format: u16 plane, then u8 plane
-        HIP_TRY(c, dalloc(&d, padded * (size_t)T.ib));
-        T.tidx = d;
-    }
+    HIP_TRY(c, ccd::launch_tile_flags(split ? T.vptr : L.ptr, split ? H.vptr.size() - 1 : (uint64_t)L.rows, ntiles, sigma,
+                                      flags, c->stream));
     if (ntiles) {
         HIP_TRY(c, ccd::launch_retile_idx(L.idx, L.idx16, T.tidx, T.ib, nnz, T.ntiles, sigma, T.vpos, c->stream));
         HIP_TRY(c, ccd::launch_tile_gmax(L.idx, L.idx16, T.segoff, T.gmax, nnz, T.ntiles, sigma, T.vpos, c->stream));
     }
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));  // the host tables end here
     T.sigma = sigma;  // only a complete layout is reused
     T.split = split;
     L.split_at = split_at;
@@ -590,18 +582,15 @@ const char* check_pointers(int64_t rows, uint64_t nnz, const uint32_t* ptr) {
 
 // The caller's indices on the device, checked there: *out_of_range set when
 // one is not below dim.
-int upload_indices(ccd_ctx* c, Scratch<uint32_t>& d, const uint32_t* idx, uint64_t nnz, int64_t dim,
+int upload_indices(ccd_ctx* c, const UploadScratch& tmp, uint32_t* d, const uint32_t* idx, uint64_t nnz, int64_t dim,
                    bool* out_of_range) {
     *out_of_range = false;
     if (nnz == 0) return CCD_OK;
-    Scratch<uint32_t> flag;
-    HIP_TRY(c, d.alloc(nnz));
-    HIP_TRY(c, flag.alloc(1));
     uint32_t bad = 0;
-    HIP_TRY(c, hipMemcpyAsync(d.p, idx, sizeof(uint32_t) * nnz, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, ccd::launch_fill(reinterpret_cast<float*>(flag.p), 0.0f, 1, c->stream));
-    HIP_TRY(c, ccd::launch_index_check(d.p, nnz, (uint32_t)dim, flag.p, c->stream));
-    HIP_TRY(c, ccd::copy_sync(c->stream, &bad, flag.p, sizeof(bad), hipMemcpyDeviceToHost));
+    HIP_TRY(c, hipMemcpyAsync(d, idx, sizeof(uint32_t) * nnz, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, ccd::launch_fill(reinterpret_cast<float*>(tmp.bad), 0.0f, 1, c->stream));
+    HIP_TRY(c, ccd::launch_index_check(d, nnz, (uint32_t)dim, tmp.bad, c->stream));
+    HIP_TRY(c, ccd::copy_sync(c->stream, &bad, tmp.bad, sizeof(bad), hipMemcpyDeviceToHost));
     *out_of_range = bad != 0;
     return CCD_OK;
 }
@@ -677,8 +666,7 @@ int32_t ccd_destroy(ccd_ctx* c) {
     dfree(c->trow);
     dfree(c->tcol);
     dfree(c->tval);
-    dfree(c->W);
-    dfree(c->H);
+    dfree(c->fmem);
     dfree(c->u);
     dfree(c->v);
     dfree(c->W16);
@@ -723,12 +711,22 @@ int32_t ccd_upload(ccd_ctx* c, int64_t m, int64_t n, uint64_t nnz, const uint32_
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     // every check comes before the first change: a refused upload leaves the
     // context as it was
-    Scratch<uint32_t> ridx, kidx;
+    UploadScratch tmp;
+    Carver mem;
+    const size_t most = (size_t)std::max(m, n) + 1;
+    mem.add(&tmp.ridx, nnz);
+    mem.add(&tmp.kidx, nnz);
+    mem.add(&tmp.rpos, (size_t)m);
+    mem.add(&tmp.cpos, (size_t)n);
+    mem.add(&tmp.ptr, most);
+    mem.add(&tmp.dup, most);
+    mem.add(&tmp.bad, 1);
+    HIP_TRY(c, mem.alloc(&tmp.mem));
     bool bad = false;
-    if (int rc = upload_indices(c, ridx, col_idx, nnz, n, &bad)) return rc;
+    if (int rc = upload_indices(c, tmp, tmp.ridx, col_idx, nnz, n, &bad)) return rc;
     if (bad) return set_err(c, CCD_ERR_INVALID, "CSR: index out of range");
     if (const char* why = check_pointers(n, nnz, col_ptr)) return set_err(c, CCD_ERR_INVALID, std::string("CSC: ") + why);
-    if (int rc = upload_indices(c, kidx, row_idx, nnz, m, &bad)) return rc;
+    if (int rc = upload_indices(c, tmp, tmp.kidx, row_idx, nnz, m, &bad)) return rc;
     if (bad) return set_err(c, CCD_ERR_INVALID, "CSC: index out of range");
     drop_graph(c);
     ++c->gen;
@@ -736,6 +734,12 @@ int32_t ccd_upload(ccd_ctx* c, int64_t m, int64_t n, uint64_t nnz, const uint32_
     free_layout(c->csc);
     c->uploaded = false;
     c->factors = false;
+    // factor buffers are sized by m and n: the next ccd_set_factors and run
+    // make them anew
+    c->k = c->k16 = 0;
+    dfree(c->u16);
+    dfree(c->v16);
+    c->u16 = c->v16 = nullptr;
     c->m = m;
     c->n = n;
     c->nnz = nnz;
@@ -747,14 +751,11 @@ int32_t ccd_upload(ccd_ctx* c, int64_t m, int64_t n, uint64_t nnz, const uint32_
         // Rows sorted by gathered index: the tiled sweeps can then split
         // each row at any bound (build_tiled) and keep the elements gathered
         // from beyond an LDS prefix in tiles of their own.
-        Scratch<uint32_t> drpos, dcpos;
-        HIP_TRY(c, drpos.alloc((size_t)m));
-        HIP_TRY(c, dcpos.alloc((size_t)n));
-        HIP_TRY(c, ccd::copy_sync(c->stream, drpos.p, rpos.data(), sizeof(uint32_t) * (size_t)m, hipMemcpyHostToDevice));
-        HIP_TRY(c, ccd::copy_sync(c->stream, dcpos.p, cpos.data(), sizeof(uint32_t) * (size_t)n, hipMemcpyHostToDevice));
-        if (int rc = upload_layout(c, c->csr, m, n, nnz, row_ptr, ridx.p, csr_val, rperm, dcpos.p)) return rc;
-        ridx.release();
-        if (int rc = upload_layout(c, c->csc, n, m, nnz, col_ptr, kidx.p, csc_val, cperm, drpos.p)) return rc;
+        HIP_TRY(c, hipMemcpyAsync(tmp.rpos, rpos.data(), sizeof(uint32_t) * (size_t)m, hipMemcpyHostToDevice, c->stream));
+        HIP_TRY(c, hipMemcpyAsync(tmp.cpos, cpos.data(), sizeof(uint32_t) * (size_t)n, hipMemcpyHostToDevice, c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        if (int rc = upload_layout(c, c->csr, m, n, nnz, row_ptr, tmp.ridx, csr_val, rperm, tmp.cpos, tmp)) return rc;
+        if (int rc = upload_layout(c, c->csc, n, m, nnz, col_ptr, tmp.kidx, csc_val, cperm, tmp.rpos, tmp)) return rc;
         c->csr.perm = std::move(rperm);
         c->csc.perm = std::move(cperm);
     }
@@ -824,19 +825,22 @@ int32_t ccd_set_factors(ccd_ctx* c, uint32_t k, const float* W, const float* H) 
     if (k != c->k) {
         drop_graph(c);
         ++c->gen;
-        dfree(c->W);
-        dfree(c->H);
-        c->W = c->H = nullptr;
-        HIP_TRY(c, dalloc(&c->W, (size_t)k * c->m));
-        HIP_TRY(c, dalloc(&c->H, (size_t)k * c->n));
+        dfree(c->fmem);
+        c->fmem = nullptr;
+        c->W = c->H = c->fstage = nullptr;
+        c->k = 0;
+        Carver mem;
+        mem.add(&c->W, (size_t)k * c->m);
+        mem.add(&c->H, (size_t)k * c->n);
+        mem.add(&c->fstage, (size_t)k * std::max(c->m, c->n));
+        HIP_TRY(c, mem.alloc(&c->fmem));
         c->k = k;
     }
     const size_t nW = (size_t)k * c->m, nH = (size_t)k * c->n;
-    if (int rc = ensure_stage(c, std::max(nW, nH))) return rc;
-    HIP_TRY(c, hipMemcpyAsync(c->stage, W, sizeof(float) * nW, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, ccd::launch_permute_ranks(c->stage, c->W, c->csr.dperm, k, c->m, true, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(c->stage, H, sizeof(float) * nH, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(c, ccd::launch_permute_ranks(c->stage, c->H, c->csc.dperm, k, c->n, true, c->stream));
+    HIP_TRY(c, hipMemcpyAsync(c->fstage, W, sizeof(float) * nW, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, ccd::launch_permute_ranks(c->fstage, c->W, c->csr.dperm, k, c->m, true, c->stream));
+    HIP_TRY(c, hipMemcpyAsync(c->fstage, H, sizeof(float) * nH, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, ccd::launch_permute_ranks(c->fstage, c->H, c->csc.dperm, k, c->n, true, c->stream));
     if (c->nnz) {
         HIP_TRY(c, hipMemcpyAsync(c->csr.val, c->csr.val0, 4 * c->nnz, hipMemcpyDeviceToDevice, c->stream));
         HIP_TRY(c, hipMemcpyAsync(c->csc.val, c->csc.val0, 4 * c->nnz, hipMemcpyDeviceToDevice, c->stream));
@@ -910,7 +914,8 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
     }
     c->iter_rmse.assign(T, NAN);
     c->prof = p->profile != 0;
-    c->prof_kinds = (uint32_t)p->profile_kinds;
+    c->prof_kinds = (uint32_t)p->profile_kinds & ~(uint32_t)CCD_PROFILE_ITER;
+    c->prof_iter = (p->profile_kinds & CCD_PROFILE_ITER) != 0;
     c->recs.clear();
     c->pool_used = 0;
     for (int q = 0; q < CCD_K_COUNT; ++q) {
@@ -964,12 +969,6 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
     // previous one starts with a fused rank 0 whose pairs are built here.
     const bool sweeps = Tin >= 1 && k > 0;
     if (sweeps) {
-        for (DevLayout* L : {&F, &S}) {  // sized for FP32 pairs, so every precision fits
-            if (L->pair) continue;
-            double2* d = nullptr;
-            HIP_TRY(c, dalloc(&d, ((size_t)L->gdim + 1) / 2));
-            L->pair = d;
-        }
         if (c->continued) {
             ccd::CommitArgs ca{nullptr, nullptr, XS, XS, F.pair, (uint64_t)dS, nullptr, nullptr, XF, XF, S.pair, (uint64_t)dF};
             HIP_TRY(c, ccd::launch_commit(ca, bf, c->stream));
@@ -982,7 +981,9 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
     size_t rec_mark = 0;
     // One outer iteration's ranks.  build_last_pairs = false: the commit of
     // the run's last rank skips the pairs of a next rank that never comes.
+    GroupTimer groups{c};
     auto outer = [&](int oiter, bool build_last_pairs) -> int {
+        groups.begin();
         for (uint32_t t = 0; t < k; ++t) {
             const char* St = XS + (size_t)t * dS * es;
             const char* Ft = XF + (size_t)t * dF * es;
@@ -1001,6 +1002,7 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
                     rc1 = pass(c, S, vF, vS, nullptr, nullptr, nullptr, nullptr, false, false, false, true, lambda, CCD_K_SWEEP_S);
                     if (rc1) return rc1;
                 }
+                groups.end(CCD_K_SWEEP_F);
                 // W, H <- u, v; pairs of the next rank (none after the last)
                 const bool last = !build_last_pairs && oiter == T && t + 1 == k;
                 const uint32_t tn = t + 1 == k ? 0 : t + 1;
@@ -1008,13 +1010,17 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
                 char* XFt = XF + (size_t)t * dF * es;
                 ccd::CommitArgs ca{vS, XSt, nullptr, XS + (size_t)tn * dS * es, last ? nullptr : F.pair, (uint64_t)dS,
                                    vF, XFt, nullptr, XF + (size_t)tn * dF * es, last ? nullptr : S.pair, (uint64_t)dF};
-                Timed tm(c, CCD_K_COPY);
-                HIP_TRY(c, ccd::launch_commit(ca, bf, c->stream));
+                {
+                    Timed tm(c, CCD_K_COPY);
+                    HIP_TRY(c, ccd::launch_commit(ca, bf, c->stream));
+                }
+                groups.end(CCD_K_COPY);
             } else if (fused) {
                 int rc1 = pass(c, F, nullptr, nullptr, Sp, Fp, St, Ft, false, pending, add, false, lambda, CCD_K_RESIDUAL);
                 if (rc1) return rc1;
                 rc1 = pass(c, S, nullptr, nullptr, Fp, Sp, Ft, St, false, pending, add, false, lambda, CCD_K_RESIDUAL);
                 if (rc1) return rc1;
+                groups.end(CCD_K_RESIDUAL);
             }
             pending = true;
             prev = t;
@@ -1072,9 +1078,13 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
             if (rc) return rc;
         }
         if (do_rmse) {
-            Timed tm(c, CCD_K_RMSE);
-            HIP_TRY(c, ccd::launch_rmse(c->trow, c->tcol, c->tval, c->nnz_test, Wr, Hr, bf, c->m, c->n, k,
-                                        c->rmse_bsum, c->rmse_dev + (oiter - 1), c->stream));
+            groups.begin();
+            {
+                Timed tm(c, CCD_K_RMSE);
+                HIP_TRY(c, ccd::launch_rmse(c->trow, c->tcol, c->tval, c->nnz_test, Wr, Hr, bf, c->m, c->n, k,
+                                            c->rmse_bsum, c->rmse_dev + (oiter - 1), c->stream));
+            }
+            groups.end(CCD_K_RMSE);
         }
         if (cb) {
             HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -1118,7 +1128,7 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
     c->loop_s = 0.0;
     if (c->prof) {
         for (const ProfRec& r : c->recs) {
-            if (r.kind < 0) continue;  // a replayed outer iteration
+            if (r.kind < 0 || c->prof_iter) continue;  // a replayed outer iteration, or a group of launches
             float ms = 0.0f;
             HIP_TRY(c, hipEventElapsedTime(&ms, r.a, r.b));
             c->kind_ms[r.kind] += ms;
@@ -1138,13 +1148,12 @@ int32_t ccd_get_factors(ccd_ctx* c, float* W, float* H) {
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     const uint32_t k = c->k;
     const size_t nW = (size_t)k * c->m, nH = (size_t)k * c->n;
-    if (int rc = ensure_stage(c, std::max(nW, nH))) return rc;
     for (int q = 0; q < 2; ++q) {
         float* out = q == 0 ? W : H;
         if (!out) continue;
-        HIP_TRY(c, ccd::launch_permute_ranks(q == 0 ? c->W : c->H, c->stage, q == 0 ? c->csr.dperm : c->csc.dperm, k,
+        HIP_TRY(c, ccd::launch_permute_ranks(q == 0 ? c->W : c->H, c->fstage, q == 0 ? c->csr.dperm : c->csc.dperm, k,
                                              q == 0 ? c->m : c->n, false, c->stream));
-        HIP_TRY(c, ccd::copy_sync(c->stream, out, c->stage, sizeof(float) * (q == 0 ? nW : nH), hipMemcpyDeviceToHost));
+        HIP_TRY(c, ccd::copy_sync(c->stream, out, c->fstage, sizeof(float) * (q == 0 ? nW : nH), hipMemcpyDeviceToHost));
     }
     return CCD_OK;
 }

@@ -15,6 +15,7 @@ namespace ccdi {
 // index array is tiled once; residual values are tiled at the start of each
 // tiled run and written back to the layout's canonical order at its end.
 struct TiledLayout {
+    void* mem = nullptr;  // the one allocation behind the device arrays below
     int sigma = 0;
     int ib = 0;  // bytes per index of tidx: 2, 3 or 4 (ccd_kernels.h)
     uint32_t ntiles = 0;
@@ -40,6 +41,7 @@ struct TiledLayout {
     bool split = false;
     uint32_t nreal = 0;
     uint32_t cold_tile0 = 0xffffffffu;  // first tile holding only second parts (split layouts)
+    uint32_t* vptr = nullptr;      // row pointer of the virtual rows
     uint32_t* vpos = nullptr;      // position in the layout of each element, in tiled order
     uint32_t* cold_row = nullptr;  // real row of each second part
     ccd::SplitRow* srows = nullptr;  // per row: tile ranges of its two parts
@@ -47,6 +49,7 @@ struct TiledLayout {
 };
 
 struct DevLayout {
+    void* mem = nullptr;  // the one allocation behind the device arrays (but the tiled copy's)
     int64_t rows = 0;   // rows of this layout (n for CSC, m for CSR)
     int64_t gdim = 0;   // length of the gathered vector (m for CSC, n for CSR)
     uint64_t nnz = 0;
@@ -81,6 +84,7 @@ struct DevLayout {
     std::vector<uint32_t> below;
     std::vector<uint32_t> perm;      // internal row -> caller's row
     uint32_t* dperm = nullptr;       // the same on the device
+    uint32_t* dbelow = nullptr;      // `below` on the device
     TiledLayout tl;
 };
 
@@ -122,8 +126,9 @@ struct ccd_ctx {
     int lds_block = 0;         // LDS bytes a block may use
     int lds_cu = 0;            // LDS bytes of a CU
     std::map<uint32_t, int> occupancy;  // persistent kernel -> blocks per CU by register use
-    // grow-only staging of the caller's arrays on the device (factors and
-    // residual on their way between the two numberings)
+    void* fmem = nullptr;     // the one allocation behind W, H and fstage
+    float* fstage = nullptr;  // one factor matrix on its way between the two numberings
+    // grow-only staging of the residual on its way back
     float* stage = nullptr;
     size_t stage_cap = 0;
     double* rmse_bsum = nullptr;
@@ -134,6 +139,7 @@ struct ccd_ctx {
     ccd_plan_params plan{4, 8192, 4096, 4096, 16, 0, 1};
     // profiling
     bool prof = false;
+    bool prof_iter = false;    // CCD_PROFILE_ITER: only what the iteration callback reports
     uint32_t prof_kinds = 0;  // bitmask of timed kernel kinds (1 << ccd_kernel_kind)
     std::vector<ccdi::ProfRec> recs;
     std::vector<hipEvent_t> pool;
@@ -165,6 +171,34 @@ hipError_t dalloc(T** p, size_t count) {
     *p = nullptr;
     return hipMalloc(reinterpret_cast<void**>(p), sizeof(T) * (count ? count : 1));
 }
+
+// Several device arrays in one allocation (256-byte aligned): a context has
+// some sixty, and each hipMalloc and hipFree costs tens of microseconds.
+class Carver {
+public:
+    template <class T>
+    void add(T** p, size_t count) {
+        slots_.push_back({reinterpret_cast<void**>(p), total_});
+        total_ += (sizeof(T) * (count ? count : 1) + 255) & ~(size_t)255;
+    }
+    hipError_t alloc(void** base) {
+        const hipError_t e = hipMalloc(base, total_ ? total_ : 1);
+        if (e != hipSuccess) {
+            *base = nullptr;
+            return e;
+        }
+        for (const Slot& s : slots_) *s.p = static_cast<char*>(*base) + s.off;
+        return e;
+    }
+
+private:
+    struct Slot {
+        void** p;
+        size_t off;
+    };
+    std::vector<Slot> slots_;
+    size_t total_ = 0;
+};
 
 void dfree(void* p);
 // Context staging of at least `count` floats (ccd_ctx::stage).

@@ -499,8 +499,8 @@ struct ccd_fold {
     uint32_t k = 0;
     int64_t n = 0;
     float lambda = 0.0f;
-    float* HT = nullptr;  // [n + 1][fold_ld(k)], ccd::FoldArgs
-    float* H = nullptr;   // the caller's [k][n], transposed into HT (kept: freeing it would wait for the device)
+    float* HT = nullptr;  // [n + 1][fold_ld(k)], ccd::FoldArgs; H and bad lie behind it
+    float* H = nullptr;   // the caller's [k][n], transposed into HT
     uint32_t *ptr = nullptr, *idx = nullptr, *long_rows = nullptr;
     uint32_t* bad = nullptr;  // fold_check_device
     uint32_t nlong = 0, nfeat = 0;  // rows longer than FOLD_WAVE, and than FOLD_SHORT
@@ -608,11 +608,15 @@ int32_t ccd_fold_create(int32_t device, uint32_t k, int64_t n, const float* H, f
     const size_t kn = (size_t)k * n, nht = ((size_t)n + 1) * fold_ld(k);
     bool ok = hipSetDevice(device) == hipSuccess && hipStreamCreateWithFlags(&f->stream, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreate(&f->ea) == hipSuccess && hipEventCreate(&f->eb) == hipSuccess &&
-              dalloc(&f->H, kn) == hipSuccess && dalloc(&f->HT, nht) == hipSuccess && dalloc(&f->bad, 1) == hipSuccess &&
-              ccd::launch_fill(f->HT, 0.0f, nht, f->stream) == hipSuccess &&
-              ccd::copy_sync(f->stream, f->H, H, 4 * kn, hipMemcpyHostToDevice) == hipSuccess &&
-              ccd::launch_transpose(f->H, f->HT, k, (uint32_t)n, fold_ld(k), f->stream) == hipSuccess &&
-              hipStreamSynchronize(f->stream) == hipSuccess && scratch_on(device, &f->scratch) == hipSuccess;
+              dalloc(&f->HT, nht + kn + 1) == hipSuccess;
+    if (ok) {
+        f->H = f->HT + nht;
+        f->bad = reinterpret_cast<uint32_t*>(f->H + kn);
+    }
+    ok = ok && ccd::launch_fill(f->HT, 0.0f, nht, f->stream) == hipSuccess &&
+         ccd::copy_sync(f->stream, f->H, H, 4 * kn, hipMemcpyHostToDevice) == hipSuccess &&
+         ccd::launch_transpose(f->H, f->HT, k, (uint32_t)n, fold_ld(k), f->stream) == hipSuccess &&
+         hipStreamSynchronize(f->stream) == hipSuccess && scratch_on(device, &f->scratch) == hipSuccess;
     if (!ok) {
         ccd_fold_destroy(f);
         return CCD_ERR_HIP;
@@ -625,7 +629,7 @@ int32_t ccd_fold_destroy(ccd_fold* f) {
     if (!f) return CCD_OK;
     (void)hipSetDevice(f->device);
     if (f->stream) (void)hipStreamSynchronize(f->stream);
-    void* bufs[] = {f->H, f->HT, f->bad, f->ptr, f->idx, f->val, f->W0, f->W, f->F, f->long_rows};
+    void* bufs[] = {f->HT, f->ptr, f->idx, f->val, f->W0, f->W, f->F, f->long_rows};
     for (void* b : bufs) dfree(b);
     if (f->ea) (void)hipEventDestroy(f->ea);
     if (f->eb) (void)hipEventDestroy(f->eb);

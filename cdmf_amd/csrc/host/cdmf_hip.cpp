@@ -116,6 +116,7 @@ void cdmf_hip(SparseMatrix& R, MatData& W, MatData& H, TestData* T, parameter& p
     p.use_graph = CDMF_PARAM_GRAPH(param);
     p.rmse_every = T != nullptr;
     p.profile = 1;
+    p.profile_kinds = CCD_PROFILE_ITER;
     IterPrint pr{T != nullptr, param.verbose != 0};
 
     std::cout << "------------------------------------------------------" << std::endl;

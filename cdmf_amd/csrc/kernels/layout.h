@@ -45,4 +45,16 @@ hipError_t launch_renumber(const RenumArgs& a, bool idx16, const RenumRows& n, u
 // *bad |= 1 when an index is not below dim (*bad set by the caller)
 hipError_t launch_index_check(const uint32_t* idx, uint64_t count, uint32_t dim, uint32_t* bad, hipStream_t s);
 
+
+// Per-element tables of a tiled layout (tile_layout.h).  ptr: row pointer of
+// its (virtual) rows.
+// flags: zeroed here; per lane one u16 (sigma <= 16) or u32
+hipError_t launch_tile_flags(const uint32_t* ptr, uint64_t rows, uint64_t ntiles, int sigma, uint32_t* flags,
+                             hipStream_t s);
+// Position map of a split layout: vptr, its virtual row pointer (vrows + 1);
+// lptr and below, the layout's row pointer and per-row split counts;
+// cold_row, the real rows of virtual rows nreal, nreal + 1, ...
+hipError_t launch_split_positions(const uint32_t* vptr, uint64_t vrows, const uint32_t* lptr, const uint32_t* below,
+                                  const uint32_t* cold_row, uint32_t nreal, uint32_t* vpos, hipStream_t s);
+
 }  // namespace ccd

@@ -215,6 +215,39 @@ __global__ __launch_bounds__(BLOCK) void renum_dup_kernel(RenumArgs a, const uin
     }
 }
 
+// One thread per row: the bit of its first element in its lane's word.
+__global__ __launch_bounds__(BLOCK) void tile_flags_kernel(const uint32_t* __restrict__ ptr, uint64_t rows,
+                                                           uint32_t sigma, uint32_t* __restrict__ flags) {
+    const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
+    for (uint64_t r = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; r < rows; r += stride) {
+        const uint32_t e = ptr[r];
+        if (ptr[r + 1] == e) continue;
+        const uint32_t ln = e / sigma, bit = e % sigma;  // a tile is 64 whole lanes
+        if (sigma <= 16) atomicOr(flags + ln / 2, 1u << (16 * (ln & 1) + bit));
+        else atomicOr(flags + ln, 1u << bit);
+    }
+}
+
+// One block per virtual row (grid-stride): its elements' positions are consecutive in the
+// layout.
+__global__ __launch_bounds__(BLOCK) void split_positions_kernel(const uint32_t* __restrict__ vptr,
+                                                                const uint32_t* __restrict__ lptr,
+                                                                const uint32_t* __restrict__ below,
+                                                                const uint32_t* __restrict__ cold_row, uint32_t nreal,
+                                                                uint64_t vrows, uint32_t* __restrict__ vpos) {
+    for (uint64_t v = blockIdx.x; v < vrows; v += gridDim.x) {
+        const uint32_t v0 = vptr[v], len = vptr[v + 1] - v0;
+        uint32_t src;
+        if (v < nreal) {
+            src = lptr[v];
+        } else {
+            const uint32_t r = cold_row[v - nreal];
+            src = lptr[r] + below[r];
+        }
+        for (uint32_t q = threadIdx.x; q < len; q += BLOCK) vpos[v0 + q] = src + q;
+    }
+}
+
 uint32_t grid_for(uint64_t count) {
     return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((count + BLOCK - 1) / BLOCK, 1), 16384);
 }
@@ -276,6 +309,23 @@ static hipError_t renumber(const RenumArgs& a, const RenumRows& n, uint32_t* dup
 
 hipError_t launch_renumber(const RenumArgs& a, bool idx16, const RenumRows& n, uint32_t* dup, hipStream_t s) {
     return idx16 ? renumber<uint16_t>(a, n, dup, s) : renumber<uint32_t>(a, n, dup, s);
+}
+
+hipError_t launch_tile_flags(const uint32_t* ptr, uint64_t rows, uint64_t ntiles, int sigma, uint32_t* flags,
+                             hipStream_t s) {
+    if (ntiles == 0) return hipSuccess;
+    const hipError_t e = launch_fill(reinterpret_cast<float*>(flags), 0.0f, ntiles * (sigma <= 16 ? 32 : 64), s);
+    if (e != hipSuccess || rows == 0) return e;
+    hipLaunchKernelGGL(tile_flags_kernel, dim3(grid_for(rows)), dim3(BLOCK), 0, s, ptr, rows, (uint32_t)sigma, flags);
+    return hipGetLastError();
+}
+
+hipError_t launch_split_positions(const uint32_t* vptr, uint64_t vrows, const uint32_t* lptr, const uint32_t* below,
+                                  const uint32_t* cold_row, uint32_t nreal, uint32_t* vpos, hipStream_t s) {
+    if (vrows == 0) return hipSuccess;
+    hipLaunchKernelGGL(split_positions_kernel, dim3((uint32_t)std::min<uint64_t>(vrows, 1u << 20)), dim3(BLOCK), 0, s,
+                       vptr, lptr, below, cold_row, nreal, vrows, vpos);
+    return hipGetLastError();
 }
 
 }  // namespace ccd

@@ -1,5 +1,5 @@
 // Host-side tables of the tiled copy of a compressed layout (tile_layout.h).
-// O(rows + tiles) except the position map of a split layout (O(nnz)).
+// O(rows + tiles) but for the position map of a split layout (O(nnz)).
 #include "tile_layout.h"
 
 #include <algorithm>
@@ -7,7 +7,7 @@
 namespace ccd {
 
 std::string build_tile_tables(const uint32_t* hptr, int64_t nrows, uint64_t nnz, const uint32_t* below, int sigma,
-                              bool split, TileTables& T) {
+                              bool split, TileTables& T, bool elements) {
     T = TileTables{};
     if (sigma <= 0 || sigma > 32 || sigma % 8) return "sigma must be 8, 16, 24 or 32";
     if (split && !below) return "a split layout needs the per-row split counts";
@@ -43,19 +43,21 @@ std::string build_tile_tables(const uint32_t* hptr, int64_t nrows, uint64_t nnz,
                 vptr.push_back(vptr.back() + rest);
             }
         }
-        T.vpos.resize(nnz);
-        for (int64_t r = 0; r < nrows; ++r)
-            for (uint32_t q = 0; q < below[r]; ++q) T.vpos[vptr[r] + q] = hptr[r] + q;
-        for (size_t k = 0; k < T.cold_row.size(); ++k) {
-            const uint32_t r = T.cold_row[k], b = vptr[nrows + k];
-            for (uint32_t q = 0; q < vptr[nrows + k + 1] - b; ++q) T.vpos[b + q] = hptr[r] + below[r] + q;
+        if (elements) {
+            T.vpos.resize(nnz);
+            for (int64_t r = 0; r < nrows; ++r)
+                for (uint32_t q = 0; q < below[r]; ++q) T.vpos[vptr[r] + q] = hptr[r] + q;
+            for (size_t k = 0; k < T.cold_row.size(); ++k) {
+                const uint32_t r = T.cold_row[k], b = vptr[nrows + k];
+                for (uint32_t q = 0; q < vptr[nrows + k + 1] - b; ++q) T.vpos[b + q] = hptr[r] + below[r] + q;
+            }
         }
         T.nreal = (uint32_t)nrows;
         T.cold_tile0 = (uint32_t)((vptr[nrows] + TS - 1) / TS);
     }
     const uint32_t* ptr = split ? T.vptr.data() : hptr;
     const int64_t rows = split ? (int64_t)T.vptr.size() - 1 : nrows;
-    T.flags.assign(ntiles * 64, 0u);
+    if (elements) T.flags.assign(ntiles * 64, 0u);
     T.row0.assign(ntiles, 0u);
     T.segoff.assign(ntiles, 0u);
     T.open.assign((ntiles + 3) & ~(uint64_t)3, 0u);  // whole words: the kernels read it a word at a time
@@ -65,7 +67,7 @@ std::string build_tile_tables(const uint32_t* hptr, int64_t nrows, uint64_t nnz,
         emp[r + 1] = emp[r] + (empty ? 1u : 0u);
         if (empty) continue;
         const uint64_t e = ptr[r], rem = e % TS;
-        T.flags[(e / TS) * 64 + rem / sigma] |= 1u << (rem % sigma);
+        if (elements) T.flags[(e / TS) * 64 + rem / sigma] |= 1u << (rem % sigma);
         const uint64_t t0 = e / TS, t1 = (ptr[r + 1] - 1ull) / TS;
         if (t0 != t1) T.spans.push_back({(uint32_t)r, (uint32_t)t0, (uint32_t)t1, ptr[r + 1] - ptr[r]});
     }

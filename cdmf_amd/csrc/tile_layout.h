@@ -59,9 +59,10 @@ struct TileTables {
 // Tables for tiles of 64 * sigma elements of the layout with row pointer ptr
 // (rows + 1 entries, ptr[rows] = nnz).  split: keep each row's two parts
 // (below[r] leading elements, then the rest) as two virtual rows, all first
-// parts before all second parts.  Returns an empty string or the reason it
-// cannot be built.
+// parts before all second parts.  elements: fill the per-element tables too
+// (flags and vpos), which the library makes on the device instead.  Returns
+// an empty string or the reason it cannot be built.
 std::string build_tile_tables(const uint32_t* ptr, int64_t rows, uint64_t nnz, const uint32_t* below, int sigma,
-                              bool split, TileTables& T);
+                              bool split, TileTables& T, bool elements = true);
 
 }  // namespace ccd

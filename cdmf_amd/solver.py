@@ -49,6 +49,8 @@ class CBatchPlan(C.Structure):
                 ("deal", C.c_uint32)]
 
 
+PROFILE_ITER = 0x40000000  # CCD_PROFILE_ITER of include/cdmf_hip.h
+
 ITER_CB = C.CFUNCTYPE(None, C.c_void_p, C.c_int32, C.c_double, C.c_double, C.c_double, C.c_double)
 
 _hip = None
@@ -239,13 +241,13 @@ class Solver:
             rmse_every: bool = True, profile: bool = False, use_graph: bool = False,
             callback=None, profile_kinds=()) -> RunResult:
         """profile_kinds: names from KERNEL_KINDS to time when profile is set
-        (empty: every kind)."""
+        (empty: every kind; "iter": only the times the callback reports)."""
         p = CParams()
         self._lib.ccd_params_default(C.byref(p))
         p.k, p.lambda_, p.maxiter, p.maxinneriter = k, lam, outer, inner
         p.variant, p.precision, p.order = variant, precision, order
         p.zero_first, p.rmse_every, p.profile, p.use_graph = int(zero_first), int(rmse_every), int(profile), int(use_graph)
-        p.profile_kinds = sum(1 << KERNEL_KINDS.index(kk) for kk in set(profile_kinds))
+        p.profile_kinds = sum(PROFILE_ITER if kk == "iter" else 1 << KERNEL_KINDS.index(kk) for kk in set(profile_kinds))
         res = RunResult()
 
         def _cb(_user, oiter, rank_t, upd_t, rmse, rmse_t):
@@ -418,7 +420,8 @@ def cdmf_hip(R: Dataset, W: np.ndarray, H: np.ndarray, T: Dataset | None, param:
         res = s.run(param.k, param.lambda_, param.maxiter, param.maxinneriter,
                     variant=param.version if variant is None else variant, precision=param.precision,
                     order=param.order, zero_first=bool(param.zero_first), rmse_every=T is not None,
-                    profile=bool(param.profile), use_graph=bool(param.use_graph), callback=cb)
+                    profile=bool(param.profile), profile_kinds=("iter",), use_graph=bool(param.use_graph),
+                    callback=cb)
         Wn, Hn = s.factors()
         W[...] = Wn
         H[...] = Hn

@@ -85,9 +85,13 @@ typedef struct ccd_params {
                               nothing between kernels but about 5 us of device time per timed launch, so
                               with profile_kinds != 0 one launch in 5 of each selected sweep kind is timed
                               (the 1st, 6th, ...); the other kinds by event records around the launch,
-                              which add a few microseconds between kernels each. */
+                              which add a few microseconds between kernels each.
+                              CCD_PROFILE_ITER instead times what the iteration callback reports and
+                              ccd_loop_time only (two event records a rank; no ccd_kernel_stats). */
     int32_t reserved[4];  /* zero */
 } ccd_params;
+
+#define CCD_PROFILE_ITER 0x40000000
 
 /* Fills the reference defaults of src/pmf.h:4-26 (k=10, lambda=0.1, 5 outer,
  * 5 inner, variant 1, FP32, H first, zero_first 1, RMSE every iteration). */

@@ -138,3 +138,51 @@ def test_refused_upload_leaves_the_context():
                 s.upload(bad, with_test=False)
         a, b = s.residual()
         assert np.array_equal(a, ds.csr_val) and np.array_equal(b, ds.csc_val)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_larger_matrix_on_the_same_context(precision):
+    """A second upload of a larger matrix at the same k gives what a new
+    context gives (the factor buffers follow the new shape)."""
+    from cdmf_amd import data as D
+    from cdmf_amd import solver as S
+    k = 5
+    small, large = _dataset(60, 50, 900, seed=3), _dataset(3000, 2000, 40000, seed=4)
+
+    def solve(s, ds):
+        s.upload(ds, with_test=False)
+        s.set_factors(D.initial_col(k, ds.m), np.zeros((k, ds.n), np.float32))
+        s.run(k, 0.05, 2, 2, variant=S.VARIANT_TILED, precision=precision)
+        return s.factors()
+
+    with S.Solver(0) as s:
+        solve(s, small)
+        got = solve(s, large)
+    with S.Solver(0) as s:
+        want = solve(s, large)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+def test_iteration_times_without_kernel_times():
+    """profile_kinds "iter": the callback's times, none per kernel kind, and
+    the same factors as without profiling."""
+    from cdmf_amd import data as D
+    from cdmf_amd import solver as S
+    ds = _dataset(500, 300, 9000, seed=8)
+    k = 3
+    W0, H0 = D.initial_col(k, ds.m), np.zeros((k, ds.n), np.float32)
+    out = []
+    with S.Solver(0) as s:
+        s.upload(ds)
+        for kw in (dict(profile=True, profile_kinds=("iter",)), dict()):
+            recs = []
+            s.set_factors(W0, H0)
+            s.run(k, 0.05, 3, 2, variant=S.VARIANT_TILED, callback=recs.append, **kw)
+            out.append(s.factors())
+            assert len(recs) == 3
+            for r in recs:
+                assert (r.rank_time > 0 and r.update_time > 0 and r.rmse_time > 0) == bool(kw)
+            if kw:
+                assert s.loop_time() >= sum(r.rank_time + r.update_time + r.rmse_time for r in recs)
+                assert all(v["launches"] == 0 for v in s.kernel_stats().values())
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
