@@ -523,7 +523,13 @@ int do_tiled_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* 
     TiledLayout& T = L.tl;
     const bool fused = sweep && (sub || add);
     const Launch sh = launch_shape(c, true, T.sigma, T.ib, sub, add, sweep, fused && x_is_cur);
-    const Hot hot = hot_prefix(c, L, sh.lds_budget, fused, sweep, x_is_cur);
+    Hot hot = hot_prefix(c, L, sh.lds_budget, fused, sweep, x_is_cur);
+    // Few elements per block: staging the prefix (up to 160 KB, about 4 us)
+    // costs more than its gathers from L2.  40,000 x 5,000 with 1M ratings:
+    // 12.5 us a pass staged, 11.4 not; 147,910 x 3,297 with 4.5M: 19.0 and
+    // 19.6.  (2-byte factors: never faster unstaged, 12.4 and 12.5 us at 1M.)
+    const uint32_t nb = std::min(sh.blocks, std::max(T.ntiles, 1u));
+    if (sweep && factor_bytes(c) == 4 && (double)L.nnz < 0.3 * nb * ((double)hot.x + 2.0 * hot.p)) hot = {0, 0};
     // tiles of second parts gather from beyond the LDS prefix only when the
     // split is at or past it (a prefix staged with two blocks per CU, or in
     // bfloat16, differs from the one the layout was split at)

@@ -62,9 +62,31 @@ __device__ __forceinline__ T ld_const(const T* p, size_t i) {
 // Copy of n elements into LDS by a block of BLOCK threads.  Each thread
 // issues a round of up to U loads before its first LDS write, so a round
 // costs one memory round trip rather than one per element (the plain loop
-// waits for every load before its write).
+// waits for every load before its write).  2-byte entries go two at a time
+// (a factor row of odd length starts at an odd entry: dword loads need no
+// alignment here), else a prefix of 81,408 of them would take five rounds:
+// a bfloat16 sweep of 18.0M ratings took 46 us where FP32 took 33.
 template <int BLOCK, class T>
 __device__ __forceinline__ void stage_lds(T* __restrict__ dst, const T* __restrict__ src, uint32_t n) {
+    if constexpr (sizeof(T) == 2) {
+        struct __attribute__((packed, aligned(2))) Two {
+            uint32_t v;
+        };
+        const Two* src2 = reinterpret_cast<const Two*>(src);
+        uint32_t* dst2 = reinterpret_cast<uint32_t*>(dst);
+        constexpr int U = 16;
+        for (uint32_t base = threadIdx.x; base < n / 2; base += U * BLOCK) {
+            uint32_t v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (base + u * BLOCK < n / 2) v[u] = src2[base + u * BLOCK].v;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (base + u * BLOCK < n / 2) dst2[base + u * BLOCK] = v[u];
+        }
+        if (threadIdx.x == 0 && n % 2) dst[n - 1] = src[n - 1];
+        return;
+    }
     constexpr int U = sizeof(T) >= 16 ? 4 : sizeof(T) >= 8 ? 8 : 16;
     for (uint32_t base = threadIdx.x; base < n; base += U * BLOCK) {
         T v[U];

@@ -297,9 +297,12 @@ hipError_t launch_tiled(const TiledArgs& a, int sigma, int prec, int ib, bool su
     const TiledFn fn = tiled_fn(sigma, prec, ib, sub, add, sweep, a.x_is_cur != 0);
     if (!fn) return hipErrorInvalidValue;
     const int bs = tile_block(sigma);
-    const uint32_t need = (a.ntiles + bs / WAVE - 1) / (bs / WAVE);
-    if (need == 0) return record_unlaunched(ev, s);
-    if (blocks > need) blocks = need;
+    if (a.ntiles == 0) return record_unlaunched(ev, s);
+    // a block per tile while there are few: 16 tiles on one CU take four
+    // times the instruction issue of one (2,000 x 1,000 with 45,000 ratings:
+    // 11.3 -> 10.1 us a pass with its finish; 8,000 x 2,000 with 200,000:
+    // 11.5 -> 9.8)
+    if (blocks > a.ntiles) blocks = a.ntiles;
     TiledArgs arg = a;
     void* args[] = {&arg};
     return hipExtLaunchKernel(reinterpret_cast<const void*>(fn), dim3(blocks), dim3(bs), args,
