@@ -35,6 +35,10 @@ struct ccd_batch {
     uint32_t* d_tickets = nullptr;  // 8 x 16 words
     int* d_status = nullptr;
     size_t cap_probs = 0, cap_blocks = 0;
+    // rotating buffers of the problems in `active`, and those to clear
+    void* d_rot = nullptr;
+    size_t cap_rot = 0;
+    std::vector<std::pair<float*, uint64_t>> rot;
     // captured run
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -208,8 +212,6 @@ int describe(ccd_batch* b, int sigma, uint32_t blocks, const Split& sp, bool tri
             L->stage = L->nnz / std::max(nb[i], 1u) >= 2ull * std::min<uint64_t>(L->gdim, b->lds_floats) ? 1u : 0u;
         P.XF = hfirst ? c->H : c->W;
         P.XS = hfirst ? c->W : c->H;
-        P.vF = hfirst ? c->v : c->u;
-        P.vS = hfirst ? c->u : c->v;
         P.k = it.p.k;
         P.T = trial ? 0u : (uint32_t)it.p.maxiter;
         P.Tin = (uint32_t)it.p.maxinneriter;
@@ -225,13 +227,52 @@ int describe(ccd_batch* b, int sigma, uint32_t blocks, const Split& sp, bool tri
             owner[sp.first[i] + v] = (uint32_t)i;
         }
     }
+    // rotating buffers of every problem (BatchProblem::nbuf), one allocation
+    {
+        using P2 = float2;  // (g, h)
+        std::vector<float*> vf(np), vs(np);
+        std::vector<P2*> parts(4 * np);
+        ccdi::Carver mem;
+        for (size_t i = 0; i < np; ++i) {
+            ccd::BatchProblem& P = probs[i];
+            const ccd_batch::Item& it = b->items[b->active[i]];
+            P.nbuf = std::max(1u, std::min((uint32_t)it.p.maxinneriter, ccd::BATCH_BUFS));
+            mem.add(&vf[i], P.nbuf * ccd::batch_stride(P.F.rows));
+            mem.add(&vs[i], P.nbuf * ccd::batch_stride(P.S.rows));
+            mem.add(&parts[4 * i], P.nbuf * ccd::batch_stride(P.F.ntiles));
+            mem.add(&parts[4 * i + 1], P.nbuf * ccd::batch_stride(P.F.ntiles));
+            mem.add(&parts[4 * i + 2], P.nbuf * ccd::batch_stride(P.S.ntiles));
+            mem.add(&parts[4 * i + 3], P.nbuf * ccd::batch_stride(P.S.ntiles));
+        }
+        if (mem.bytes() > b->cap_rot) {
+            ccdi::dfree(b->d_rot);
+            b->d_rot = nullptr;
+            b->cap_rot = 0;
+            BATCH_TRY(b, mem.alloc(&b->d_rot));
+            b->cap_rot = mem.bytes();
+        } else {
+            mem.place(b->d_rot);
+        }
+        b->rot.clear();
+        for (size_t i = 0; i < np; ++i) {
+            ccd::BatchProblem& P = probs[i];
+            P.vF = vf[i];
+            P.vS = vs[i];
+            P.F.head = parts[4 * i];
+            P.F.tail = parts[4 * i + 1];
+            P.S.head = parts[4 * i + 2];
+            P.S.tail = parts[4 * i + 3];
+            b->rot.push_back({P.vF, P.nbuf * ccd::batch_stride(P.F.rows)});
+            b->rot.push_back({P.vS, P.nbuf * ccd::batch_stride(P.S.rows)});
+        }
+    }
     if (np > b->cap_probs) {
         ccdi::dfree(b->d_probs);
         ccdi::dfree(b->d_barriers);
         b->d_probs = nullptr;
         b->d_barriers = nullptr;
         BATCH_TRY(b, ccdi::dalloc(&b->d_probs, np));
-        BATCH_TRY(b, ccdi::dalloc(&b->d_barriers, np));
+        BATCH_TRY(b, ccdi::dalloc(&b->d_barriers, np * ccd::BATCH_BARRIER_STRIDE));
         b->cap_probs = np;
     }
     if (blocks > b->cap_blocks) {
@@ -260,7 +301,7 @@ int describe(ccd_batch* b, int sigma, uint32_t blocks, const Split& sp, bool tri
 // kernel, per-problem tear-down.  Graph-safe (fill kernels, no memsets).
 int enqueue_run(ccd_batch* b, int sigma, const ccd::BatchArgs& a, bool trial) {
     hipStream_t s = b->stream;
-    BATCH_TRY(b, ccd::launch_fill(reinterpret_cast<float*>(b->d_barriers), 0.0f, a.nprob, s));
+    BATCH_TRY(b, ccd::launch_fill(reinterpret_cast<float*>(b->d_barriers), 0.0f, a.nprob * ccd::BATCH_BARRIER_STRIDE, s));
     BATCH_TRY(b, ccd::launch_fill(reinterpret_cast<float*>(b->d_status), 0.0f, 1, s));
     BATCH_TRY(b, ccd::launch_fill(reinterpret_cast<float*>(b->d_tickets), 0.0f, 8 * 16, s));
     for (size_t i : b->active) {
@@ -273,9 +314,9 @@ int enqueue_run(ccd_batch* b, int sigma, const ccd::BatchArgs& a, bool trial) {
             BATCH_TRY(b, ccd::launch_fill(hfirst ? c->H : c->W, 0.0f, (uint64_t)it.p.k * F.rows, s));
         if (F.tl.ntiles) BATCH_TRY(b, ccd::launch_retile_f32(F.val, F.tl.tval, F.nnz, F.tl.ntiles, sigma, true, s));
         if (S.tl.ntiles) BATCH_TRY(b, ccd::launch_retile_f32(S.val, S.tl.tval, S.nnz, S.tl.ntiles, sigma, true, s));
-        BATCH_TRY(b, ccd::launch_fill(hfirst ? c->v : c->u, 0.0f, (uint64_t)F.rows, s));
-        BATCH_TRY(b, ccd::launch_fill(hfirst ? c->u : c->v, 0.0f, (uint64_t)S.rows, s));
     }
+    // rows without entries keep y = 0 in every buffer
+    for (const auto& r : b->rot) BATCH_TRY(b, ccd::launch_fill(r.first, 0.0f, r.second, s));
     BATCH_TRY(b, ccd::launch_batch(a, sigma, s));
     if (!trial) {
         for (size_t i : b->active) {
@@ -378,6 +419,7 @@ int32_t ccd_batch_destroy(ccd_batch* b) {
     ccdi::dfree(b->d_probs);
     ccdi::dfree(b->d_block_problem);
     ccdi::dfree(b->d_barriers);
+    ccdi::dfree(b->d_rot);
     ccdi::dfree(b->d_status);
     ccdi::dfree(b->d_tickets);
     if (b->ev_a) (void)hipEventDestroy(b->ev_a);
@@ -620,14 +662,15 @@ int32_t ccd_batch_run(ccd_batch* b, int32_t use_graph) {
     // it was captured with: a context's generation moves whenever it
     // reallocates any of them (upload, a new k, a rebuilt tile layout), and
     // the addresses the capture bakes in are keyed as well
-    std::vector<uint64_t> key{(uint64_t)sigma, blocks, (uint64_t)b->active.size(), deal_min(b->plan.deal)};
+    std::vector<uint64_t> key{(uint64_t)sigma, blocks, (uint64_t)b->active.size(), deal_min(b->plan.deal),
+                              (uint64_t)(uintptr_t)b->d_rot};
     for (size_t i : b->active) {
         const ccd_batch::Item& it = b->items[i];
         const ccd_ctx* c = it.ctx;
         key.push_back(i);
         key.push_back((it.ctx->continued ? 1u : 0u) | (it.p.zero_first ? 2u : 0u));
         key.push_back(c->gen);
-        for (const void* q : {(const void*)c->W, (const void*)c->H, (const void*)c->u, (const void*)c->v,
+        for (const void* q : {(const void*)c->W, (const void*)c->H,
                               (const void*)c->csr.val, (const void*)c->csc.val, (const void*)c->csr.tl.tval,
                               (const void*)c->csc.tl.tval, (const void*)c->csr.pair, (const void*)c->csc.pair})
             key.push_back((uint64_t)(uintptr_t)q);

@@ -187,9 +187,14 @@ public:
             *base = nullptr;
             return e;
         }
-        for (const Slot& s : slots_) *s.p = static_cast<char*>(*base) + s.off;
+        place(*base);
         return e;
     }
+    // the arrays in an allocation of at least bytes()
+    void place(void* base) const {
+        for (const Slot& s : slots_) *s.p = static_cast<char*>(base) + s.off;
+    }
+    size_t bytes() const { return total_; }
 
 private:
     struct Slot {

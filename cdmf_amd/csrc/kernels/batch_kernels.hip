@@ -39,12 +39,19 @@ struct Team {
 
 // Barrier of the blocks of one team; all of a team's blocks run on one XCD
 // and share its L2.  Release: every wave waits until its stores are
-// acknowledged (s_waitcnt vmcnt(0)), then one arrival per block is counted
-// with an L2 atomic.  Acquire: after the count is complete, an agent-scope
-// acquire fence drops the CU's stale cached copies, so the loads that follow
-// see the other blocks' data.  (No L2 write-back is needed inside one XCD;
-// an agent-scope release fence, which does one, costs 30-40 us a barrier.)
+// acknowledged by L2 (s_waitcnt vmcnt(0)); then one arrival per block is
+// counted with an L2 atomic, and read with L2 atomics until it is complete
+// (workgroup scope: nothing wider leaves the L2 that the whole team shares).
+// What the caller reads next is then in L2.  It may not be in the CU's L1,
+// which still holds lines read before: FRESH says that every address the
+// team exchanged has not been read since the last barrier without it
+// (BatchProblem's rotating buffers), so nothing needs to be dropped.
+// Otherwise an agent-scope acquire drops the cached copies; it drops the
+// XCD's L2 copies of every team as well, so it is kept to one per rank.
+// (Agent-scope counting and that acquire at every barrier: 6-10 us a barrier,
+// 23 us a pass of 200,000 ratings on 49 blocks; now 14 us.)
 // false: the wait ran out (status set); the caller returns.
+template <bool FRESH>
 __device__ __forceinline__ bool team_sync(Team& t) {
     __shared__ int s_ok;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -54,9 +61,11 @@ __device__ __forceinline__ bool team_sync(Team& t) {
     t.target += t.nb;
     if (threadIdx.x == 0) {
         int ok = 1;
-        __hip_atomic_fetch_add(t.cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint32_t zero = 0;  // unknown to the compiler, so that the read stays an atomic performed in L2
+        asm volatile("" : "+v"(zero));
+        __hip_atomic_fetch_add(t.cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         const long long t0 = wall_clock64();
-        while (__hip_atomic_load(t.cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < t.target) {
+        while (__hip_atomic_fetch_add(t.cnt, zero, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < t.target) {
             __builtin_amdgcn_s_sleep(1);
             if ((uint64_t)(wall_clock64() - t0) > t.wait_ticks) {
                 __hip_atomic_store(t.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -64,7 +73,7 @@ __device__ __forceinline__ bool team_sync(Team& t) {
                 break;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if constexpr (!FRESH) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         s_ok = ok;
     }
     __syncthreads();
@@ -83,7 +92,8 @@ struct PassVecs {
     float lambda;
 };
 
-__device__ __forceinline__ TiledArgs layout_args(const BatchLayout& L, const PassVecs& v) {
+// buf: which of the rotating partial arrays the pass leaves its tiles' sums in
+__device__ __forceinline__ TiledArgs layout_args(const BatchLayout& L, const PassVecs& v, uint32_t buf) {
     TiledArgs a;
     a.ptr = L.ptr;
     a.tidx = L.tidx;
@@ -106,8 +116,8 @@ __device__ __forceinline__ TiledArgs layout_args(const BatchLayout& L, const Pas
     a.cold_tile0 = 0xffffffffu;
     a.spread_tile0 = 0xffffffffu;
     a.part = nullptr;
-    a.head = L.head;
-    a.tail = L.tail;
+    a.head = static_cast<tiled::Pair<float>*>(L.head) + (size_t)buf * batch_stride(L.ntiles);
+    a.tail = static_cast<tiled::Pair<float>*>(L.tail) + (size_t)buf * batch_stride(L.ntiles);
     a.nnz = L.nnz;
     a.ntiles = L.ntiles;
     a.hot_x = 0;  // set per pass by the caller (LDS staging)
@@ -165,9 +175,9 @@ __device__ __forceinline__ void tile_loop(const TiledArgs& a, const float* lds, 
 }
 
 template <int SIGMA, bool SUB, bool ADD, bool SWEEP, bool XCUR>
-__device__ __forceinline__ void tiles_t(const BatchLayout* Lp, PassVecs v, const Staged& st, const Deal& d) {
+__device__ __forceinline__ void tiles_t(const BatchLayout* Lp, PassVecs v, uint32_t buf, const Staged& st, const Deal& d) {
     const BatchLayout& L = *Lp;
-    TiledArgs a = layout_args(L, v);
+    TiledArgs a = layout_args(L, v, buf);
     a.hot_x = st.hot_x;
     a.hot_p = st.hot_p;
     if (L.ib == 2) tile_loop<uint16_t, SIGMA, SUB, ADD, SWEEP, XCUR>(a, st.lds, st.ldsp, d);
@@ -182,17 +192,17 @@ __device__ __forceinline__ void tiles_t(const BatchLayout* Lp, PassVecs v, const
 // as the fused add-only pass of the single-problem path, which is left out
 // here because it makes the compiler spill the whole kernel.)
 template <int SIGMA>
-__device__ __forceinline__ void tiles(const BatchLayout* L, const PassVecs& v, const Staged& st, bool sub, bool add,
-                                      bool sweep, const Deal& d) {
+__device__ __forceinline__ void tiles(const BatchLayout* L, const PassVecs& v, uint32_t buf, const Staged& st, bool sub,
+                                      bool add, bool sweep, const Deal& d) {
     const int code = (sub ? 4 : 0) | (add ? 2 : 0) | (sweep ? 1 : 0) | (sweep && (sub || add) && v.xcur ? 8 : 0);
     switch (code) {
-        case 1: tiles_t<SIGMA, false, false, true, false>(L, v, st, d); break;
-        case 2: tiles_t<SIGMA, false, true, false, false>(L, v, st, d); break;
-        case 4: tiles_t<SIGMA, true, false, false, false>(L, v, st, d); break;
-        case 5: tiles_t<SIGMA, true, false, true, false>(L, v, st, d); break;
-        case 7: tiles_t<SIGMA, true, true, true, false>(L, v, st, d); break;
-        case 8 + 5: tiles_t<SIGMA, true, false, true, true>(L, v, st, d); break;
-        case 8 + 7: tiles_t<SIGMA, true, true, true, true>(L, v, st, d); break;
+        case 1: tiles_t<SIGMA, false, false, true, false>(L, v, buf, st, d); break;
+        case 2: tiles_t<SIGMA, false, true, false, false>(L, v, buf, st, d); break;
+        case 4: tiles_t<SIGMA, true, false, false, false>(L, v, buf, st, d); break;
+        case 5: tiles_t<SIGMA, true, false, true, false>(L, v, buf, st, d); break;
+        case 7: tiles_t<SIGMA, true, true, true, false>(L, v, buf, st, d); break;
+        case 8 + 5: tiles_t<SIGMA, true, false, true, true>(L, v, buf, st, d); break;
+        case 8 + 7: tiles_t<SIGMA, true, true, true, true>(L, v, buf, st, d); break;
         default: break;  // not produced by the loop below
     }
 }
@@ -246,7 +256,7 @@ __global__ __launch_bounds__(BATCH_BLOCK) void batch_kernel(BatchArgs ba) {
     if (p >= ba.nprob) return;
     const BatchProblem& P = ba.probs[p];
     const uint32_t rank = v - P.first;
-    Team tm{ba.barriers + p, P.nblocks, 0u, ba.status, ba.wait_ticks};
+    Team tm{ba.barriers + BATCH_BARRIER_STRIDE * p, P.nblocks, 0u, ba.status, ba.wait_ticks};
     const int lane = threadIdx.x & (WAVE - 1);
     const uint32_t w = rank * WPB + threadIdx.x / WAVE, nw = P.nblocks * WPB;
     const uint32_t tid = rank * BATCH_BLOCK + threadIdx.x, nth = P.nblocks * BATCH_BLOCK;
@@ -258,34 +268,48 @@ __global__ __launch_bounds__(BATCH_BLOCK) void batch_kernel(BatchArgs ba) {
     __shared__ uint32_t s_pos;  // the block's next tile position in a dealt sweep
     const Deal fixed{w, nw, 0u, 0u, nullptr, false};
 
+    // Inner iteration `it` of a rank uses buffers it % nbuf of the swept
+    // vectors and of the tile partials, so that every address exchanged at
+    // its barriers is one no CU has read since the last commit's acquire;
+    // where the buffers come round again (more inner iterations than
+    // buffers), the first barrier of a pass acquires too.
+    const uint32_t nbuf = P.nbuf;
+    auto buf_of = [&](uint32_t it) { return it % nbuf; };
+    auto vF = [&](uint32_t it) { return P.vF + (size_t)buf_of(it) * batch_stride(dF); };
+    auto vS = [&](uint32_t it) { return P.vS + (size_t)buf_of(it) * batch_stride(dS); };
+
     // one sweep (or fused) pass: LDS staging, tiles, barrier, rows spanning
     // tiles, barrier
-    auto pass = [&](const BatchLayout& L, const PassVecs& pv, bool sub, bool add) -> bool {
+    auto pass = [&](const BatchLayout& L, const PassVecs& pv, uint32_t it, bool sub, bool add) -> bool {
         __syncthreads();  // every wave of the block is done with the LDS of the last pass
         const bool dyn = (uint64_t)L.ntiles >= (uint64_t)ba.deal_min * nw;
         if (dyn && threadIdx.x == 0) s_pos = WPB;
         const Staged st = stage_pass(L, pv, sub || add, batch_lds, ba.lds_floats);
         if (dyn) __syncthreads();  // s_pos seen by every wave
-        tiles<SIGMA>(&L, pv, st, sub, add, true, Deal{w, nw, rank, P.nblocks, &s_pos, dyn});
-        if (!team_sync(tm)) return false;
+        const uint32_t buf = buf_of(it);
+        tiles<SIGMA>(&L, pv, buf, st, sub, add, true, Deal{w, nw, rank, P.nblocks, &s_pos, dyn});
+        if (!(it >= nbuf && buf == 0 ? team_sync<false>(tm) : team_sync<true>(tm))) return false;
         if (L.nspan) {
-            const SpanArgs sa{L.spans, L.head, L.tail, pv.y, L.nspan, L.nshort, lambda};
+            const size_t po = (size_t)buf * batch_stride(L.ntiles);
+            const SpanArgs sa{L.spans, static_cast<const tiled::Pair<float>*>(L.head) + po,
+                              static_cast<const tiled::Pair<float>*>(L.tail) + po,
+                              pv.y, L.nspan, L.nshort, lambda};
             for (uint32_t i = tid; i < L.nshort; i += nth) tiled::span_short<float, float>(sa, i);
             for (uint32_t i = L.nshort + w; i < L.nspan; i += nw) tiled::span_row<float, float>(sa, i, lane);
-            if (!team_sync(tm)) return false;
+            if (!team_sync<true>(tm)) return false;
         }
         return true;
     };
     auto commit = [&](const CommitArgs& ca) -> bool {
         for (uint64_t e = tid; e < ca.nS + ca.nF; e += nth) commit_elem<float>(ca, e);
-        return team_sync(tm);
+        return team_sync<false>(tm);
     };
     auto plain = [&](const float* x, float* y) { return PassVecs{x, y, nullptr, nullptr, nullptr, nullptr, 0u, lambda}; };
 
     if (ba.trial) {  // autotuner: plain sweeps of rank 0; no state changes but vF, vS
         for (uint32_t it = 0; it < P.trial_reps; ++it) {
-            if (!pass(P.F, plain(P.XS, P.vF), false, false)) return;
-            if (!pass(P.S, plain(P.vF, P.vS), false, false)) return;
+            if (!pass(P.F, plain(P.XS, vF(it)), it, false, false)) return;
+            if (!pass(P.S, plain(vF(it), vS(it)), it, false, false)) return;
         }
         return;
     }
@@ -300,28 +324,28 @@ __global__ __launch_bounds__(BATCH_BLOCK) void batch_kernel(BatchArgs ba) {
             const float* Fp = P.XF + (size_t)prev * dF;
             const bool add = oiter > 1 || P.continued;
             if (add && !pending) {  // rank 0 of a continued run: add back, then plain sweeps
-                tiles<SIGMA>(&P.F, PassVecs{nullptr, nullptr, nullptr, nullptr, St, Ft, 0u, lambda}, none, false, true,
-                             false, fixed);
-                tiles<SIGMA>(&P.S, PassVecs{nullptr, nullptr, nullptr, nullptr, Ft, St, 0u, lambda}, none, false, true,
-                             false, fixed);
+                tiles<SIGMA>(&P.F, PassVecs{nullptr, nullptr, nullptr, nullptr, St, Ft, 0u, lambda}, 0u, none, false,
+                             true, false, fixed);
+                tiles<SIGMA>(&P.S, PassVecs{nullptr, nullptr, nullptr, nullptr, Ft, St, 0u, lambda}, 0u, none, false,
+                             true, false, fixed);
                 // a dealt sweep may give a tile to another wave than the
                 // add-back did
-                if (!team_sync(tm)) return;
-                if (!pass(P.F, plain(St, P.vF), false, false)) return;
-                if (!pass(P.S, plain(P.vF, P.vS), false, false)) return;
+                if (!team_sync<false>(tm)) return;
+                if (!pass(P.F, plain(St, vF(0)), 0, false, false)) return;
+                if (!pass(P.S, plain(vF(0), vS(0)), 0, false, false)) return;
             } else {
-                if (!pass(P.F, PassVecs{St, P.vF, Sp, Fp, St, Ft, 1u, lambda}, pending, add)) return;
-                if (!pass(P.S, PassVecs{P.vF, P.vS, Fp, Sp, Ft, St, 0u, lambda}, pending, add)) return;
+                if (!pass(P.F, PassVecs{St, vF(0), Sp, Fp, St, Ft, 1u, lambda}, 0, pending, add)) return;
+                if (!pass(P.S, PassVecs{vF(0), vS(0), Fp, Sp, Ft, St, 0u, lambda}, 0, pending, add)) return;
             }
-            for (uint32_t it = 2; it <= P.Tin; ++it) {
-                if (!pass(P.F, plain(P.vS, P.vF), false, false)) return;
-                if (!pass(P.S, plain(P.vF, P.vS), false, false)) return;
+            for (uint32_t it = 1; it < P.Tin; ++it) {
+                if (!pass(P.F, plain(vS(it - 1), vF(it)), it, false, false)) return;
+                if (!pass(P.S, plain(vF(it), vS(it)), it, false, false)) return;
             }
             const bool last = oiter == P.T && t + 1 == P.k;
             const uint32_t tn = t + 1 == P.k ? 0u : t + 1;
-            const CommitArgs ca{P.vS, P.XS + (size_t)t * dS, nullptr, P.XS + (size_t)tn * dS,
+            const CommitArgs ca{vS(P.Tin - 1), P.XS + (size_t)t * dS, nullptr, P.XS + (size_t)tn * dS,
                                 last ? nullptr : P.F.pair, dS,
-                                P.vF, P.XF + (size_t)t * dF, nullptr, P.XF + (size_t)tn * dF,
+                                vF(P.Tin - 1), P.XF + (size_t)t * dF, nullptr, P.XF + (size_t)tn * dF,
                                 last ? nullptr : P.S.pair, dF};
             if (!commit(ca)) return;
             pending = true;
@@ -331,10 +355,10 @@ __global__ __launch_bounds__(BATCH_BLOCK) void batch_kernel(BatchArgs ba) {
     if (pending) {  // rank prev's final subtraction; the two layouts are independent
         const float* Sp = P.XS + (size_t)prev * dS;
         const float* Fp = P.XF + (size_t)prev * dF;
-        tiles<SIGMA>(&P.F, PassVecs{nullptr, nullptr, Sp, Fp, nullptr, nullptr, 0u, lambda}, none, true, false, false,
-                     fixed);
-        tiles<SIGMA>(&P.S, PassVecs{nullptr, nullptr, Fp, Sp, nullptr, nullptr, 0u, lambda}, none, true, false, false,
-                     fixed);
+        tiles<SIGMA>(&P.F, PassVecs{nullptr, nullptr, Sp, Fp, nullptr, nullptr, 0u, lambda}, 0u, none, true, false,
+                     false, fixed);
+        tiles<SIGMA>(&P.S, PassVecs{nullptr, nullptr, Fp, Sp, nullptr, nullptr, 0u, lambda}, 0u, none, true, false,
+                     false, fixed);
     }
 }
 

@@ -436,6 +436,11 @@ hipError_t launch_fill_bytes16(uint16_t* dst, uint16_t value, uint64_t count, hi
 // device, and every barrier wait is bounded in time: a wait that runs out
 // sets *status and the team leaves the kernel.
 constexpr int BATCH_BLOCK = 256;
+constexpr uint32_t BATCH_BARRIER_STRIDE = 32;  // words: a 128-byte line each, so no two XCDs share one
+constexpr uint32_t BATCH_BUFS = 8;             // most rotating buffers (BatchProblem::nbuf)
+// Entries from one rotating buffer to the next: whole 256-byte lines, so
+// that reading one buffer's end caches nothing of the next.
+__host__ __device__ constexpr uint64_t batch_stride(uint64_t entries) { return (entries + 63) & ~(uint64_t)63; }
 
 struct BatchLayout {  // one tiled layout of one problem (see TiledArgs)
     const uint32_t* ptr;
@@ -446,7 +451,7 @@ struct BatchLayout {  // one tiled layout of one problem (see TiledArgs)
     const uint32_t* tile_segoff;
     const uint32_t* segrows;
     const uint8_t* tile_open;
-    void* head;
+    void* head;  // (g, h) per tile, nbuf arrays, batch_stride apart
     void* tail;
     const SpanRow* spans;
     void* pair;  // FPair<float>[gathered length]
@@ -464,9 +469,10 @@ struct BatchProblem {
     BatchLayout F, S;  // first- and second-swept layouts
     float* XF;         // [k][F.rows] factor produced by the F sweeps
     float* XS;         // [k][S.rows]
-    float* vF;         // work vectors
+    float* vF;         // work vectors, nbuf of them, batch_stride apart
     float* vS;
     uint32_t k, T, Tin;
+    uint32_t nbuf;     // rotating buffers of vF, vS and the layouts' head and tail
     uint32_t continued;  // residual already holds R - W H^T: add back from the first rank on
     uint32_t first, nblocks;  // team: virtual block ids [first, first + nblocks)
     uint32_t trial_reps;      // autotuner trial: plain sweep pairs of rank 0 to run
@@ -478,7 +484,7 @@ struct BatchArgs {
     const uint32_t* block_problem;  // virtual block id -> problem (0xffffffff: idle)
     uint32_t nprob;
     uint32_t nblocks;               // grid size (a multiple of 8)
-    uint32_t* barriers;             // one counter per problem, zero at launch
+    uint32_t* barriers;             // one counter per problem, BATCH_BARRIER_STRIDE apart, zero at launch
     uint32_t* xcd_tickets;          // 8 counters, 64 bytes apart, zero at launch
     int* status;                    // 0; 1 after a barrier wait ran out
     uint64_t wait_ticks;            // bound of one barrier wait in wall_clock64() ticks
