@@ -421,7 +421,7 @@ int upload_layout(ccd_ctx* c, DevLayout& L, int64_t rows, int64_t gdim, uint64_t
     if (nnz) {
         // the caller's values pass through L.val
         HIP_TRY(c, to_device(tmp.ptr, cptr, sizeof(uint32_t) * (rows + 1)));
-        HIP_TRY(c, to_device(L.val, val, sizeof(float) * nnz));
+        HIP_TRY(c, c->pipe.in(c->device, L.val, val, sizeof(float) * nnz, c->stream));
         const ccd::RenumArgs ra{tmp.ptr, didx, L.val, L.dperm, ipos, L.ptr, L.idx, L.val0, L.src, (uint32_t)gdim};
         HIP_TRY(c, ccd::launch_renumber(ra, L.idx16, cls, tmp.dup, c->stream));
         HIP_TRY(c, hipMemcpyAsync(L.val, L.val0, sizeof(float) * nnz, hipMemcpyDeviceToDevice, c->stream));
@@ -593,7 +593,7 @@ int upload_indices(ccd_ctx* c, const UploadScratch& tmp, uint32_t* d, const uint
     *out_of_range = false;
     if (nnz == 0) return CCD_OK;
     uint32_t bad = 0;
-    HIP_TRY(c, hipMemcpyAsync(d, idx, sizeof(uint32_t) * nnz, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, c->pipe.in(c->device, d, idx, sizeof(uint32_t) * nnz, c->stream));
     HIP_TRY(c, ccd::launch_fill(reinterpret_cast<float*>(tmp.bad), 0.0f, 1, c->stream));
     HIP_TRY(c, ccd::launch_index_check(d, nnz, (uint32_t)dim, tmp.bad, c->stream));
     HIP_TRY(c, ccd::copy_sync(c->stream, &bad, tmp.bad, sizeof(bad), hipMemcpyDeviceToHost));
@@ -684,6 +684,7 @@ int32_t ccd_destroy(ccd_ctx* c) {
     dfree(c->rmse_dev);
     dfree(c->obj_dev);
     drop_graph(c);
+    c->pipe.release();
     for (hipEvent_t e : c->pool) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -843,9 +844,9 @@ int32_t ccd_set_factors(ccd_ctx* c, uint32_t k, const float* W, const float* H) 
         c->k = k;
     }
     const size_t nW = (size_t)k * c->m, nH = (size_t)k * c->n;
-    HIP_TRY(c, hipMemcpyAsync(c->fstage, W, sizeof(float) * nW, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, c->pipe.in(c->device, c->fstage, W, sizeof(float) * nW, c->stream));
     HIP_TRY(c, ccd::launch_permute_ranks(c->fstage, c->W, c->csr.dperm, k, c->m, true, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(c->fstage, H, sizeof(float) * nH, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, c->pipe.in(c->device, c->fstage, H, sizeof(float) * nH, c->stream));
     HIP_TRY(c, ccd::launch_permute_ranks(c->fstage, c->H, c->csc.dperm, k, c->n, true, c->stream));
     if (c->nnz) {
         HIP_TRY(c, hipMemcpyAsync(c->csr.val, c->csr.val0, 4 * c->nnz, hipMemcpyDeviceToDevice, c->stream));
@@ -1159,7 +1160,7 @@ int32_t ccd_get_factors(ccd_ctx* c, float* W, float* H) {
         if (!out) continue;
         HIP_TRY(c, ccd::launch_permute_ranks(q == 0 ? c->W : c->H, c->fstage, q == 0 ? c->csr.dperm : c->csc.dperm, k,
                                              q == 0 ? c->m : c->n, false, c->stream));
-        HIP_TRY(c, ccd::copy_sync(c->stream, out, c->fstage, sizeof(float) * (q == 0 ? nW : nH), hipMemcpyDeviceToHost));
+        HIP_TRY(c, c->pipe.out(c->device, out, c->fstage, sizeof(float) * (q == 0 ? nW : nH), c->stream));
     }
     return CCD_OK;
 }
@@ -1176,7 +1177,7 @@ int32_t ccd_get_residual(ccd_ctx* c, float* csr_val, float* csc_val) {
         const DevLayout& L = q == 0 ? c->csr : c->csc;
         if (!out) continue;
         HIP_TRY(c, ccd::launch_scatter(L.val, L.src, c->stage, c->nnz, c->stream));
-        HIP_TRY(c, ccd::copy_sync(c->stream, out, c->stage, 4 * c->nnz, hipMemcpyDeviceToHost));
+        HIP_TRY(c, c->pipe.out(c->device, out, c->stage, 4 * c->nnz, c->stream));
     }
     return CCD_OK;
 }

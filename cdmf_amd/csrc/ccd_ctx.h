@@ -4,6 +4,7 @@
 #pragma once
 #include "cdmf_hip.h"
 #include "ccd_kernels.h"
+#include "host_pipe.h"
 
 #include <map>
 #include <string>
@@ -128,6 +129,7 @@ struct ccd_ctx {
     std::map<uint32_t, int> occupancy;  // persistent kernel -> blocks per CU by register use
     void* fmem = nullptr;     // the one allocation behind W, H and fstage
     float* fstage = nullptr;  // one factor matrix on its way between the two numberings
+    ccd::HostPipe pipe;       // the caller's large arrays
     // grow-only staging of the residual on its way back
     float* stage = nullptr;
     size_t stage_cap = 0;

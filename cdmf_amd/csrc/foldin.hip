@@ -3,6 +3,7 @@
 // the fold-in of new rows (kernels/foldin_kernels.hip).
 #include "cdmf_foldin.h"
 #include "ccd_kernels.h"
+#include "host_pipe.h"
 #include "layout.h"
 
 #include <algorithm>
@@ -66,6 +67,7 @@ static int obj_err(std::string& err, int code, const std::string& msg) {
 struct ccd_mlp {
     int device = 0;
     hipStream_t stream = nullptr;
+    ccd::HostPipe pipe;
     std::string err;
     uint32_t in = 0, hid = 0, out = 0;
     uint64_t np = 0;
@@ -378,9 +380,9 @@ int32_t ccd_mlp_forward(ccd_mlp* m, uint64_t rows, const float* X, float* Y, int
     // the rows pass through the training set's buffers
     OBJ_TRY(m, ensure(&m->X, &m->cap_x, rows * m->in));
     OBJ_TRY(m, ensure(&m->T, &m->cap_t, rows * m->out));
-    OBJ_TRY(m, hipMemcpyAsync(m->X, X, 4 * rows * m->in, hipMemcpyHostToDevice, m->stream));
+    OBJ_TRY(m, m->pipe.in(m->device, m->X, X, 4 * rows * m->in, m->stream));
     if (int rc = mlp_forward_dev(m, rows, m->X, m->T, bf16_weights, m->stream)) return rc;
-    OBJ_TRY(m, ccd::copy_sync(m->stream, Y, m->T, 4 * rows * m->out, hipMemcpyDeviceToHost));
+    OBJ_TRY(m, m->pipe.out(m->device, Y, m->T, 4 * rows * m->out, m->stream));
     return CCD_OK;
 }
 
@@ -410,8 +412,8 @@ int32_t ccd_mlp_train(ccd_mlp* m, uint64_t rows, const float* X, const float* T,
     OBJ_TRY(m, ensure(&m->perm, &m->cap_perm, rows));
     const uint64_t nb = (rows + batch - 1) / batch;
     OBJ_TRY(m, ensure(&m->loss, &m->cap_loss, nb));
-    OBJ_TRY(m, ccd::copy_sync(m->stream, m->X, X, 4 * rows * m->in, hipMemcpyHostToDevice));
-    OBJ_TRY(m, ccd::copy_sync(m->stream, m->T, T, 4 * rows * m->out, hipMemcpyHostToDevice));
+    OBJ_TRY(m, m->pipe.in(m->device, m->X, X, 4 * rows * m->in, m->stream));
+    OBJ_TRY(m, m->pipe.in(m->device, m->T, T, 4 * rows * m->out, m->stream));
     std::vector<uint32_t> perm(rows);
     std::vector<double> losses(nb);
     uint64_t st = seed ^ 0x747261696eull;
@@ -495,6 +497,7 @@ hipError_t scratch_on(int device, unsigned char** out) {
 struct ccd_fold {
     int device = 0;
     hipStream_t stream = nullptr;
+    ccd::HostPipe pipe;
     std::string err;
     uint32_t k = 0;
     int64_t n = 0;
@@ -581,8 +584,8 @@ int fold_upload(ccd_fold* f, int64_t rows, const uint32_t* ptr, const uint32_t* 
     f->nlong = (uint32_t)lr.size();
     f->nfeat = count_long(rows, ptr, ccd::FOLD_SHORT);
     if (nnz) {
-        OBJ_TRY(f, hipMemcpyAsync(f->idx, idx, 4 * nnz, hipMemcpyHostToDevice, f->stream));
-        OBJ_TRY(f, hipMemcpyAsync(f->val, val, 4 * nnz, hipMemcpyHostToDevice, f->stream));
+        OBJ_TRY(f, f->pipe.in(f->device, f->idx, idx, 4 * nnz, f->stream));
+        OBJ_TRY(f, f->pipe.in(f->device, f->val, val, 4 * nnz, f->stream));
         if (int rc = fold_check_device(f, f->idx, nnz)) return rc;
     }
     *a = ccd::FoldArgs{f->ptr, f->idx, f->val, f->HT, (uint32_t)rows, f->k, fold_ld(f->k), (uint32_t)f->n, 0, f->lambda};
@@ -649,7 +652,7 @@ int32_t ccd_fold_features(ccd_fold* f, int64_t rows, const uint32_t* ptr, const 
     OBJ_TRY(f, ensure(&f->F, &f->cap_f, nf));
     OBJ_TRY(f, ccd::launch_fold_features(a, f->long_rows, f->nfeat, f->F, f->stream));
     OBJ_TRY(f, hipStreamSynchronize(f->stream));
-    if (nf) OBJ_TRY(f, hipMemcpy(F, f->F, 4 * nf, hipMemcpyDeviceToHost));
+    OBJ_TRY(f, f->pipe.out(f->device, F, f->F, 4 * nf, f->stream));
     return CCD_OK;
 }
 
@@ -672,7 +675,7 @@ int32_t ccd_fold_rows(ccd_fold* f, int64_t rows, const uint32_t* ptr, const uint
     float ms = 0.0f;
     OBJ_TRY(f, hipEventElapsedTime(&ms, f->ea, f->eb));
     if (seconds) *seconds = ms * 1e-3;
-    if (nw) OBJ_TRY(f, hipMemcpy(W, f->W, 4 * nw, hipMemcpyDeviceToHost));
+    OBJ_TRY(f, f->pipe.out(f->device, W, f->W, 4 * nw, f->stream));
     return CCD_OK;
 }
 
@@ -745,7 +748,7 @@ int32_t ccd_fold_warm(ccd_fold* f, ccd_mlp* m, int64_t rows, const uint32_t* ptr
     float ms = 0.0f;
     OBJ_TRY(f, hipEventElapsedTime(&ms, f->ea, f->eb));
     if (seconds) *seconds = ms * 1e-3;
-    if (nw) OBJ_TRY(f, hipMemcpy(W, f->W, 4 * nw, hipMemcpyDeviceToHost));
+    OBJ_TRY(f, f->pipe.out(f->device, W, f->W, 4 * nw, f->stream));
     return CCD_OK;
 }
 
