@@ -518,6 +518,16 @@ int build_tiled(ccd_ctx* c, DevLayout& L, int sigma, uint32_t split_at) {
     return CCD_OK;
 }
 
+// Whether a sweep over layout L can finish the rows of P that the sweep
+// before it left as tile partials (TiledArgs::prev): few enough that every
+// block may do them all (the long ones in two rounds of its waves), and the
+// gathered vector short enough to stage whole in one round.
+bool can_merge_spans(const DevLayout& P, const DevLayout& L) {
+    const TiledLayout &T = P.tl, &U = L.tl;
+    return !T.split && T.nspan != 0 && T.nshort <= ccd::SPAN_MERGE_SHORT && T.nspan - T.nshort <= 32 && U.ntiles != 0 &&
+           U.ib == 2 && L.gdim <= 16384;
+}
+
 int do_tiled_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* xs, const void* ys, const void* xa,
                   const void* ya, bool x_is_cur, bool sub, bool add, bool sweep, float lambda, int kind) {
     TiledLayout& T = L.tl;
@@ -528,8 +538,13 @@ int do_tiled_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* 
     // costs more than its gathers from L2.  40,000 x 5,000 with 1M ratings:
     // 12.5 us a pass staged, 11.4 not; 147,910 x 3,297 with 4.5M: 19.0 and
     // 19.6.  (2-byte factors: never faster unstaged, 12.4 and 12.5 us at 1M.)
+    const ccd::SpanArgs prev = c->pending_spans;
+    c->pending_spans = ccd::SpanArgs{};
     const uint32_t nb = std::min(sh.blocks, std::max(T.ntiles, 1u));
-    if (sweep && factor_bytes(c) == 4 && (double)L.nnz < 0.3 * nb * ((double)hot.x + 2.0 * hot.p)) hot = {0, 0};
+    if (prev.nspan) {  // x staged whole, the rest of the LDS for pairs
+        const size_t left = sh.lds_budget / factor_bytes(c) - (size_t)L.gdim - 8;
+        hot = {(uint32_t)L.gdim, fused ? (uint32_t)std::min<size_t>(left / 2, (size_t)L.gdim) : 0u};
+    } else if (sweep && factor_bytes(c) == 4 && (double)L.nnz < 0.3 * nb * ((double)hot.x + 2.0 * hot.p)) hot = {0, 0};
     // tiles of second parts gather from beyond the LDS prefix only when the
     // split is at or past it (a prefix staged with two blocks per CU, or in
     // bfloat16, differs from the one the layout was split at)
@@ -537,7 +552,7 @@ int do_tiled_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* 
     ccd::TiledArgs a{L.ptr, T.tidx, T.tval, sweep ? x : nullptr, y, xs, ys, xa, ya, fused ? L.pair : nullptr,
                      T.flags, T.row0, T.segoff, T.segrows, T.open, T.gmax, T.head, T.tail, L.nnz, T.ntiles,
                      hot.x, hot.p, (uint32_t)(fused && x_is_cur), lambda, T.cold_row, T.nreal,
-                     sweep ? T.part : nullptr, cold0, T.cold_tile0};
+                     sweep ? T.part : nullptr, cold0, T.cold_tile0, prev};
     {
         Timed tm(c, kind, true);
         HIP_TRY(c, ccd::launch_tiled(a, T.sigma, c->prec, T.ib, sub, add, sweep, sh.blocks, c->stream, tm.ev()));
@@ -547,8 +562,12 @@ int do_tiled_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* 
         const ccd::SplitArgs fa{T.srows, T.part, T.head, T.tail, y, lambda, T.nreal};
         HIP_TRY(c, ccd::launch_split_finish(fa, c->prec, c->stream));
     } else if (sweep && T.nspan) {
+        const ccd::SpanArgs sa{T.spans, T.head, T.tail, y, T.nspan, T.nshort, lambda, nullptr};
+        if (c->defer_spans) {
+            c->pending_spans = sa;
+            return CCD_OK;
+        }
         Timed tm(c, CCD_K_FINALIZE);
-        ccd::SpanArgs sa{T.spans, T.head, T.tail, y, T.nspan, T.nshort, lambda, nullptr};
         HIP_TRY(c, ccd::launch_span(sa, c->prec, c->stream));
     }
     return CCD_OK;
@@ -936,6 +955,9 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
         if (!rc0) rc0 = build_tiled(c, S, (int)c->plan.sigma, split_bound(c));
         if (rc0) return rc0;
     }
+    const bool f_to_s = tiled && can_merge_spans(F, S), s_to_f = tiled && can_merge_spans(S, F);
+    c->defer_spans = false;
+    c->pending_spans = ccd::SpanArgs{};
     const bool tl = tiled, sp = c->plan.split_rows != 0;
     c->kind_bytes[CCD_K_SWEEP_F] = layout_bytes(F, tl, sp, false, 1, 0, true);
     c->kind_bytes[CCD_K_SWEEP_S] = layout_bytes(S, tl, sp, false, 1, 0, true);
@@ -999,13 +1021,19 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
             const bool add = oiter > 1 || c->continued;
             const bool fused = pending || add;
             if (sweeps) {
+                // a sweep's spanning rows go to the next sweep, but for the
+                // rank's last, whose vector the commit reads
+                c->defer_spans = f_to_s;
                 int rc1 = pass(c, F, St, vF, Sp, Fp, St, Ft, true, pending, add, true, lambda, fused ? CCD_K_FUSED_F : CCD_K_SWEEP_F);
                 if (rc1) return rc1;
+                c->defer_spans = s_to_f && Tin > 1;
                 rc1 = pass(c, S, vF, vS, Fp, Sp, Ft, St, false, pending, add, true, lambda, fused ? CCD_K_FUSED_S : CCD_K_SWEEP_S);
                 if (rc1) return rc1;
                 for (int it = 2; it <= Tin; ++it) {
+                    c->defer_spans = f_to_s;
                     rc1 = pass(c, F, vS, vF, nullptr, nullptr, nullptr, nullptr, false, false, false, true, lambda, CCD_K_SWEEP_F);
                     if (rc1) return rc1;
+                    c->defer_spans = s_to_f && it < Tin;
                     rc1 = pass(c, S, vF, vS, nullptr, nullptr, nullptr, nullptr, false, false, false, true, lambda, CCD_K_SWEEP_S);
                     if (rc1) return rc1;
                 }

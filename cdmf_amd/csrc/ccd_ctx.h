@@ -133,6 +133,10 @@ struct ccd_ctx {
     // grow-only staging of the residual on its way back
     float* stage = nullptr;
     size_t stage_cap = 0;
+    // tiled sweeps: whether the pass about to be launched may leave its
+    // spanning rows to the next one, and what the last one left
+    bool defer_spans = false;
+    ccd::SpanArgs pending_spans{};
     double* rmse_bsum = nullptr;
     double* rmse_dev = nullptr;  // one slot per outer iteration
     double* obj_dev = nullptr;   // objective, loss, regulariser

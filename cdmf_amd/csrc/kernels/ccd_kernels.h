@@ -306,6 +306,19 @@ hipError_t launch_copy(const float4* src, float4* dst, uint64_t count, hipStream
 hipError_t launch_count_below(const uint32_t* ptr, const void* idx, bool idx16, uint64_t rows, uint32_t bound,
                               uint32_t* out, hipStream_t s);
 
+// spans[0, nshort) cover two tiles (t1 = t0 + 1) and are finished one per
+// lane; spans[nshort, nspan) cover more and are finished one per wave.
+struct SpanArgs {
+    const SpanRow* spans;
+    const void* head;
+    const void* tail;
+    void* y;
+    uint32_t nspan;
+    uint32_t nshort;
+    float lambda;
+    void* part;  // split layout: (g, h) of each spanning virtual row go here instead of finishing it
+};
+
 // ---------------------------------------------------------------- tiled ---
 // Tiled layout of one compressed matrix (the CSR5 idea of
 // src/detail/kcode/csr5_spmv.cl, re-derived for 64-wide waves): the nnz
@@ -365,20 +378,13 @@ struct TiledArgs {
     // First tile of the layout's costly tail (second parts of split rows),
     // whose tiles a block spreads over its whole pass; 0xffffffff: none.
     uint32_t spread_tile0;
+    // Rows of x that the previous sweep left as tile partials, finished by
+    // this sweep's blocks before their first tile (prev.nspan != 0): x is
+    // prev.y and staged whole (hot_x is its length), 16-bit indices, at most
+    // SPAN_MERGE_SHORT two-tile spans.  Block 0 also stores them to prev.y.
+    SpanArgs prev;
 };
-
-// spans[0, nshort) cover two tiles (t1 = t0 + 1) and are finished one per
-// lane; spans[nshort, nspan) cover more and are finished one per wave.
-struct SpanArgs {
-    const SpanRow* spans;
-    const void* head;
-    const void* tail;
-    void* y;
-    uint32_t nspan;
-    uint32_t nshort;
-    float lambda;
-    void* part;  // split layout: (g, h) of each spanning virtual row go here instead of finishing it
-};
+constexpr uint32_t SPAN_MERGE_SHORT = 512;  // threads of the smallest tiled block
 
 // Finish of a split layout's sweep, one wave per row: each part's (g, h) is
 // the tile kernel's part[] entry when the part lies in one tile, else its
