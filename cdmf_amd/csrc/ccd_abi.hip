@@ -519,13 +519,15 @@ int build_tiled(ccd_ctx* c, DevLayout& L, int sigma, uint32_t split_at) {
 }
 
 // Whether a sweep over layout L can finish the rows of P that the sweep
-// before it left as tile partials (TiledArgs::prev): few enough that every
+// before it left as tile partials (MergedArgs): few enough that every
 // block may do them all (the long ones in two rounds of its waves), and the
-// gathered vector short enough to stage whole in one round.
+// gathered vector short enough to stage whole.  A pass, merged and not: about
+// 200 spans (8,000 x 2,000) 9.1 and 9.9 us, about 490 (20,000 x 3,000) 10.8
+// and 10.6; a vector of 10,000, which is else not staged, 12.6 and 12.4.
 bool can_merge_spans(const DevLayout& P, const DevLayout& L) {
     const TiledLayout &T = P.tl, &U = L.tl;
     return !T.split && T.nspan != 0 && T.nshort <= ccd::SPAN_MERGE_SHORT && T.nspan - T.nshort <= 32 && U.ntiles != 0 &&
-           U.ib == 2 && L.gdim <= 16384;
+           U.ib == 2 && L.gdim <= 8192;
 }
 
 int do_tiled_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* xs, const void* ys, const void* xa,
@@ -552,10 +554,11 @@ int do_tiled_pass(ccd_ctx* c, DevLayout& L, const void* x, void* y, const void* 
     ccd::TiledArgs a{L.ptr, T.tidx, T.tval, sweep ? x : nullptr, y, xs, ys, xa, ya, fused ? L.pair : nullptr,
                      T.flags, T.row0, T.segoff, T.segrows, T.open, T.gmax, T.head, T.tail, L.nnz, T.ntiles,
                      hot.x, hot.p, (uint32_t)(fused && x_is_cur), lambda, T.cold_row, T.nreal,
-                     sweep ? T.part : nullptr, cold0, T.cold_tile0, prev};
+                     sweep ? T.part : nullptr, cold0, T.cold_tile0};
     {
         Timed tm(c, kind, true);
-        HIP_TRY(c, ccd::launch_tiled(a, T.sigma, c->prec, T.ib, sub, add, sweep, sh.blocks, c->stream, tm.ev()));
+        HIP_TRY(c, ccd::launch_tiled(a, prev.nspan ? &prev : nullptr, T.sigma, c->prec, T.ib, sub, add, sweep, sh.blocks,
+                                     c->stream, tm.ev()));
     }
     if (sweep && T.split) {
         Timed tm(c, CCD_K_FINALIZE);

@@ -378,13 +378,17 @@ struct TiledArgs {
     // First tile of the layout's costly tail (second parts of split rows),
     // whose tiles a block spreads over its whole pass; 0xffffffff: none.
     uint32_t spread_tile0;
-    // Rows of x that the previous sweep left as tile partials, finished by
-    // this sweep's blocks before their first tile (prev.nspan != 0): x is
-    // prev.y and staged whole (hot_x is its length), 16-bit indices, at most
-    // SPAN_MERGE_SHORT two-tile spans.  Block 0 also stores them to prev.y.
+};
+// A sweep whose blocks finish, before their first tile, the rows of x that
+// the previous sweep left as tile partials: x is prev.y and staged whole
+// (hot_x is its length), 16-bit indices, at most SPAN_MERGE_SHORT two-tile
+// spans.  Block 0 also stores the rows to prev.y.  A type of its own: the 64
+// bytes more cost the sweeps that merge nothing 0.2 to 0.5 us a pass.
+struct MergedArgs {
+    TiledArgs tile;
     SpanArgs prev;
 };
-constexpr uint32_t SPAN_MERGE_SHORT = 512;  // threads of the smallest tiled block
+constexpr uint32_t SPAN_MERGE_SHORT = 256;  // at most a tiled block's threads (512)
 
 // Finish of a split layout's sweep, one wave per row: each part's (g, h) is
 // the tile kernel's part[] entry when the part lies in one tile, else its
@@ -412,8 +416,9 @@ struct Idx24 {};
 // sigma 8, 16 or 32 for FP32 (32 in 512-thread blocks: at 1024 threads
 // its kernels spilled to scratch and the spilled passes gave wrong
 // results), 16 for the other precisions; ib: bytes per index
-hipError_t launch_tiled(const TiledArgs& a, int sigma, int prec, int ib, bool sub, bool add, bool sweep,
-                        uint32_t blocks, hipStream_t s, const LaunchEvents* ev = nullptr);
+// prev (may be null): the previous sweep's spanning rows (MergedArgs).
+hipError_t launch_tiled(const TiledArgs& a, const SpanArgs* prev, int sigma, int prec, int ib, bool sub, bool add,
+                        bool sweep, uint32_t blocks, hipStream_t s, const LaunchEvents* ev = nullptr);
 hipError_t launch_span(const SpanArgs& a, int prec, hipStream_t s);
 int tiled_blocks_per_cu(int sigma, int prec, int ib, bool sub, bool add, bool sweep, bool x_is_cur);
 // Layout order <-> tiled order (to_tiled = true: src in layout order, dst

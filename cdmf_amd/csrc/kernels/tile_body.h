@@ -466,25 +466,15 @@ __device__ __forceinline__ void tile_body(const TiledArgs& a, const TF* lds, con
 // A row spanning two tiles, by one lane: tail[t0] + head[t0 + 1], rounded
 // exactly as span_row rounds it (the head first passes through a sum with
 // zero, as in span_row's tree).
-template <typename TA>
-__device__ __forceinline__ Pair<TA> span_short_sum(const SpanArgs& a, const SpanRow& sp) {
-    const Pair<TA> tl = static_cast<const Pair<TA>*>(a.tail)[sp.t0];
-    const Pair<TA> hd = static_cast<const Pair<TA>*>(a.head)[sp.t1];
-    return Pair<TA>{tl.g + ((TA)0 + hd.g), tl.h + ((TA)0 + hd.h)};
-}
-
-// The finished value of a spanning row.
-template <typename TA>
-__device__ __forceinline__ float span_value(const SpanArgs& a, const SpanRow& sp, const Pair<TA>& s) {
-    return (float)(s.g / ((TA)a.lambda * (TA)sp.len + s.h));
-}
-
 template <typename TF, typename TA>
 __device__ __forceinline__ void span_short(const SpanArgs& a, uint32_t i) {
     const SpanRow sp = a.spans[i];
-    const Pair<TA> s = span_short_sum<TA>(a, sp);
-    if (a.part) static_cast<Pair<TA>*>(a.part)[sp.row] = s;
-    else stf<TF>(a.y, sp.row, span_value<TA>(a, sp, s));
+    const Pair<TA> tl = static_cast<const Pair<TA>*>(a.tail)[sp.t0];
+    const Pair<TA> hd = static_cast<const Pair<TA>*>(a.head)[sp.t1];
+    const TA g = tl.g + ((TA)0 + hd.g);
+    const TA h = tl.h + ((TA)0 + hd.h);
+    if (a.part) static_cast<Pair<TA>*>(a.part)[sp.row] = Pair<TA>{g, h};
+    else stf<TF>(a.y, sp.row, (float)(g / ((TA)a.lambda * (TA)sp.len + h)));
 }
 
 // tail[t0] + head[t0+1] + ... + head[t1] by one wave: lane-strided partial
@@ -517,7 +507,7 @@ __device__ __forceinline__ void span_row(const SpanArgs& a, uint32_t i, int lane
     const Pair<TA> s = span_sum<TA>(a.head, a.tail, sp.t0, sp.t1, lane);
     if (lane == 0) {
         if (a.part) static_cast<Pair<TA>*>(a.part)[sp.row] = s;
-        else stf<TF>(a.y, sp.row, span_value<TA>(a, sp, s));
+        else stf<TF>(a.y, sp.row, (float)(s.g / ((TA)a.lambda * (TA)sp.len + s.h)));
     }
 }
 

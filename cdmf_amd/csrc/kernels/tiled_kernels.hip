@@ -36,6 +36,7 @@
 #include "tile_body.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace ccd {
 namespace {
@@ -53,13 +54,17 @@ using tiled::tile_body;
 // registers a 1024-thread block leaves a lane.
 constexpr int tile_block(int sigma) { return sigma > 16 ? 512 : SWEEP_BLOCK; }
 
-// MERGE: the previous sweep's spanning rows are finished here (TiledArgs::prev)
+__device__ __forceinline__ const TiledArgs& tile_args(const TiledArgs& a) { return a; }
+__device__ __forceinline__ const TiledArgs& tile_args(const MergedArgs& a) { return a.tile; }
+
+// MERGE: the previous sweep's spanning rows are finished here (MergedArgs)
 // instead of by a launch of their own.  Every block does all of them, which
-// pays while they are few: 10.1 -> 8.7 us a pass at 45,000 ratings, 9.8 -> 9.1
+// pays while they are few: 10.2 -> 8.6 us a pass at 45,000 ratings, 9.8 -> 9.0
 // at 200,000.
 template <typename IdxT, int SIGMA, typename TF, typename TA, bool SUB, bool ADD, bool SWEEP, bool XCUR,
           bool MERGE = false>
-__global__ __launch_bounds__(tile_block(SIGMA)) void tiled_kernel(TiledArgs a) {
+__global__ __launch_bounds__(tile_block(SIGMA)) void tiled_kernel(std::conditional_t<MERGE, MergedArgs, TiledArgs> arg) {
+    const TiledArgs& a = tile_args(arg);
     extern __shared__ __align__(16) unsigned char lds_raw[];
     TF* lds = reinterpret_cast<TF*>(lds_raw);
     FPair<TF>* ldsp = reinterpret_cast<FPair<TF>*>(lds_raw + lds_pair_offset<TF>(a.hot_x));
@@ -78,14 +83,18 @@ __global__ __launch_bounds__(tile_block(SIGMA)) void tiled_kernel(TiledArgs a) {
     constexpr int BS = tile_block(SIGMA);
     constexpr uint32_t NW = BS / WAVE;
     if (threadIdx.x == 0) s_next = NW;  // positions 0 .. NW-1 go to the waves in order
-    // two-tile spans, one per thread, their loads ahead of the staging's
+    // two-tile spans, one per thread (rounded as span_short does), their
+    // loads ahead of the staging's
     uint32_t span_row = 0xffffffffu;
     float span_val = 0.0f;
     if constexpr (MERGE) {
-        if (threadIdx.x < a.prev.nshort) {
-            const SpanRow sp = a.prev.spans[threadIdx.x];
+        if (threadIdx.x < arg.prev.nshort) {
+            const SpanRow sp = arg.prev.spans[threadIdx.x];
             span_row = sp.row;
-            span_val = tiled::span_value<TA>(a.prev, sp, tiled::span_short_sum<TA>(a.prev, sp));
+            const auto tl = static_cast<const tiled::Pair<TA>*>(arg.prev.tail)[sp.t0];
+            const auto hd = static_cast<const tiled::Pair<TA>*>(arg.prev.head)[sp.t1];
+            const TA h = tl.h + ((TA)0 + hd.h);
+            span_val = (float)((tl.g + ((TA)0 + hd.g)) / ((TA)arg.prev.lambda * (TA)sp.len + h));
         }
     }
     stage_lds<BS>(lds, static_cast<const TF*>(a.x), a.hot_x);
@@ -96,13 +105,13 @@ __global__ __launch_bounds__(tile_block(SIGMA)) void tiled_kernel(TiledArgs a) {
     if constexpr (MERGE) {
         auto put = [&](uint32_t row, float v) {
             stf<TF>(lds, row, v);
-            if (b == 0) stf<TF>(a.prev.y, row, v);
+            if (b == 0) stf<TF>(arg.prev.y, row, v);
         };
         if (span_row != 0xffffffffu) put(span_row, span_val);
-        for (uint32_t i = a.prev.nshort + threadIdx.x / WAVE; i < a.prev.nspan; i += NW) {
-            const SpanRow sp = a.prev.spans[i];
-            const tiled::Pair<TA> s = tiled::span_sum<TA>(a.prev.head, a.prev.tail, sp.t0, sp.t1, lane);
-            if (lane == 0) put(sp.row, tiled::span_value<TA>(a.prev, sp, s));
+        for (uint32_t i = arg.prev.nshort + threadIdx.x / WAVE; i < arg.prev.nspan; i += NW) {
+            const SpanRow sp = arg.prev.spans[i];
+            const tiled::Pair<TA> s = tiled::span_sum<TA>(arg.prev.head, arg.prev.tail, sp.t0, sp.t1, lane);
+            if (lane == 0) put(sp.row, (float)(s.g / ((TA)arg.prev.lambda * (TA)sp.len + s.h)));
         }
         __syncthreads();
     }
@@ -269,7 +278,8 @@ uint32_t grid_for(uint64_t count) {
     return (uint32_t)(b ? b : 1);
 }
 
-using TiledFn = void (*)(TiledArgs);
+// the kernels take TiledArgs or, from code 16 on, MergedArgs
+using TiledFn = const void*;
 
 // code: SUB << 2 | ADD << 1 | SWEEP, plus 8 for a fused pass whose x is the
 // pair's current value, plus 16 for a sweep that finishes the previous one's
@@ -277,24 +287,24 @@ using TiledFn = void (*)(TiledArgs);
 template <typename IdxT, int SIGMA, typename TF, typename TA>
 TiledFn tiled_fn_s(int code) {
     switch (code) {
-        case 1: return tiled_kernel<IdxT, SIGMA, TF, TA, false, false, true, false>;
-        case 2: return tiled_kernel<IdxT, SIGMA, TF, TA, false, true, false, false>;
-        case 3: return tiled_kernel<IdxT, SIGMA, TF, TA, false, true, true, false>;
-        case 4: return tiled_kernel<IdxT, SIGMA, TF, TA, true, false, false, false>;
-        case 5: return tiled_kernel<IdxT, SIGMA, TF, TA, true, false, true, false>;
-        case 6: return tiled_kernel<IdxT, SIGMA, TF, TA, true, true, false, false>;
-        case 7: return tiled_kernel<IdxT, SIGMA, TF, TA, true, true, true, false>;
-        case 8 + 3: return tiled_kernel<IdxT, SIGMA, TF, TA, false, true, true, true>;
-        case 8 + 5: return tiled_kernel<IdxT, SIGMA, TF, TA, true, false, true, true>;
-        case 8 + 7: return tiled_kernel<IdxT, SIGMA, TF, TA, true, true, true, true>;
+        case 1: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, false, false, true, false>);
+        case 2: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, false, true, false, false>);
+        case 3: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, false, true, true, false>);
+        case 4: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, true, false, false, false>);
+        case 5: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, true, false, true, false>);
+        case 6: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, true, true, false, false>);
+        case 7: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, true, true, true, false>);
+        case 8 + 3: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, false, true, true, true>);
+        case 8 + 5: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, true, false, true, true>);
+        case 8 + 7: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, true, true, true, true>);
         default: break;
     }
     if constexpr (std::is_same<IdxT, uint16_t>::value) {
         switch (code) {
-            case 16 + 1: return tiled_kernel<IdxT, SIGMA, TF, TA, false, false, true, false, true>;
-            case 16 + 3: return tiled_kernel<IdxT, SIGMA, TF, TA, false, true, true, false, true>;
-            case 16 + 5: return tiled_kernel<IdxT, SIGMA, TF, TA, true, false, true, false, true>;
-            case 16 + 7: return tiled_kernel<IdxT, SIGMA, TF, TA, true, true, true, false, true>;
+            case 16 + 1: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, false, false, true, false, true>);
+            case 16 + 3: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, false, true, true, false, true>);
+            case 16 + 5: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, true, false, true, false, true>);
+            case 16 + 7: return reinterpret_cast<TiledFn>(&tiled_kernel<IdxT, SIGMA, TF, TA, true, true, true, false, true>);
             default: break;
         }
     }
@@ -330,12 +340,11 @@ TiledFn tiled_fn(int sigma, int prec, int ib, bool sub, bool add, bool sweep, bo
 
 }  // namespace
 
-hipError_t launch_tiled(const TiledArgs& a, int sigma, int prec, int ib, bool sub, bool add, bool sweep,
-                        uint32_t blocks, hipStream_t s, const LaunchEvents* ev) {
+hipError_t launch_tiled(const TiledArgs& a, const SpanArgs* prev, int sigma, int prec, int ib, bool sub, bool add,
+                        bool sweep, uint32_t blocks, hipStream_t s, const LaunchEvents* ev) {
     if (!sub && !add && !sweep) return record_unlaunched(ev, s);
-    const bool merge = a.prev.nspan != 0;
-    if (merge && (a.prev.nshort > SPAN_MERGE_SHORT || a.prev.y != a.x || a.prev.part)) return hipErrorInvalidValue;
-    const TiledFn fn = tiled_fn(sigma, prec, ib, sub, add, sweep, a.x_is_cur != 0, merge);
+    if (prev && (prev->nshort > SPAN_MERGE_SHORT || prev->y != a.x || prev->part)) return hipErrorInvalidValue;
+    const TiledFn fn = tiled_fn(sigma, prec, ib, sub, add, sweep, a.x_is_cur != 0, prev != nullptr);
     if (!fn) return hipErrorInvalidValue;
     const int bs = tile_block(sigma);
     if (a.ntiles == 0) return record_unlaunched(ev, s);
@@ -344,9 +353,9 @@ hipError_t launch_tiled(const TiledArgs& a, int sigma, int prec, int ib, bool su
     // 11.3 -> 10.1 us a pass with its finish; 8,000 x 2,000 with 200,000:
     // 11.5 -> 9.8)
     if (blocks > a.ntiles) blocks = a.ntiles;
-    TiledArgs arg = a;
-    void* args[] = {&arg};
-    return hipExtLaunchKernel(reinterpret_cast<const void*>(fn), dim3(blocks), dim3(bs), args,
+    MergedArgs arg{a, prev ? *prev : SpanArgs{}};
+    void* args[] = {prev ? (void*)&arg : (void*)&arg.tile};
+    return hipExtLaunchKernel(fn, dim3(blocks), dim3(bs), args,
                               staged_lds_bytes(prec, a.hot_x, a.hot_p), s, ev ? ev->start : nullptr,
                               ev ? ev->stop : nullptr, 0);
 }
@@ -354,8 +363,7 @@ hipError_t launch_tiled(const TiledArgs& a, int sigma, int prec, int ib, bool su
 int tiled_blocks_per_cu(int sigma, int prec, int ib, bool sub, bool add, bool sweep, bool xcur) {
     const TiledFn fn = tiled_fn(sigma, prec, ib, sub, add, sweep, xcur, false);
     int nb = 0;
-    if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(fn), tile_block(sigma),
-                                                            0) != hipSuccess)
+    if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, tile_block(sigma), 0) != hipSuccess)
         return 1;
     return nb < 1 ? 1 : nb;
 }

@@ -1,4 +1,4 @@
-"""Rows spanning tiles finished by the next sweep (TiledArgs::prev) instead of
+"""Rows spanning tiles finished by the next sweep (MergedArgs) instead of
 a launch of their own: bit for bit what the batched solver, which finishes
 them between two barriers, computes for the same problem."""
 import numpy as np
@@ -24,13 +24,20 @@ CASES = {
     # one tile and none spanning, two tiles and one span
     "one_tile": lambda: _uniform(20, 40, 10, 1),
     "two_tiles": lambda: _uniform(50, 60, 25, 2),
-    # about 512 two-tile spans in the rows' layout, just below and above
+    # about 256 two-tile spans in the rows' layout (sigma 16), the bound of
+    # the merge: just below and above
+    "spans_252": lambda: _uniform(8900, 300, 30, 9),
+    "spans_262": lambda: _uniform(9270, 300, 30, 10),
+    # about 512 in the rows' layout, just below and above
     "spans_500": lambda: _uniform(17100, 300, 30, 3),
     "spans_530": lambda: _uniform(18100, 300, 30, 4),
     # 32 and 33 rows over more than two tiles
     "long_32": lambda: _rows([4000] * 32 + [7] * 500, 5000, 5),
     "long_33": lambda: _rows([4000] * 33 + [7] * 500, 5000, 6),
     # the gathered vector at the bound of the merge, and past it
+    "wide_8192": lambda: _rows([1500] * 40 + [3] * 900, 8192, 11),
+    "wide_8193": lambda: _rows([1500] * 40 + [3] * 900, 8193, 12),
+    # past it, where the vector fills much of the LDS
     "wide_16384": lambda: _rows([1500] * 40 + [3] * 900, 16384, 7),
     "wide_16385": lambda: _rows([1500] * 40 + [3] * 900, 16385, 8),
 }
