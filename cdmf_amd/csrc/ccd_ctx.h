@@ -184,8 +184,10 @@ class Carver {
 public:
     template <class T>
     void add(T** p, size_t count) {
+        const size_t bytes = sizeof(T) * (count ? count : 1);
+        if (bytes >= BIG) total_ = (total_ + PAGE - 1) & ~(PAGE - 1);
         slots_.push_back({reinterpret_cast<void**>(p), total_});
-        total_ += (sizeof(T) * (count ? count : 1) + 255) & ~(size_t)255;
+        total_ += (bytes + 255) & ~(size_t)255;
     }
     hipError_t alloc(void** base) {
         const hipError_t e = hipMalloc(base, total_ ? total_ : 1);
@@ -203,6 +205,11 @@ public:
     size_t bytes() const { return total_; }
 
 private:
+    // The largest arrays start on a 2 MB boundary, where an allocation of
+    // their own would.  99M ratings, 480,189 x 17,770: 52.7 -> 52.2 ms an
+    // outer iteration of rank 40.  With all arrays from 2 MB on there, 4.5M
+    // ratings took 19.0 -> 19.2 us a pass and 9M 25.9 -> 26.1.
+    static constexpr size_t BIG = (size_t)64 << 20, PAGE = (size_t)2 << 20;
     struct Slot {
         void** p;
         size_t off;
