@@ -333,8 +333,9 @@ __device__ __forceinline__ void fold_chain(const double* m, uint32_t groups, con
 
 // The sweeps of one row from its G and b in LDS, by one wave: lane l holds
 // ranks l and, for k > 64 (NS = 2), l + 64.  Column s of G is only touched by
-// rank s's lane, which scales it in place.  Rows k .. of G up to a multiple
-// of CHAIN are cleared, so the chain runs in whole groups.
+// rank s's lane, which scales it in place.  The chain runs in whole groups:
+// columns k .. of G, which the products leave unwritten, and rows k .. up to
+// a multiple of CHAIN are cleared, so the ranks there stay zero.
 template <int NS, int LD>
 __device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint32_t d, double* G, const double* b,
                                            const float* __restrict__ W0, float* __restrict__ W) {
@@ -345,6 +346,7 @@ __device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
         const uint32_t s = lane + WAVE * j;
+        double scale = 0.0;
         e[j] = 0.0;
         w[j] = 0.0;
         if (s < k) {
@@ -359,11 +361,16 @@ __device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint
                 }
             }
             e[j] = __builtin_fma(p, inv, -w[j]);
-#pragma unroll 4
-            for (uint32_t u = 0; u < k; ++u) col[u * LD] = u == s ? 1.0 : col[u * LD] * inv;
+            scale = inv;
         }
-        if (s < (uint32_t)LD)
+        if (s < (uint32_t)LD) {
+#pragma unroll 4
+            for (uint32_t u = 0; u < k; ++u) {
+                const double v = G[u * LD + s] * scale;
+                G[u * LD + s] = s >= k ? 0.0 : u == s ? 1.0 : v;
+            }
             for (uint32_t u = k; u % CHAIN; ++u) G[u * LD + s] = 0.0;
+        }
     }
     // one wave: its LDS writes above come before its reads below
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

@@ -145,6 +145,34 @@ def test_fold_rows_normal_equations(k):
     fold.close()
 
 
+@pytest.mark.parametrize("k", [1, 7, 8, 9, 57, 63, 65, 71, 100, 121])
+def test_fold_rows_after_rows_without_a_number(k):
+    """Ranks around a whole group of the chain, after rows whose products are
+    NaN: what they left on the chip reaches no other call.  Bound as in
+    test_fold_rows_normal_equations."""
+    F = _gpu()
+    rng = np.random.default_rng(k)
+    rows, n = 4096, 50
+    ptr = (2 * np.arange(rows + 1)).astype(np.uint32)
+    idx = np.tile(np.array([0, 1], np.uint32), rows)
+    val = np.ones(2 * rows, np.float32)
+    wide = F.FoldIn(np.full((128, n), np.nan, np.float32), 0.05)
+    H = rng.normal(0.1, 0.4, (k, n)).astype(np.float32)
+    fold = F.FoldIn(H, 0.05)
+    deg = [1, 5, 20, 40]
+    p2 = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+    i2 = np.concatenate([rng.choice(n, size=d, replace=False) for d in deg]).astype(np.uint32)
+    v2 = rng.integers(1, 6, size=i2.size).astype(np.float32)
+    ref = _fold_f64(p2, i2, v2, H, 0.05, 2, None)
+    for call in (fold.rows, fold.rows_noalloc):
+        bad, _ = wide.rows(ptr, idx, val, 1)
+        assert np.isnan(bad).all()
+        W, _ = call(p2, i2, v2, 2)
+        np.testing.assert_allclose(W, ref, rtol=6.1e-8, atol=1e-9 * float(np.abs(ref).max()))
+    wide.close()
+    fold.close()
+
+
 @pytest.mark.parametrize("nnz", [300, 65536, 70000])  # the index check on the host, and on the device
 def test_fold_refuses_indices_out_of_range(nnz):
     from cdmf_amd.solver import CCDError
