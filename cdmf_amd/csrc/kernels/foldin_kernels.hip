@@ -10,6 +10,12 @@
 #include "ccd_kernels.h"
 
 namespace ccd {
+
+// old with lane `lane` (constant) replaced by the uniform x: the compiler's
+// own lane write, which it keeps two wait states behind the lane read that x
+// comes from.  (It does not look into inline assembly.)
+__device__ int write_lane(int x, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+
 namespace {
 
 constexpr int WAVE = 64;
@@ -290,13 +296,13 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
     return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
 
-// v with lane LANE replaced by the uniform x
+// old with lane LANE replaced by the uniform x
 template <int LANE>
-__device__ __forceinline__ double with_lane(double v, double x) {
-    unsigned long long a = (unsigned long long)__double_as_longlong(v), b = (unsigned long long)__double_as_longlong(x);
-    uint32_t lo = (uint32_t)a, hi = (uint32_t)(a >> 32);
-    asm("v_writelane_b32 %0, %1, %2" : "+v"(lo) : "s"((uint32_t)b), "n"(LANE));
-    asm("v_writelane_b32 %0, %1, %2" : "+v"(hi) : "s"((uint32_t)(b >> 32)), "n"(LANE));
+__device__ __forceinline__ double with_lane(double old, double x) {
+    const unsigned long long a = (unsigned long long)__double_as_longlong(old);
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const uint32_t lo = (uint32_t)write_lane((int)(uint32_t)b, LANE, (int)(uint32_t)a);
+    const uint32_t hi = (uint32_t)write_lane((int)(uint32_t)(b >> 32), LANE, (int)(uint32_t)(a >> 32));
     return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
 
