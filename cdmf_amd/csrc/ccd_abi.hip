@@ -1105,10 +1105,12 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
                 HIP_TRY(c, ei);
                 c->graph_key = gkey;
             }
+            groups.begin();
             {
                 Timed tm(c, -1);
                 HIP_TRY(c, hipGraphLaunch(c->graph_exec, c->stream));
             }
+            groups.end(-1);
             pending = true;
             prev = k - 1;
         } else {
