@@ -623,6 +623,68 @@ int upload_indices(ccd_ctx* c, const UploadScratch& tmp, uint32_t* d, const uint
     return CCD_OK;
 }
 
+// The context's test set from checked entries in the caller's numbering.
+int store_test(ccd_ctx* c, uint64_t nnz, const uint32_t* row, const uint32_t* col, const float* val) {
+    dfree(c->trow);
+    dfree(c->tcol);
+    dfree(c->tval);
+    c->trow = c->tcol = nullptr;
+    c->tval = nullptr;
+    c->nnz_test = 0;
+    c->test_rperm.clear();
+    c->test_cperm.clear();
+    HIP_TRY(c, dalloc(&c->trow, nnz));
+    HIP_TRY(c, dalloc(&c->tcol, nnz));
+    HIP_TRY(c, dalloc(&c->tval, nnz));
+    if (nnz) {
+        // Internal numbering of the test entries, sorted by (row, column):
+        // neighbouring threads of the RMSE kernel then read neighbouring
+        // entries of each rank-major factor row, one or two cache lines a
+        // load instead of one per lane.  Only the order of the FP64 sum of
+        // squared errors changes.
+        std::vector<uint32_t> rpos((size_t)c->m), cpos((size_t)c->n), r2(nnz), c2(nnz);
+        std::vector<float> v2(nnz);
+        std::vector<uint64_t> key(nnz);
+        for (int64_t i = 0; i < c->m; ++i) rpos[c->csr.perm[i]] = (uint32_t)i;
+        for (int64_t j = 0; j < c->n; ++j) cpos[c->csc.perm[j]] = (uint32_t)j;
+        for (uint64_t e = 0; e < nnz; ++e) key[e] = (uint64_t)rpos[row[e]] << 32 | cpos[col[e]];
+        std::vector<uint64_t> order(nnz);
+        for (uint64_t e = 0; e < nnz; ++e) order[e] = e;
+        std::stable_sort(order.begin(), order.end(), [&](uint64_t x, uint64_t y) { return key[x] < key[y]; });
+        for (uint64_t q = 0; q < nnz; ++q) {
+            const uint64_t e = order[q];
+            r2[q] = (uint32_t)(key[e] >> 32);
+            c2[q] = (uint32_t)key[e];
+            v2[q] = val[e];
+        }
+        HIP_TRY(c, ccd::copy_sync(c->stream, c->trow, r2.data(), 4 * nnz, hipMemcpyHostToDevice));
+        HIP_TRY(c, ccd::copy_sync(c->stream, c->tcol, c2.data(), 4 * nnz, hipMemcpyHostToDevice));
+        HIP_TRY(c, ccd::copy_sync(c->stream, c->tval, v2.data(), 4 * nnz, hipMemcpyHostToDevice));
+    }
+    c->nnz_test = nnz;
+    return CCD_OK;
+}
+
+// A test set that is older than the last ccd_upload (test_rperm) into the
+// numbering of the matrix there is now, as if it were uploaded again;
+// dropped when that matrix is too small for one of its entries.
+int carry_test(ccd_ctx* c) {
+    if (c->test_rperm.empty()) return CCD_OK;
+    const uint64_t nnz = c->nnz_test;
+    std::vector<uint32_t> row(nnz), col(nnz);
+    std::vector<float> val(nnz);
+    HIP_TRY(c, ccd::copy_sync(c->stream, row.data(), c->trow, 4 * nnz, hipMemcpyDeviceToHost));
+    HIP_TRY(c, ccd::copy_sync(c->stream, col.data(), c->tcol, 4 * nnz, hipMemcpyDeviceToHost));
+    HIP_TRY(c, ccd::copy_sync(c->stream, val.data(), c->tval, 4 * nnz, hipMemcpyDeviceToHost));
+    bool fits = true;
+    for (uint64_t e = 0; e < nnz; ++e) {
+        row[e] = c->test_rperm[row[e]];
+        col[e] = c->test_cperm[col[e]];
+        fits = fits && (int64_t)row[e] < c->m && (int64_t)col[e] < c->n;
+    }
+    return store_test(c, fits ? nnz : 0, row.data(), col.data(), val.data());
+}
+
 }  // namespace ccdi
 
 using namespace ccdi;
@@ -759,6 +821,10 @@ int32_t ccd_upload(ccd_ctx* c, int64_t m, int64_t n, uint64_t nnz, const uint32_
     if (bad) return set_err(c, CCD_ERR_INVALID, "CSC: index out of range");
     drop_graph(c);
     ++c->gen;
+    if (c->nnz_test && c->test_rperm.empty()) {  // its entries are in the numbering that goes
+        c->test_rperm = std::move(c->csr.perm);
+        c->test_cperm = std::move(c->csc.perm);
+    }
     free_layout(c->csr);
     free_layout(c->csc);
     c->uploaded = false;
@@ -808,41 +874,7 @@ int32_t ccd_upload_test(ccd_ctx* c, uint64_t nnz, const uint32_t* row, const uin
     for (uint64_t e = 0; e < nnz; ++e)
         if ((int64_t)row[e] >= c->m || (int64_t)col[e] >= c->n) return set_err(c, CCD_ERR_INVALID, "test index out of range");
     HIP_TRY(c, hipSetDevice(c->device));
-    dfree(c->trow);
-    dfree(c->tcol);
-    dfree(c->tval);
-    c->trow = c->tcol = nullptr;
-    c->tval = nullptr;
-    c->nnz_test = nnz;
-    HIP_TRY(c, dalloc(&c->trow, nnz));
-    HIP_TRY(c, dalloc(&c->tcol, nnz));
-    HIP_TRY(c, dalloc(&c->tval, nnz));
-    if (nnz) {
-        // Internal numbering of the test entries, sorted by (row, column):
-        // neighbouring threads of the RMSE kernel then read neighbouring
-        // entries of each rank-major factor row, one or two cache lines a
-        // load instead of one per lane.  Only the order of the FP64 sum of
-        // squared errors changes.
-        std::vector<uint32_t> rpos((size_t)c->m), cpos((size_t)c->n), r2(nnz), c2(nnz);
-        std::vector<float> v2(nnz);
-        std::vector<uint64_t> key(nnz);
-        for (int64_t i = 0; i < c->m; ++i) rpos[c->csr.perm[i]] = (uint32_t)i;
-        for (int64_t j = 0; j < c->n; ++j) cpos[c->csc.perm[j]] = (uint32_t)j;
-        for (uint64_t e = 0; e < nnz; ++e) key[e] = (uint64_t)rpos[row[e]] << 32 | cpos[col[e]];
-        std::vector<uint64_t> order(nnz);
-        for (uint64_t e = 0; e < nnz; ++e) order[e] = e;
-        std::stable_sort(order.begin(), order.end(), [&](uint64_t x, uint64_t y) { return key[x] < key[y]; });
-        for (uint64_t q = 0; q < nnz; ++q) {
-            const uint64_t e = order[q];
-            r2[q] = (uint32_t)(key[e] >> 32);
-            c2[q] = (uint32_t)key[e];
-            v2[q] = val[e];
-        }
-        HIP_TRY(c, ccd::copy_sync(c->stream, c->trow, r2.data(), 4 * nnz, hipMemcpyHostToDevice));
-        HIP_TRY(c, ccd::copy_sync(c->stream, c->tcol, c2.data(), 4 * nnz, hipMemcpyHostToDevice));
-        HIP_TRY(c, ccd::copy_sync(c->stream, c->tval, v2.data(), 4 * nnz, hipMemcpyHostToDevice));
-    }
-    return CCD_OK;
+    return store_test(c, nnz, row, col, val);
 }
 
 int32_t ccd_set_factors(ccd_ctx* c, uint32_t k, const float* W, const float* H) {
@@ -933,6 +965,8 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
     char* const vS = hfirst ? ur : vr;
     const float lambda = p->lambda;
     const int T = p->maxiter, Tin = p->maxinneriter;
+    if (p->rmse_every)
+        if (int rc0 = carry_test(c)) return rc0;
     const bool do_rmse = p->rmse_every && c->nnz_test > 0;
 
     if (T > c->rmse_cap) {
@@ -1218,8 +1252,9 @@ int32_t ccd_get_residual(ccd_ctx* c, float* csr_val, float* csc_val) {
 int32_t ccd_rmse(ccd_ctx* c, double* out) {
     if (!c || !out) return CCD_ERR_INVALID;
     if (!c->factors) return set_err(c, CCD_ERR_STATE, "no factors");
-    if (c->nnz_test == 0) return set_err(c, CCD_ERR_STATE, "no test set");
     HIP_TRY(c, hipSetDevice(c->device));
+    if (int rc = carry_test(c)) return rc;
+    if (c->nnz_test == 0) return set_err(c, CCD_ERR_STATE, "no test set");
     if (c->rmse_cap < 1) {
         HIP_TRY(c, dalloc(&c->rmse_dev, 1));
         c->rmse_cap = 1;

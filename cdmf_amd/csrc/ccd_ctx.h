@@ -111,6 +111,9 @@ struct ccd_ctx {
     uint32_t* trow = nullptr;
     uint32_t* tcol = nullptr;
     float* tval = nullptr;
+    // internal -> caller's numbering of the test set where a later ccd_upload
+    // replaced the matrix it was stored for (else empty; carry_test)
+    std::vector<uint32_t> test_rperm, test_cperm;
     uint32_t k = 0;
     float* W = nullptr;
     float* H = nullptr;

@@ -121,7 +121,9 @@ int32_t ccd_upload(ccd_ctx* ctx, int64_t m, int64_t n, uint64_t nnz, const uint3
                    const uint32_t* col_idx, const float* csr_val, const uint32_t* col_ptr, const uint32_t* row_idx,
                    const float* csc_val);
 
-/* COO test set (0-based).  nnz may be 0 (no RMSE). */
+/* COO test set (0-based).  nnz may be 0 (no RMSE).  It stays with the context
+ * when ccd_upload replaces the matrix, and is dropped at its next use when
+ * the new matrix is too small for one of its entries. */
 int32_t ccd_upload_test(ccd_ctx* ctx, uint64_t nnz, const uint32_t* row, const uint32_t* col, const float* val);
 
 /* W rank-major [k][m], H rank-major [k][n] (the [t][i] indexing of MatData,
