@@ -61,26 +61,28 @@ __device__ __forceinline__ void put(const RenumArgs& a, uint32_t o, uint32_t key
     a.osrc[o] = e;
 }
 
-// Rows of at most RENUM_SHORT elements, one wave each: an element's place is
-// the number of elements before it in (index, caller's position) order,
-// counted against every lane's key in turn.
+// Rows of at most RENUM_SHORT elements, a wave at a time (waves stride over
+// the rows): an element's place is the number of elements before it in
+// (index, caller's position) order, counted against every lane's key in turn.
 template <typename IdxT>
 __global__ __launch_bounds__(BLOCK) void renum_short_kernel(RenumArgs a, uint32_t row0, uint32_t rows) {
-    const uint32_t w = blockIdx.x * (BLOCK / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (w >= rows) return;
-    const uint32_t row = row0 + w, lane = threadIdx.x & (WAVE - 1);
-    const uint32_t o = a.optr[row], len = a.optr[row + 1] - o, e = a.ptr[a.perm[row]] + lane;
-    const bool ok = lane < len;
-    const uint32_t key = ok ? a.ipos[a.idx[e]] : 0xffffffffu;
-    uint32_t rank = 0;
-    for (uint32_t j = 0; j < len; ++j) {
-        const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)key, (int)j);
-        rank += kj < key + (j < lane ? 1u : 0u) ? 1u : 0u;
+    const uint32_t lane = threadIdx.x & (WAVE - 1);
+    uint32_t w = blockIdx.x * (BLOCK / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (; w < rows; w += gridDim.x * (BLOCK / WAVE)) {
+        const uint32_t row = row0 + w;
+        const uint32_t o = a.optr[row], len = a.optr[row + 1] - o, e = a.ptr[a.perm[row]] + lane;
+        const bool ok = lane < len;
+        const uint32_t key = ok ? a.ipos[a.idx[e]] : 0xffffffffu;
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < len; ++j) {
+            const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)key, (int)j);
+            rank += kj < key + (j < lane ? 1u : 0u) ? 1u : 0u;
+        }
+        if (ok) put<IdxT>(a, o + rank, key, e);
     }
-    if (ok) put<IdxT>(a, o + rank, key, e);
 }
 
-// Rows of RENUM_SHORT + 1 .. MID_MAX elements, one block each, the same
+// Rows of RENUM_SHORT + 1 .. MID_MAX elements, a block at a time, the same
 // count against the row's keys in LDS (four a read, the same four for every
 // lane).  len^2 / 64 compares a wave: past the bound of renum_long_len the
 // bitmap below is cheaper.
@@ -114,13 +116,16 @@ __device__ __forceinline__ void renum_mid_row(const RenumArgs& a, uint32_t* keys
 }
 
 template <typename IdxT>
-__global__ __launch_bounds__(BLOCK) void renum_mid_kernel(RenumArgs a, uint32_t row0) {
+__global__ __launch_bounds__(BLOCK) void renum_mid_kernel(RenumArgs a, uint32_t row0, uint32_t rows) {
     __shared__ __align__(16) uint32_t keys[MID_MAX];
-    const uint32_t row = row0 + blockIdx.x;
-    const uint32_t o = a.optr[row], len = a.optr[row + 1] - o, e0 = a.ptr[a.perm[row]];
-    if (len <= BLOCK) renum_mid_row<IdxT, 1>(a, keys, o, len, e0);
-    else if (len <= 2 * BLOCK) renum_mid_row<IdxT, 2>(a, keys, o, len, e0);
-    else renum_mid_row<IdxT, 4>(a, keys, o, len, e0);
+    for (uint32_t b = blockIdx.x; b < rows; b += gridDim.x) {
+        const uint32_t row = row0 + b;
+        const uint32_t o = a.optr[row], len = a.optr[row + 1] - o, e0 = a.ptr[a.perm[row]];
+        if (b != blockIdx.x) __syncthreads();  // every wave is done with the last row's keys
+        if (len <= BLOCK) renum_mid_row<IdxT, 1>(a, keys, o, len, e0);
+        else if (len <= 2 * BLOCK) renum_mid_row<IdxT, 2>(a, keys, o, len, e0);
+        else renum_mid_row<IdxT, 4>(a, keys, o, len, e0);
+    }
 }
 
 // Longer rows, one block each: the row's indices are set in a bitmap of the
@@ -248,8 +253,9 @@ __global__ __launch_bounds__(BLOCK) void split_positions_kernel(const uint32_t* 
     }
 }
 
+constexpr uint32_t MAX_BLOCKS = 16384;
 uint32_t grid_for(uint64_t count) {
-    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((count + BLOCK - 1) / BLOCK, 1), 16384);
+    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((count + BLOCK - 1) / BLOCK, 1), MAX_BLOCKS);
 }
 
 }  // namespace
@@ -300,10 +306,14 @@ static hipError_t renumber(const RenumArgs& a, const RenumRows& n, uint32_t* dup
                            n.long_elems);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    if (n.nmid) hipLaunchKernelGGL(renum_mid_kernel<IdxT>, dim3(n.nmid), dim3(BLOCK), 0, s, a, n.nlong);
+    // A launch takes less than 2^32 threads, which is 16.7M rows at a block
+    // each and 67M at a wave each: a bounded grid strides over the rows.
+    if (n.nmid)
+        hipLaunchKernelGGL(renum_mid_kernel<IdxT>, dim3(std::min(n.nmid, MAX_BLOCKS)), dim3(BLOCK), 0, s, a, n.nlong,
+                           n.nmid);
     if (n.nshort)
-        hipLaunchKernelGGL(renum_short_kernel<IdxT>, dim3((n.nshort + BLOCK / WAVE - 1) / (BLOCK / WAVE)), dim3(BLOCK),
-                           0, s, a, n.nlong + n.nmid, n.nshort);
+        hipLaunchKernelGGL(renum_short_kernel<IdxT>, dim3(grid_for((uint64_t)n.nshort * WAVE)), dim3(BLOCK), 0, s, a,
+                           n.nlong + n.nmid, n.nshort);
     return hipGetLastError();
 }
 
