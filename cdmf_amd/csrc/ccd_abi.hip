@@ -371,14 +371,13 @@ int upload_layout(ccd_ctx* c, DevLayout& L, int64_t rows, int64_t gdim, uint64_t
     L.split_cap = 0;
     L.hptr.resize((size_t)rows + 1);
     L.hptr[0] = 0;
-    ccd::RenumRows cls{0, 0, 0, 0};
+    ccd::RenumRows cls{0, 0, 0};
     const uint32_t long_len = ccd::renum_long_len((uint32_t)gdim);
     for (int64_t i = 0; i < rows; ++i) {
         const uint32_t len = cptr[perm[i] + 1] - cptr[perm[i]];
         L.hptr[i + 1] = L.hptr[i] + len;
         if (len > long_len) {
             ++cls.nlong;
-            cls.long_elems = L.hptr[i + 1];
         } else if (len > ccd::RENUM_SHORT) {
             ++cls.nmid;
         } else if (len) {

@@ -38,7 +38,6 @@ constexpr uint32_t RENUM_SHORT = 64;
 uint32_t renum_long_len(uint32_t gdim);
 struct RenumRows {
     uint32_t nlong, nmid, nshort;
-    uint32_t long_elems;  // elements of the long rows (they come first)
 };
 // dup: nlong + 1 words of scratch
 hipError_t launch_renumber(const RenumArgs& a, bool idx16, const RenumRows& n, uint32_t* dup, hipStream_t s);
