@@ -150,7 +150,7 @@ __global__ __launch_bounds__(BS) void renum_long_kernel(RenumArgs a, uint32_t* _
         const uint32_t lo = (uint32_t)w0;
         for (uint32_t q = threadIdx.x; q < words; q += BS) bits[q] = 0u;
         __syncthreads();
-        for (uint32_t p = threadIdx.x; p < len; p += BS) {
+        for (uint64_t p = threadIdx.x; p < len; p += BS) {  // 64 bits: len + BS may pass 2^32
             const uint32_t k = a.ipos[a.idx[e0 + p]] - lo;  // wraps past the window for smaller indices
             if (k < words * 32) {
                 const uint32_t bit = 1u << (k & 31u);
@@ -180,13 +180,13 @@ __global__ __launch_bounds__(BS) void renum_long_kernel(RenumArgs a, uint32_t* _
         }
         for (uint32_t g = threadIdx.x * per; g < min(ng, (threadIdx.x + 1) * per); ++g) pre[g] += off;
         __syncthreads();
-        for (uint32_t p = threadIdx.x; p < len; p += BS) {
+        for (uint64_t p = threadIdx.x; p < len; p += BS) {
             const uint32_t key = a.ipos[a.idx[e0 + p]], k = key - lo;
             if (k >= words * 32) continue;
             const uint32_t w = k >> 5;
             uint32_t rank = below + pre[w / GROUP] + (uint32_t)__popc(bits[w] & ((1u << (k & 31u)) - 1u));
             for (uint32_t u = w / GROUP * GROUP; u < w; ++u) rank += (uint32_t)__popc(bits[u]);
-            put<IdxT>(a, o + rank, key, e0 + p);
+            put<IdxT>(a, o + rank, key, e0 + (uint32_t)p);
         }
         below += total;
         __syncthreads();
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(BLOCK) void split_positions_kernel(const uint32_t* 
             const uint32_t r = cold_row[v - nreal];
             src = lptr[r] + below[r];
         }
-        for (uint32_t q = threadIdx.x; q < len; q += BLOCK) vpos[v0 + q] = src + q;
+        for (uint64_t q = threadIdx.x; q < len; q += BLOCK) vpos[v0 + q] = src + (uint32_t)q;
     }
 }
 
