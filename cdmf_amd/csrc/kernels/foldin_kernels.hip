@@ -9,6 +9,8 @@
 // the others.  Per-row sums are reduced in a fixed order: deterministic.
 #include "ccd_kernels.h"
 
+#include <algorithm>
+
 namespace ccd {
 
 // old with lane `lane` (constant) replaced by the uniform x: the compiler's
@@ -224,10 +226,11 @@ __device__ __forceinline__ void gram_store(const f64x4 (&acc)[P], double* G, uin
 // G (k x k, rows of 16 NT) and b (k) in LDS of the ratings s .. s + d - 1, by the NW waves of
 // the block: wave wv takes chunks wv, wv + NW, ... of 64 ratings, and the
 // waves' sums are added in wave order.  Ends with every wave's part stored
-// (the caller synchronises).
-template <int NT, int NW, int P0 = 0>
+// (the caller synchronises).  P0, P1: the tile pairs to form (b comes with
+// pair 0).
+template <int NT, int NW, int P0 = 0, int P1 = pair_count(NT)>
 __device__ __forceinline__ void gram(const FoldArgs& a, uint32_t s, uint32_t d, double* G, double* b) {
-    constexpr int PALL = pair_count(NT), P = PALL - P0 < GRAM_PAIRS ? PALL - P0 : GRAM_PAIRS;
+    constexpr int P = P1 - P0 < GRAM_PAIRS ? P1 - P0 : GRAM_PAIRS;
     const int lane = threadIdx.x & (WAVE - 1);
     const uint32_t wv = NW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const uint32_t k = a.k, sub = lane / 16, col = lane % 16;
@@ -286,7 +289,17 @@ __device__ __forceinline__ void gram(const FoldArgs& a, uint32_t s, uint32_t d, 
         }
         if (NW > 1) __syncthreads();
     }
-    if constexpr (P0 + P < PALL) gram<NT, NW, P0 + P>(a, s, d, G, b);
+    if constexpr (P0 + P < P1) gram<NT, NW, P0 + P, P1>(a, s, d, G, b);
+}
+
+// The same by SW waves that share the tile pairs, each over all ratings (the
+// sums are those of one wave).
+template <int NT, int SW, int W = 0>
+__device__ __forceinline__ void gram_by_pairs(const FoldArgs& a, uint32_t s, uint32_t d, double* G, double* b,
+                                              uint32_t wv) {
+    constexpr int PALL = pair_count(NT), PER = (PALL + SW - 1) / SW;
+    if (wv == (uint32_t)W) gram<NT, 1, PER * W, (PER * W + PER < PALL ? PER * W + PER : PALL)>(a, s, d, G, b);
+    else if constexpr (W + 1 < SW) gram_by_pairs<NT, SW, W + 1>(a, s, d, G, b, wv);
 }
 
 __device__ __forceinline__ double lane_value(double v, int lane) {
@@ -337,46 +350,59 @@ __device__ __forceinline__ void fold_chain(const double* m, uint32_t groups, con
     if constexpr (Q + 1 < WAVE / CHAIN) fold_chain<NS, J, LD, Q + 1>(m, groups, gn, e, cap);
 }
 
-// The sweeps of one row from its G and b in LDS, by one wave: lane l holds
-// ranks l and, for k > 64 (NS = 2), l + 64.  Column s of G is only touched by
+// The sweeps of one row from its G and b in LDS, by the first of the SW waves
+// that call (the others help to scale G): lane l holds ranks l and, for k >
+// 64 (NS = 2), l + 64.  Column s of G is only touched by
 // rank s's lane, which scales it in place.  The chain runs in whole groups:
 // columns k .. of G, which the products leave unwritten, and rows k .. up to
 // a multiple of CHAIN are cleared, so the ranks there stay zero.
-template <int NS, int LD>
+template <int NS, int LD, int SW = 1>
 __device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint32_t d, double* G, const double* b,
                                            const float* __restrict__ W0, float* __restrict__ W) {
     const uint32_t lane = threadIdx.x & (WAVE - 1), k = a.k;
+    const uint32_t wv = SW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const double lamd = (double)(a.lambda * (float)d);
-    double e[NS], w[NS];
+    double e[NS], w[NS], scale[NS];
     const double* base = G + (lane < (uint32_t)LD ? lane : 0u);  // lanes past the matrix read column 0, times 0
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
         const uint32_t s = lane + WAVE * j;
-        double scale = 0.0;
         e[j] = 0.0;
         w[j] = 0.0;
+        scale[j] = 0.0;
         if (s < k) {
             double* col = G + s;
-            w[j] = W0 ? (double)W0[(size_t)row * k + s] : 0.0;
-            const double inv = 1.0 / (lamd + col[s * LD]);
-            double p = b[s];
-            if (W0) {  // the numerator leaves the rank's own term out
-                for (uint32_t u = 0; u < k; ++u) {
-                    const double wu = (double)W0[(size_t)row * k + u];
-                    if (u != s) p = __builtin_fma(-col[u * LD], wu, p);
+            scale[j] = 1.0 / (lamd + col[s * LD]);
+            if (wv == 0) {
+                w[j] = W0 ? (double)W0[(size_t)row * k + s] : 0.0;
+                double p = b[s];
+                if (W0) {  // the numerator leaves the rank's own term out
+                    for (uint32_t u = 0; u < k; ++u) {
+                        const double wu = (double)W0[(size_t)row * k + u];
+                        if (u != s) p = __builtin_fma(-col[u * LD], wu, p);
+                    }
                 }
+                e[j] = __builtin_fma(p, scale[j], -w[j]);
             }
-            e[j] = __builtin_fma(p, inv, -w[j]);
-            scale = inv;
         }
+    }
+    if (SW > 1) __syncthreads();  // the diagonal and the numerators are read
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+        const uint32_t s = lane + WAVE * j;
         if (s < (uint32_t)LD) {
 #pragma unroll 4
-            for (uint32_t u = 0; u < k; ++u) {
-                const double v = G[u * LD + s] * scale;
+            for (uint32_t u = wv; u < k; u += SW) {
+                const double v = G[u * LD + s] * scale[j];
                 G[u * LD + s] = s >= k ? 0.0 : u == s ? 1.0 : v;
             }
-            for (uint32_t u = k; u % CHAIN; ++u) G[u * LD + s] = 0.0;
+            if (wv == 0)
+                for (uint32_t u = k; u % CHAIN; ++u) G[u * LD + s] = 0.0;
         }
+    }
+    if (SW > 1) {
+        __syncthreads();
+        if (wv) return;
     }
     // one wave: its LDS writes above come before its reads below
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -426,23 +452,34 @@ __global__ __launch_bounds__(FOLD_LWAVES* WAVE) void fold_sweep_long_kernel(Fold
     fold_solve<(NT > 4 ? 2 : 1), 16 * NT>(a, row, d, fold_lds, b, W0, W);
 }
 
-// The other rows, one single-wave block each.
+// The other rows, one block each: a single wave up to k = 64.  Past that the
+// matrix (46 to 131 KB) leaves a CU room for three rows down to one, so four
+// waves, or from k = 97 one for each 16 ranks, share a row's products and
+// scaling.  With one wave a sweep or two over short rows took longer than
+// over the row's residual: 48,019 rows of 5 ratings, k = 128, one sweep 4.8
+// ms (residual 2.5, now 2.0); of 100 ratings, k = 100, 8.6 (3.0, 2.9), k =
+// 65, 2.05 (1.97, 1.23).
+constexpr int short_waves(int nt) { return nt > 6 ? nt : nt > 4 ? 4 : 1; }
 template <int NT>
-__global__ __launch_bounds__(WAVE) void fold_sweep_short_kernel(FoldArgs a, const float* __restrict__ W0,
-                                                                float* __restrict__ W) {
+__global__ __launch_bounds__(short_waves(NT)* WAVE) void fold_sweep_short_kernel(FoldArgs a,
+                                                                                const float* __restrict__ W0,
+                                                                                float* __restrict__ W) {
+    constexpr int SW = short_waves(NT);
     extern __shared__ __align__(16) double fold_lds[];
     double* b = fold_lds + fold_matrix(NT, a.k);
-    const uint32_t row = blockIdx.x;
+    const uint32_t row = blockIdx.y * gridDim.x + blockIdx.x;
+    if (row >= a.rows) return;
     const uint32_t s = a.ptr[row], d = a.ptr[row + 1] - s;
     if (d > FOLD_WAVE) return;
     if (d == 0 || a.sweeps == 0) {  // nothing to solve: 0 after a sweep, the start before one
-        for (uint32_t t = threadIdx.x; t < a.k; t += WAVE)
+        for (uint32_t t = threadIdx.x; t < a.k; t += SW * WAVE)
             W[(size_t)row * a.k + t] = a.sweeps == 0 && W0 ? W0[(size_t)row * a.k + t] : 0.0f;
         return;
     }
-    gram<NT, 1>(a, s, d, fold_lds, b);
-    __syncthreads();  // one wave: orders its LDS writes and reads
-    fold_solve<(NT > 4 ? 2 : 1), 16 * NT>(a, row, d, fold_lds, b, W0, W);
+    const uint32_t wv = SW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    gram_by_pairs<NT, SW>(a, s, d, fold_lds, b, wv);
+    __syncthreads();
+    fold_solve<(NT > 4 ? 2 : 1), 16 * NT, SW>(a, row, d, fold_lds, b, W0, W);
 }
 
 template <int NT>
@@ -452,8 +489,11 @@ hipError_t launch_sweeps_nt(const FoldArgs& a, const uint32_t* long_rows, uint32
     if (nlong)
         hipLaunchKernelGGL(fold_sweep_long_kernel<NT>, dim3(nlong), dim3(FOLD_LWAVES * WAVE), lds, s, a, long_rows, W0,
                            W);
-    if (nlong < a.rows)
-        hipLaunchKernelGGL(fold_sweep_short_kernel<NT>, dim3(a.rows), dim3(WAVE), lds, s, a, W0, W);
+    if (nlong < a.rows) {
+        const uint32_t x = std::min(a.rows, 1u << 20);  // a launch takes less than 2^32 threads along x
+        hipLaunchKernelGGL(fold_sweep_short_kernel<NT>, dim3(x, (a.rows + x - 1) / x), dim3(short_waves(NT) * WAVE), lds,
+                           s, a, W0, W);
+    }
     return hipGetLastError();
 }
 

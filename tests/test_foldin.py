@@ -297,3 +297,22 @@ def test_mlp_gemm_shapes(oracle_lib, dims, rows):
         f = np.linalg.norm(Y - ref) / np.linalg.norm(ref)
         assert f <= bar, "forward mode %d: %.3g" % (mode, f)
     mlp.close()
+
+
+@pytest.mark.parametrize("k", [3, 65])
+def test_fold_rows_past_one_grid_row(k):
+    """More rows than one row of the sweeps' grid (2^20): the rows at its end
+    and past it.  Bound as in test_fold_rows_normal_equations."""
+    F = _gpu()
+    rows, n = (1 << 20) + 5, 300
+    rng = np.random.default_rng(k)
+    ptr = np.arange(rows + 1, dtype=np.uint32)
+    idx = rng.integers(0, n, rows).astype(np.uint32)
+    val = rng.integers(1, 6, rows).astype(np.float32)
+    H = rng.normal(0.1, 0.4, (k, n)).astype(np.float32)
+    fold = F.FoldIn(H, 0.05)
+    W, _ = fold.rows(ptr, idx, val, 2)
+    fold.close()
+    sel = np.r_[0:3, (1 << 20) - 3:rows]
+    ref = _fold_f64(np.arange(sel.size + 1, dtype=np.uint32), idx[sel], val[sel], H, 0.05, 2, None)
+    np.testing.assert_allclose(W[sel], ref, rtol=6.1e-8, atol=1e-9 * float(np.abs(ref).max()))
