@@ -114,20 +114,26 @@ private:
         return p < (512u << 10) ? 512u << 10 : p < PIECE ? p : PIECE;
     }
 
+    // false: the runtime's copies are taken instead, and the error that
+    // hipGetLastError would report after the next launch is cleared.
     bool ready() {
         if (buf_) return true;
         for (hipEvent_t& e : ev_)
             if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
                 e = nullptr;
-                release();
-                return false;
+                return give_up();
             }
         if (hipHostMalloc(reinterpret_cast<void**>(&buf_), WORKERS * SLOTS * PIECE, hipHostMallocDefault) != hipSuccess) {
             buf_ = nullptr;
-            release();
-            return false;
+            return give_up();
         }
         return true;
+    }
+
+    bool give_up() {
+        release();
+        (void)hipGetLastError();
+        return false;
     }
 
     // The calling thread is worker 0; pieces are taken from a shared counter,

@@ -59,3 +59,22 @@ def test_two_threads_two_objects():
         t.join()
     for i in range(2):
         assert np.array_equal(out[i][0], out["alone"][0]) and np.array_equal(out[i][1], out["alone"][1])
+
+
+@pytest.mark.parametrize("entries", [3 * MB - 1, 3 * MB, 3 * MB + 1, 8 * MB + 1, 9 * MB + 12345])
+def test_factors_come_back_as_given(entries):
+    """What comes back is what was handed over, on calls that reuse the pinned
+    pieces: sizes with a partial last piece and more pieces than slots."""
+    from cdmf_amd import datadir
+    from cdmf_amd import solver as S
+    ds = datadir.from_triplets(entries, 2, (np.array([0, entries - 1]), np.array([0, 1]), np.ones(2)),
+                               (np.array([0]), np.array([0]), np.ones(1)))
+    r = np.random.default_rng(entries)
+    with S.Solver(0) as s:
+        s.upload(ds, with_test=False)
+        for _ in range(3):
+            W = r.standard_normal((1, entries), dtype=np.float32)
+            given = W.copy()
+            s.set_factors(W, np.ones((1, 2), np.float32))
+            W[:] = 0.0  # the call is done with the caller's array
+            assert np.array_equal(s.factors()[0], given)
