@@ -363,7 +363,13 @@ __device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint
     const uint32_t wv = SW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const double lamd = (double)(a.lambda * (float)d);
     double e[NS], w[NS], scale[NS];
-    const double* base = G + (lane < (uint32_t)LD ? lane : 0u);  // lanes past the matrix read column 0, times 0
+    // Lanes past the matrix hold no rank: their e is never read by a step nor
+    // stored, so what the chain gathers for them does not matter, only that
+    // it lies in the block's LDS.  With one slot they read column 0; a second
+    // slot of lanes from LD - 64 on reads past its row, in the last row up to
+    // 128 - LD entries into b.
+    static_assert(NS == 1 || WAVE * NS - LD <= LD - 15, "b has more than LD - 16 entries");
+    const double* base = G + (lane < (uint32_t)LD ? lane : 0u);
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
         const uint32_t s = lane + WAVE * j;
