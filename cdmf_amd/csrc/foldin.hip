@@ -381,7 +381,10 @@ int32_t ccd_mlp_forward(ccd_mlp* m, uint64_t rows, const float* X, float* Y, int
     OBJ_TRY(m, ensure(&m->X, &m->cap_x, rows * m->in));
     OBJ_TRY(m, ensure(&m->T, &m->cap_t, rows * m->out));
     OBJ_TRY(m, m->pipe.in(m->device, m->X, X, 4 * rows * m->in, m->stream));
-    if (int rc = mlp_forward_dev(m, rows, m->X, m->T, bf16_weights, m->stream)) return rc;
+    if (int rc = mlp_forward_dev(m, rows, m->X, m->T, bf16_weights, m->stream)) {
+        (void)hipStreamSynchronize(m->stream);  // the rows may still be on their way out of the caller's array
+        return rc;
+    }
     OBJ_TRY(m, m->pipe.out(m->device, Y, m->T, 4 * rows * m->out, m->stream));
     return CCD_OK;
 }
@@ -739,9 +742,15 @@ int32_t ccd_fold_warm(ccd_fold* f, ccd_mlp* m, int64_t rows, const uint32_t* ptr
     OBJ_TRY(f, hipStreamSynchronize(m->stream));
     OBJ_TRY(f, hipEventRecord(f->ea, f->stream));
     OBJ_TRY(f, ccd::launch_fold_features(a, f->long_rows, f->nfeat, f->F, f->stream));
-    if (bf16_weights < 0 || bf16_weights > 2) return obj_err(f->err, CCD_ERR_INVALID, "bf16_weights must be 0, 1 or 2");
-    if (int rc = mlp_forward_dev(m, (uint64_t)rows, f->F, f->W0, bf16_weights, f->stream))
-        return obj_err(f->err, rc, "MLP: " + m->err);
+    int rc = CCD_OK;
+    if (bf16_weights < 0 || bf16_weights > 2)
+        rc = obj_err(f->err, CCD_ERR_INVALID, "bf16_weights must be 0, 1 or 2");
+    else if ((rc = mlp_forward_dev(m, (uint64_t)rows, f->F, f->W0, bf16_weights, f->stream)))
+        rc = obj_err(f->err, rc, "MLP: " + m->err);
+    if (rc) {  // refused: the batch may still be on its way out of the caller's arrays
+        (void)hipStreamSynchronize(f->stream);
+        return rc;
+    }
     OBJ_TRY(f, ccd::launch_fold_sweeps(a, f->long_rows, f->nlong, f->W0, f->W, f->stream));
     OBJ_TRY(f, hipEventRecord(f->eb, f->stream));
     OBJ_TRY(f, hipEventSynchronize(f->eb));

@@ -316,3 +316,34 @@ def test_fold_rows_past_one_grid_row(k):
     sel = np.r_[0:3, (1 << 20) - 3:rows]
     ref = _fold_f64(np.arange(sel.size + 1, dtype=np.uint32), idx[sel], val[sel], H, 0.05, 2, None)
     np.testing.assert_allclose(W[sel], ref, rtol=6.1e-8, atol=1e-9 * float(np.abs(ref).max()))
+
+
+def test_warm_refused_after_the_upload():
+    """A network or a mode that is refused once the batch is on its way: the
+    caller may reuse its arrays at once, and the next call is right."""
+    import torch
+
+    from cdmf_amd.solver import CCDError
+    F = _gpu()
+    rng = np.random.default_rng(3)
+    k, n, rows = 8, 500, 300
+    ptr = (np.arange(rows + 1) * 20).astype(np.uint32)
+    idx = rng.integers(0, n, rows * 20).astype(np.uint32)
+    val = torch.empty(rows * 20, pin_memory=True).numpy()  # memory the device reads in place
+    want_val = rng.integers(1, 6, rows * 20).astype(np.float32)
+    H = rng.normal(0.1, 0.4, (k, n)).astype(np.float32)
+    fold, narrow, wide = F.FoldIn(H, 0.05), F.MLP(2 * k + 2, 64, k, seed=1), F.MLP(2 * k + 2, 256, k, seed=1)
+    val[:] = want_val
+    want, _ = fold.warm(wide, ptr, idx, val, 2, bf16=2)
+    for mlp, mode in ((narrow, 2), (wide, 3), (wide, -1)):
+        val[:] = want_val
+        with pytest.raises(CCDError):
+            fold.warm(mlp, ptr, idx, val, 2, bf16=mode)
+        val[:] = -1.0
+        with pytest.raises(CCDError):
+            mlp.forward(np.zeros((100, 2 * k + 2), np.float32), bf16=mode)
+    val[:] = want_val
+    got, _ = fold.warm(wide, ptr, idx, val, 2, bf16=2)
+    assert np.array_equal(got, want)
+    for x in (fold, narrow, wide):
+        x.close()
