@@ -270,3 +270,23 @@ def test_batch_solo_problems_bitwise(solo):
             _same(g, _single(S, ds, k, lam, outer, inner, order, W0, H0, 16), "%s (solo=%d, graph=%s)" % (
                 name, solo, graph))
         b.close()
+
+
+@pytest.mark.parametrize("sigma", [16, 8])
+@pytest.mark.parametrize("inner", [7, 8, 9, 16, 17, 25])
+def test_batch_more_inner_iterations_than_buffers(inner, sigma):
+    """The rotating buffers of a rank (8) used up exactly, and coming round
+    once, twice and a third time: bitwise equal to the single-problem runs,
+    for teams of many blocks and of one, with spanning rows and without."""
+    S = _solver()
+    cases = [(name, ds, min(k, 3), lam, 2, inner, order, W0[:3], H0[:3])
+             for name, ds, k, lam, _, _, order, W0, H0 in _cases()]
+    b, solvers = _build(S, cases, sigma)
+    b.run()
+    _say("teams %s" % b.teams())
+    got = _batch_results(solvers)
+    for (name, ds, k, lam, outer, inn, order, W0, H0), g in zip(cases, got):
+        _say("compare %s" % name)
+        assert np.all(np.isfinite(g[0])) and np.any(g[0] != 0)
+        _same(g, _single(S, ds, k, lam, outer, inn, order, W0, H0, sigma), name)
+    b.close()
