@@ -93,3 +93,37 @@ def test_other_precisions_match_oracle(precision, sigma):
         W, H = s.factors()
     tol = {0: 1e-4, 2: 2e-5}[precision]
     assert np.linalg.norm(W - Wo) <= tol * np.linalg.norm(Wo) and np.linalg.norm(H - Ho) <= tol * np.linalg.norm(Ho)
+
+
+@pytest.mark.parametrize("name", ["two_tiles", "spans_252", "long_32", "wide_8192"])
+@pytest.mark.parametrize("precision,sigma", [(1, 16), (2, 16), (0, 8), (0, 16), (0, 32)])
+def test_merged_equals_finished_by_its_own_launch(name, precision, sigma):
+    """The same matrix with empty rows and columns added until both gathered
+    vectors are past the bound of the merge: the same tiles, each sweep's
+    spanning rows finished by a launch of their own.  Every precision, bit
+    for bit (with bfloat16 storage the merged rows are rounded as stored
+    ones are)."""
+    import dataclasses
+
+    from cdmf_amd import data as D
+    from cdmf_amd import solver as S
+    ds = CASES[name]()
+    k, lam, outer, inner = 2, 0.05, 2, 3
+    m2, n2 = max(ds.m, 8300), max(ds.n, 8300)
+    pad = lambda p, size: np.concatenate([p, np.full(size + 1 - p.size, p[-1], p.dtype)])
+    wide = dataclasses.replace(ds, m=m2, n=n2, csr_ptr=pad(ds.csr_ptr, m2), csc_ptr=pad(ds.csc_ptr, n2))
+    W0 = D.initial_col(k, ds.m)
+    out = []
+    for one in (ds, wide):
+        W1 = np.zeros((k, one.m), np.float32)
+        W1[:, :ds.m] = W0
+        with S.Solver(0) as s:
+            s.set_plan(sigma=sigma, split_rows=0)
+            s.upload(one, with_test=False)
+            s.set_factors(W1, np.zeros((k, one.n), np.float32))
+            s.run(k, lam, outer, inner, variant=S.VARIANT_TILED, precision=precision)
+            W, H = s.factors()
+            out.append((W[:, :ds.m], H[:, :ds.n], *s.residual()))
+    assert np.all(np.isfinite(out[0][0])) and np.any(out[0][0] != 0)
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
