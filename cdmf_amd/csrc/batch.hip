@@ -110,6 +110,18 @@ ccd::BatchLayout batch_layout(const ccdi::DevLayout& L) {
     return d;
 }
 
+// The contexts still hold what ccd_batch_add saw: a matrix, and factors of
+// its shape and of at least the problem's rank.
+int check_contexts(ccd_batch* b) {
+    for (size_t i = 0; i < b->items.size(); ++i) {
+        const ccd_ctx* c = b->items[i].ctx;
+        if (!c->uploaded || !c->factors || c->k < b->items[i].p.k)
+            return berr(b, CCD_ERR_STATE, "problem " + std::to_string(i) +
+                                              ": its context was uploaded again without ccd_set_factors of its k");
+    }
+    return CCD_OK;
+}
+
 // Tiled layouts of every problem for sigma, pair buffers, FP32 state.
 int prepare(ccd_batch* b, int sigma) {
     for (size_t i : b->active) {
@@ -552,6 +564,7 @@ extern "C" {
 int32_t ccd_batch_tune(ccd_batch* b, double* best_ms) {
     if (!b) return CCD_ERR_INVALID;
     if (b->items.empty()) return berr(b, CCD_ERR_STATE, "empty batch");
+    if (int rc = check_contexts(b)) return rc;
     BATCH_TRY(b, hipSetDevice(b->device));
     ccd_batch_plan best = b->plan;
     double bms = INFINITY;
@@ -635,6 +648,7 @@ int32_t ccd_batch_tune(ccd_batch* b, double* best_ms) {
 int32_t ccd_batch_run(ccd_batch* b, int32_t use_graph) {
     if (!b) return CCD_ERR_INVALID;
     if (b->items.empty()) return berr(b, CCD_ERR_STATE, "empty batch");
+    if (int rc = check_contexts(b)) return rc;
     BATCH_TRY(b, hipSetDevice(b->device));
     const int sigma = (int)b->plan.sigma;
     for (size_t i = 0; i < b->items.size(); ++i)

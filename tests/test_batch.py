@@ -290,3 +290,30 @@ def test_batch_more_inner_iterations_than_buffers(inner, sigma):
         assert np.all(np.isfinite(g[0])) and np.any(g[0] != 0)
         _same(g, _single(S, ds, k, lam, outer, inn, order, W0, H0, sigma), name)
     b.close()
+
+
+def test_batch_refuses_a_context_without_its_factors():
+    """A matrix uploaded again after ccd_batch_add: refused until factors of
+    the new shape and the problem's rank are set, then solved."""
+    S = _solver()
+    from cdmf_amd import data as D
+    small, large = D.gen_uniform(300, 200, 3000, 300, seed=13), D.gen_uniform(900, 700, 9000, 300, seed=14)
+    fac = lambda ds, k: (D.initial_col(k, ds.m), np.zeros((k, ds.n), np.float32))
+    with S.Solver(0) as s:
+        s.upload(small)
+        s.set_factors(*fac(small, 4))
+        b = S.Batch(0)
+        b.set_plan(sigma=16)
+        b.add(s, 4, 0.05, 2, 2, zero_first=False)
+        s.upload(large)
+        for call in (b.run, b.tune):
+            with pytest.raises(S.CCDError, match="ccd_set_factors"):
+                call()
+        s.set_factors(*fac(large, 3))
+        with pytest.raises(S.CCDError, match="ccd_set_factors"):
+            b.run()
+        s.set_factors(*fac(large, 4))
+        b.run()
+        got = _batch_results([s])[0]
+        b.close()
+    _same(got, _single(S, large, 4, 0.05, 2, 2, S.ORDER_H_FIRST, *fac(large, 4), 16), "the new matrix")
