@@ -17,8 +17,9 @@ namespace ccd {
 // besides its bytes: 31 GB/s with pieces of 1 MB).  Below the bounds starting
 // the threads costs what they save, and the runtime's path is taken.  One
 // pipe belongs to one object and is used by one thread at a time, as the
-// object is; it holds 32 MB of pinned memory and eight events from its first
-// large copy until release().
+// object is.  From its first large copy until release() it holds eight events
+// and eight pinned pieces as large as its largest copy asked for: 4 MB after
+// a copy of 2 MB, 32 MB after one of more than 16.
 class HostPipe {
 public:
     static constexpr size_t BIG_IN = 12u << 20, BIG_OUT = 2u << 20;
@@ -36,20 +37,21 @@ public:
         }
         if (buf_) (void)hipHostFree(buf_);
         buf_ = nullptr;
+        slot_ = 0;
     }
 
     // dst (device) = src (host), ordered on stream s; src may change once it
     // returns for large copies, and once s has been waited for otherwise.
     hipError_t in(int device, void* dst, const void* src, size_t bytes, hipStream_t s) {
         if (bytes == 0) return hipSuccess;
-        if (bytes < BIG_IN || !ready()) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
         const size_t piece = piece_of(bytes);
+        if (bytes < BIG_IN || !ready(piece)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
         return run(device, bytes, [&](int w, std::atomic<size_t>& next) -> hipError_t {
             int n = 0;
             for (size_t c; (c = next.fetch_add(piece)) < bytes; ++n) {
                 const int q = w * SLOTS + n % SLOTS;
                 const size_t len = bytes - c < piece ? bytes - c : piece;
-                char* p = buf_ + (size_t)q * PIECE;
+                char* p = buf_ + (size_t)q * slot_;
                 hipError_t e = hipEventSynchronize(ev_[q]);  // the piece last sent from here (none: returns at once)
                 if (e != hipSuccess) return e;
                 std::memcpy(p, static_cast<const char*>(src) + c, len);
@@ -64,12 +66,12 @@ public:
     // dst (host) = src (device) after the work on stream s; complete on return.
     hipError_t out(int device, void* dst, const void* src, size_t bytes, hipStream_t s) {
         if (bytes == 0) return hipStreamSynchronize(s);
-        if (bytes < BIG_OUT || !ready()) {
+        const size_t piece = piece_of(bytes);
+        if (bytes < BIG_OUT || !ready(piece)) {
             const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
             const hipError_t w = hipStreamSynchronize(s);
             return e != hipSuccess ? e : w;
         }
-        const size_t piece = piece_of(bytes);
         return run(device, bytes, [&](int w, std::atomic<size_t>& next) -> hipError_t {
             size_t at[SLOTS], len[SLOTS];
             auto fetch = [&](int q, bool& got) -> hipError_t {
@@ -80,7 +82,7 @@ public:
                 const int x = w * SLOTS + q;
                 hipError_t e = hipEventSynchronize(ev_[x]);
                 if (e == hipSuccess)
-                    e = hipMemcpyAsync(buf_ + (size_t)x * PIECE, static_cast<const char*>(src) + at[q], len[q],
+                    e = hipMemcpyAsync(buf_ + (size_t)x * slot_, static_cast<const char*>(src) + at[q], len[q],
                                        hipMemcpyDeviceToHost, s);
                 if (e == hipSuccess) e = hipEventRecord(ev_[x], s);
                 return e;
@@ -94,7 +96,7 @@ public:
                 const int x = w * SLOTS + q;
                 hipError_t e = hipEventSynchronize(ev_[x]);
                 if (e != hipSuccess) return e;
-                std::memcpy(static_cast<char*>(dst) + at[q], buf_ + (size_t)x * PIECE, len[q]);
+                std::memcpy(static_cast<char*>(dst) + at[q], buf_ + (size_t)x * slot_, len[q]);
                 e = fetch(q, got[q]);
                 if (e != hipSuccess) return e;
             }
@@ -106,6 +108,7 @@ private:
     static constexpr int WORKERS = 4, SLOTS = 2;
     static constexpr size_t PIECE = 4u << 20;  // largest
     char* buf_ = nullptr;
+    size_t slot_ = 0;  // bytes of a pinned piece
     hipEvent_t ev_[WORKERS * SLOTS] = {};
 
     // every worker two pieces, within 512 KB and 4 MB
@@ -114,16 +117,23 @@ private:
         return p < (512u << 10) ? 512u << 10 : p < PIECE ? p : PIECE;
     }
 
-    // false: the runtime's copies are taken instead, and the error that
-    // hipGetLastError would report after the next launch is cleared.
-    bool ready() {
-        if (buf_) return true;
-        for (hipEvent_t& e : ev_)
-            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+    // Pinned pieces of at least `piece` bytes.  false: the runtime's copies
+    // are taken instead, and the error that hipGetLastError would report after
+    // the next launch is cleared.
+    bool ready(size_t piece) {
+        if (slot_ >= piece) return true;
+        for (hipEvent_t& e : ev_) {
+            if (e) {
+                if (hipEventSynchronize(e) != hipSuccess) return give_up();  // the smaller pieces are done with
+            } else if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
                 e = nullptr;
                 return give_up();
             }
-        if (hipHostMalloc(reinterpret_cast<void**>(&buf_), WORKERS * SLOTS * PIECE, hipHostMallocDefault) != hipSuccess) {
+        }
+        if (buf_) (void)hipHostFree(buf_);
+        slot_ = 512u << 10;
+        while (slot_ < piece) slot_ *= 2;
+        if (hipHostMalloc(reinterpret_cast<void**>(&buf_), WORKERS * SLOTS * slot_, hipHostMallocDefault) != hipSuccess) {
             buf_ = nullptr;
             return give_up();
         }

@@ -24,6 +24,7 @@ struct Op {
 std::deque<Op> queue;
 thread_local hipError_t last = hipSuccess;
 int events = 0, pinned = 0;       // alive
+size_t pinned_bytes = 0;          // of the last pinned allocation
 int fail_event = -1;              // the n-th event to create from now on fails
 bool fail_pinned = false;
 int fail_copy = -1;               // the n-th copy from now on fails
@@ -89,6 +90,7 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKin
 hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
     if (fail_pinned) return *p = nullptr, fail(hipErrorOutOfMemory);
     ++pinned;
+    pinned_bytes = bytes;
     *p = std::malloc(bytes);
     return hipSuccess;
 }
@@ -154,6 +156,28 @@ int main() {
         for (size_t n : {HostPipe::BIG_OUT, 13 * MB}) round_trip(p, n, ++seed);
     }
     check(events == 0 && pinned == 0, "what is left of a pipe", 0);
+    {  // as much as the largest copy asks for, grown while copies are still queued
+        HostPipe p;
+        round_trip(p, HostPipe::BIG_OUT, ++seed);
+        check(pinned == 1 && pinned_bytes == 4 * MB, "after a copy of", HostPipe::BIG_OUT);
+        const std::vector<unsigned char> a = bytes_of(13 * MB, ++seed), b = bytes_of(20 * MB, ++seed);
+        std::vector<unsigned char> src = a, src2 = b, da(a.size()), db(b.size());
+        check(p.in(0, da.data(), src.data(), a.size(), nullptr) == hipSuccess, "in", a.size());
+        std::memset(src.data(), 0, src.size());
+        check(pinned == 1 && pinned_bytes == 16 * MB, "after a copy of", a.size());
+        check(p.in(0, db.data(), src2.data(), b.size(), nullptr) == hipSuccess, "in", b.size());
+        std::memset(src2.data(), 0, src2.size());
+        check(pinned == 1 && pinned_bytes == 32 * MB, "after a copy of", b.size());
+        (void)hipStreamSynchronize(nullptr);
+        check(da == a && db == b, "copies about a growth", 0);
+        round_trip(p, HostPipe::BIG_OUT + 1, ++seed);
+        check(pinned == 1 && pinned_bytes == 32 * MB, "what stays", 0);
+        fail_pinned = true;
+        p.release();
+        round_trip(p, HostPipe::BIG_OUT, ++seed);
+        fail_pinned = false;
+    }
+    check(events == 0 && pinned == 0, "what is left of a grown pipe", 0);
     {  // no pinned memory, no events: the runtime's own copies, and no error for the next call to find
         HostPipe p;
         fail_pinned = true;
