@@ -26,6 +26,9 @@ void dfree(void* p) {
     if (p) (void)hipFree(p);
 }
 
+// Most device memory that rows on their way through a network leave behind.
+constexpr size_t KEEP_BYTES = (size_t)1 << 30;
+
 // Grow-only device buffer.
 template <class T>
 hipError_t ensure(T** p, size_t* cap, size_t count) {
@@ -379,13 +382,21 @@ int32_t ccd_mlp_forward(ccd_mlp* m, uint64_t rows, const float* X, float* Y, int
     if (bf16_weights < 0 || bf16_weights > 2) return obj_err(m->err, CCD_ERR_INVALID, "bf16_weights must be 0, 1 or 2");
     // the rows pass through the training set's buffers
     OBJ_TRY(m, ensure(&m->X, &m->cap_x, rows * m->in));
-    OBJ_TRY(m, ensure(&m->T, &m->cap_t, rows * m->out));
+    if (ensure(&m->T, &m->cap_t, rows * m->out) != hipSuccess) return obj_err(m->err, CCD_ERR_ALLOC, "output buffer");
     OBJ_TRY(m, m->pipe.in(m->device, m->X, X, 4 * rows * m->in, m->stream));
     if (int rc = mlp_forward_dev(m, rows, m->X, m->T, bf16_weights, m->stream)) {
         (void)hipStreamSynchronize(m->stream);  // the rows may still be on their way out of the caller's array
         return rc;
     }
     OBJ_TRY(m, m->pipe.out(m->device, Y, m->T, 4 * rows * m->out, m->stream));
+    // Kept for the next call, where allocating takes longer than a small
+    // call's kernels; a large call's copies dwarf it, and its memory goes back.
+    if (4 * (m->cap_x + m->cap_t) > KEEP_BYTES) {
+        dfree(m->X);
+        dfree(m->T);
+        m->X = m->T = nullptr;
+        m->cap_x = m->cap_t = 0;
+    }
     return CCD_OK;
 }
 

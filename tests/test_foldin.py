@@ -347,3 +347,22 @@ def test_warm_refused_after_the_upload():
     assert np.array_equal(got, want)
     for x in (fold, narrow, wide):
         x.close()
+
+
+def test_mlp_forward_gives_large_buffers_back():
+    """1.1 GB of rows and outputs: what the device has free after the call is
+    what it had before, and the rows are those of smaller calls."""
+    import torch
+    F = _gpu()
+    mlp = F.MLP(82, 256, 40, seed=2)
+    X = np.random.default_rng(1).standard_normal((1 << 16, 82), dtype=np.float32)
+    want = mlp.forward(X, bf16=2)
+    reps = 35  # 35 x 65,536 x 122 floats
+    big = np.concatenate([X] * reps)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    got = mlp.forward(big, bf16=2)
+    assert torch.cuda.mem_get_info()[0] >= before - (64 << 20)
+    assert all(np.array_equal(got[i << 16:(i + 1) << 16], want) for i in (0, 17, reps - 1))
+    assert np.array_equal(mlp.forward(X, bf16=2), want)
+    mlp.close()
