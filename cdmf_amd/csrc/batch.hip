@@ -54,6 +54,7 @@ struct ccd_batch {
 namespace {
 
 int berr(ccd_batch* b, int code, const std::string& msg) {
+    if (code == CCD_ERR_HIP || code == CCD_ERR_ALLOC) (void)hipGetLastError();  // as in set_err
     if (b) b->err = msg;
     return code;
 }
@@ -411,7 +412,7 @@ int32_t ccd_batch_create(int32_t device, ccd_batch** out) {
         hipEventCreate(&b->ev_a) != hipSuccess || hipEventCreate(&b->ev_b) != hipSuccess ||
         ccdi::dalloc(&b->d_status, 1) != hipSuccess || ccdi::dalloc(&b->d_tickets, 8 * 16) != hipSuccess) {
         delete b;
-        return CCD_ERR_HIP;
+        return berr(nullptr, CCD_ERR_HIP, "");
     }
     if (hipDeviceGetAttribute(&b->ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || b->ncu <= 0)
         b->ncu = 1;

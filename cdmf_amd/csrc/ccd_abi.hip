@@ -39,7 +39,10 @@
 
 namespace ccdi {
 
+// The runtime keeps a call's error until it is asked for, and a launch asks:
+// an error that is reported here must not fail the next call.
 int set_err(ccd_ctx* c, int code, const std::string& msg) {
+    if (code == CCD_ERR_HIP || code == CCD_ERR_ALLOC) (void)hipGetLastError();
     if (c) c->err = msg;
     return code;
 }
@@ -725,7 +728,7 @@ int32_t ccd_create(int32_t device, ccd_ctx** out) {
     c->device = device;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         delete c;
-        return CCD_ERR_HIP;
+        return set_err(nullptr, CCD_ERR_HIP, "");
     }
     int ncu = 0, lds_block = 0, lds_cu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || ncu <= 0) ncu = 256;
@@ -740,7 +743,7 @@ int32_t ccd_create(int32_t device, ccd_ctx** out) {
     if (dalloc(&c->rmse_bsum, ccd::RMSE_BLOCKS) != hipSuccess) {
         (void)hipStreamDestroy(c->stream);
         delete c;
-        return CCD_ERR_ALLOC;
+        return set_err(nullptr, CCD_ERR_ALLOC, "");
     }
     *out = c;
     return CCD_OK;

@@ -52,19 +52,19 @@ double uniform01(uint64_t& s) { return (double)(splitmix(s) >> 11) * (1.0 / 9007
 
 }  // namespace
 
-#define OBJ_TRY(o, expr)                                                                                  \
-    do {                                                                                                  \
-        hipError_t e_ = (expr);                                                                           \
-        if (e_ != hipSuccess) {                                                                           \
-            (o)->err = std::string(#expr) + ": " + hipGetErrorString(e_);                                 \
-            return CCD_ERR_HIP;                                                                           \
-        }                                                                                                 \
-    } while (0)
-
+// The runtime's own error is cleared: the next call's launches would find it.
 static int obj_err(std::string& err, int code, const std::string& msg) {
+    if (code == CCD_ERR_HIP || code == CCD_ERR_ALLOC) (void)hipGetLastError();
     err = msg;
     return code;
 }
+
+#define OBJ_TRY(o, expr)                                                                                     \
+    do {                                                                                                     \
+        hipError_t e_ = (expr);                                                                              \
+        if (e_ != hipSuccess)                                                                                \
+            return obj_err((o)->err, CCD_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));        \
+    } while (0)
 
 // ------------------------------------------------------------------ MLP ---
 struct ccd_mlp {
@@ -302,6 +302,7 @@ int32_t ccd_mlp_create(int32_t device, uint32_t in, uint32_t hidden, uint32_t ou
               hipStreamSynchronize(m->stream) == hipSuccess;
     if (!ok) {
         ccd_mlp_destroy(m);
+        (void)hipGetLastError();
         return CCD_ERR_HIP;
     }
     *mo = m;
@@ -636,6 +637,7 @@ int32_t ccd_fold_create(int32_t device, uint32_t k, int64_t n, const float* H, f
          hipStreamSynchronize(f->stream) == hipSuccess && scratch_on(device, &f->scratch) == hipSuccess;
     if (!ok) {
         ccd_fold_destroy(f);
+        (void)hipGetLastError();
         return CCD_ERR_HIP;
     }
     *fo = f;

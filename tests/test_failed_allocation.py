@@ -1,0 +1,48 @@
+"""A call that fails for want of device memory fails alone: the next call on
+the same thread, on that object or another, is right."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def test_the_next_call_is_right():
+    from cdmf_amd import data as D
+    from cdmf_amd import foldin as F
+    from cdmf_amd import solver as S
+    ds = D.gen_uniform(300, 200, 3000, 100, seed=1)
+    k = 4
+    W0, H0 = D.initial_col(k, ds.m), np.zeros((k, ds.n), np.float32)
+    ptr, idx, val = np.array([0, 3], np.uint32), np.array([1, 5, 9], np.uint32), np.ones(3, np.float32)
+
+    def solve(s):
+        s.upload(ds)
+        s.set_factors(W0, H0)
+        s.run(k, 0.05, 2, 2, variant=S.VARIANT_TILED)
+        return s.factors()
+
+    with S.Solver(0) as s, S.Solver(0) as other:
+        want = solve(other)
+        fold = F.FoldIn(want[1], 0.05)
+        want_row = fold.rows(ptr, idx, val, 2)[0]
+
+        def fail():
+            with pytest.raises(S.CCDError, match="memory"):
+                s.copy_probe(1 << 46)  # 64 TB
+
+        for who in (s, other):
+            fail()
+            got = solve(who)
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        fail()
+        assert np.array_equal(fold.rows(ptr, idx, val, 2)[0], want_row)
+        fail()
+        b = S.Batch(0)
+        s.set_factors(W0, H0)
+        b.add(s, k, 0.05, 2, 2)
+        b.run()
+        b.close()
+        fold.close()
+        fail()  # nothing is left behind for torch either
+        import torch
+        assert float(torch.ones(8, device="cuda").sum()) == 8.0
