@@ -892,6 +892,7 @@ int32_t ccd_set_factors(ccd_ctx* c, uint32_t k, const float* W, const float* H) 
         c->fmem = nullptr;
         c->W = c->H = c->fstage = nullptr;
         c->k = 0;
+        c->factors = false;
         Carver mem;
         mem.add(&c->W, (size_t)k * c->m);
         mem.add(&c->H, (size_t)k * c->n);

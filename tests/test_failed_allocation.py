@@ -46,3 +46,34 @@ def test_the_next_call_is_right():
         fail()  # nothing is left behind for torch either
         import torch
         assert float(torch.ones(8, device="cuda").sum()) == 8.0
+
+
+def test_factors_that_do_not_fit():
+    """ccd_set_factors of a rank too large for the device: the old factors are
+    gone, so what needs factors says so; new ones are taken as usual."""
+    import ctypes as C
+
+    from cdmf_amd import data as D
+    from cdmf_amd import datadir
+    from cdmf_amd import solver as S
+    m = n = 1 << 20
+    i = np.arange(2000) * 500
+    ds = datadir.from_triplets(m, n, (i, i[::-1].copy(), np.ones(i.size)), (i[:5], i[:5], np.ones(5)))
+    W0, H0 = D.initial_col(2, m), np.zeros((2, n), np.float32)
+    with S.Solver(0) as s:
+        s.upload(ds)
+        s.set_factors(W0, H0)
+        s.run(2, 0.05, 1, 1, variant=S.VARIANT_TILED)
+        want = s.factors()
+        one = np.zeros(1, np.float32)  # not read: 800 GB of factors are refused first
+        p = one.ctypes.data_as(C.POINTER(C.c_float))
+        with pytest.raises(S.CCDError, match="memory"):
+            s._check(s._lib.ccd_set_factors(s._ctx, 1 << 16, p, p))
+        for call in (s.factors, s.rmse, lambda: s.objective(0.1), lambda: s.run(2, 0.05, 1, 1),
+                     lambda: s.run(0, 0.05, 1, 1)):
+            with pytest.raises(S.CCDError, match="factors"):
+                call()
+        s.set_factors(W0, H0)
+        s.run(2, 0.05, 1, 1, variant=S.VARIANT_TILED)
+        got = s.factors()
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
