@@ -284,6 +284,7 @@ int describe(ccd_batch* b, int sigma, uint32_t blocks, const Split& sp, bool tri
         ccdi::dfree(b->d_barriers);
         b->d_probs = nullptr;
         b->d_barriers = nullptr;
+        b->cap_probs = 0;
         BATCH_TRY(b, ccdi::dalloc(&b->d_probs, np));
         BATCH_TRY(b, ccdi::dalloc(&b->d_barriers, np * ccd::BATCH_BARRIER_STRIDE));
         b->cap_probs = np;
@@ -291,6 +292,7 @@ int describe(ccd_batch* b, int sigma, uint32_t blocks, const Split& sp, bool tri
     if (blocks > b->cap_blocks) {
         ccdi::dfree(b->d_block_problem);
         b->d_block_problem = nullptr;
+        b->cap_blocks = 0;
         BATCH_TRY(b, ccdi::dalloc(&b->d_block_problem, blocks));
         b->cap_blocks = blocks;
     }

@@ -863,6 +863,7 @@ int32_t ccd_upload(ccd_ctx* c, int64_t m, int64_t n, uint64_t nnz, const uint32_
     }
     dfree(c->u);
     dfree(c->v);
+    c->u = c->v = nullptr;
     HIP_TRY(c, dalloc(&c->u, m));
     HIP_TRY(c, dalloc(&c->v, n));
     c->uploaded = true;
@@ -947,6 +948,7 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
             dfree(c->W16);
             dfree(c->H16);
             c->W16 = c->H16 = nullptr;
+            c->k16 = 0;
             HIP_TRY(c, dalloc(&c->W16, (size_t)k * c->m));
             HIP_TRY(c, dalloc(&c->H16, (size_t)k * c->n));
             c->k16 = k;
@@ -975,6 +977,7 @@ int32_t ccd_run(ccd_ctx* c, const ccd_params* p, ccd_iter_cb cb, void* user) {
     if (T > c->rmse_cap) {
         dfree(c->rmse_dev);
         c->rmse_dev = nullptr;
+        c->rmse_cap = 0;
         HIP_TRY(c, dalloc(&c->rmse_dev, T));
         c->rmse_cap = T;
     }

@@ -110,6 +110,7 @@ namespace {
 
 int mlp_workspace(ccd_mlp* m, size_t rows) {
     if (rows <= m->cap) return CCD_OK;
+    m->cap = 0;
     float** bufs_h[] = {&m->Z1, &m->A1, &m->Z2, &m->A2, &m->dZ2, &m->dZ1};
     for (float** b : bufs_h) {
         dfree(*b);

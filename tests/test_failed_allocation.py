@@ -77,3 +77,26 @@ def test_factors_that_do_not_fit():
         s.run(2, 0.05, 1, 1, variant=S.VARIANT_TILED)
         got = s.factors()
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+def test_a_workspace_that_does_not_fit():
+    """With the device nearly full, a training step whose workspace does not
+    fit fails part way through its allocation; a small one after it is right."""
+    import torch
+
+    from cdmf_amd import foldin as F
+    from cdmf_amd import solver as S
+    r = np.random.default_rng(1)
+    X, T = r.standard_normal((1 << 19, 34), dtype=np.float32), r.standard_normal((1 << 19, 16), dtype=np.float32)
+    mlp = F.MLP(34, 256, 16, seed=1)
+    want = mlp.loss_grad(X[:100], T[:100])
+    torch.cuda.synchronize()
+    # room for two or three of the six hidden-layer arrays of 512 MB
+    full = torch.empty(torch.cuda.mem_get_info()[0] - (1400 << 20), dtype=torch.uint8, device="cuda")
+    with pytest.raises(S.CCDError, match="memory"):
+        mlp.loss_grad(X, T)
+    got = mlp.loss_grad(X[:100], T[:100])
+    assert got[0] == want[0] and np.array_equal(got[1], want[1])
+    del full
+    torch.cuda.empty_cache()
+    mlp.close()
