@@ -363,6 +363,7 @@ __device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint
     const uint32_t wv = SW == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const double lamd = (double)(a.lambda * (float)d);
     double e[NS], w[NS], scale[NS];
+    bool lost = false;
     // Lanes past the matrix hold no rank: their e is never read by a step nor
     // stored, so what the chain gathers for them does not matter, only that
     // it lies in the block's LDS.  With one slot they read column 0; a second
@@ -378,7 +379,9 @@ __device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint
         scale[j] = 0.0;
         if (s < k) {
             double* col = G + s;
-            scale[j] = 1.0 / (lamd + col[s * LD]);
+            const double sq = col[s * LD];
+            lost = lost || !(sq - sq == 0.0);
+            scale[j] = 1.0 / (lamd + sq);
             if (wv == 0) {
                 w[j] = W0 ? (double)W0[(size_t)row * k + s] : 0.0;
                 double p = b[s];
@@ -391,6 +394,13 @@ __device__ __forceinline__ void fold_solve(const FoldArgs& a, uint32_t row, uint
                 e[j] = __builtin_fma(p, scale[j], -w[j]);
             }
         }
+    }
+    // A rated item with a factor that is not finite (its square stands on the
+    // diagonal): from zero the row's residual starts as r - 0 h, no number, and
+    // every rank sums over it, the ones before that factor's too.
+    if (!W0 && __any(lost)) {
+#pragma unroll
+        for (int j = 0; j < NS; ++j) e[j] = __builtin_nan("");
     }
     if (SW > 1) __syncthreads();  // the diagonal and the numerators are read
 #pragma unroll

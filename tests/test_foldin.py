@@ -366,3 +366,35 @@ def test_mlp_forward_gives_large_buffers_back():
     assert all(np.array_equal(got[i << 16:(i + 1) << 16], want) for i in (0, 17, reps - 1))
     assert np.array_equal(mlp.forward(X, bf16=2), want)
     mlp.close()
+
+
+@pytest.mark.parametrize("k", [1, 8, 40, 65, 128])
+def test_fold_rows_with_factors_that_are_not_finite(k):
+    """An item factor that is NaN or infinite: the rows that rate the item are
+    no number where the sweeps over the residual make them so (every rank: the
+    residual starts as r - W0 h), the others are as without it."""
+    F = _gpu()
+    rng = np.random.default_rng(k)
+    deg = [1, 5, 64, 70, 128, 129, 600]
+    n = 700
+    ptr = np.concatenate([[0], np.cumsum(2 * deg)]).astype(np.uint32)
+    # the first seven rows rate item 0, the others do not
+    idx = np.concatenate([np.append(0, 1 + rng.choice(n - 1, size=d - 1, replace=False)) for d in deg]
+                         + [1 + rng.choice(n - 1, size=d, replace=False) for d in deg]).astype(np.uint32)
+    val = rng.integers(1, 6, size=idx.size).astype(np.float32)
+    H = rng.normal(0.1, 0.4, (k, n)).astype(np.float32)
+    W0 = rng.normal(0, 0.3, (len(ptr) - 1, k)).astype(np.float32)
+    for what in (np.nan, np.inf, -np.inf):
+        for rank in sorted({0, k // 2, k - 1}):
+            Hx = H.copy()
+            Hx[rank, 0] = what
+            fold = F.FoldIn(Hx, 0.05)
+            for sweeps in (0, 1, 2):
+                for start in (None, np.zeros_like(W0), W0):
+                    W, _ = fold.rows(ptr, idx, val, sweeps, W0=start)
+                    with np.errstate(all="ignore"):
+                        ref = _fold_f64(ptr, idx, val, Hx, 0.05, sweeps, start)
+                    assert np.array_equal(np.isfinite(W), np.isfinite(ref)), (what, rank, sweeps, start is None)
+                    ok = np.isfinite(ref)
+                    np.testing.assert_allclose(W[ok], ref[ok], rtol=6.1e-8, atol=1e-9 * max(1.0, np.abs(ref[ok]).max()))
+            fold.close()
