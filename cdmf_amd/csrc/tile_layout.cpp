@@ -1,7 +1,7 @@
 // Host-side tables of the tiled copy of a compressed layout (tile_layout.h).
 // O(rows + tiles), as the library calls it.  The per-element tables, O(nnz),
 // are the library's layout_kernels.hip; the host's, of the same definition,
-// complete the tables for the CPU checker that decodes them.
+// complete the tables for tests/native/tile_check.cpp, which decodes them.
 #include "tile_layout.h"
 
 #include <algorithm>
